@@ -18,13 +18,17 @@ constexpr int kOrderWords = 8;
 // persistent-kernel launches timed per solve
 constexpr int kMaxTimedScans = 8;
 
+// the launch geometry of a new context; a call that finds it unchanged picks
+// its own by the amount of work (choose_cfg)
+constexpr pnjl_launch_cfg kDefaultCfg{4, 4, 8, 0};
+
 struct pnjl_ctx {
     int device = 0;
     int num_cu = 256;
     pnjl_model_params params{};
     pnjl::DevParams dp{};
     std::string err;
-    pnjl_launch_cfg cfg{4, 4, 8, 0};
+    pnjl_launch_cfg cfg = kDefaultCfg;
     std::map<std::pair<int, int>, double*> tabs;
     size_t lds_block = 64 * 1024;       // LDS budget of one scan-kernel block (bytes)
     unsigned long long* queue = nullptr;

@@ -229,6 +229,41 @@ ScanGeom scan_geom(int lpp, int pn, int tn, size_t lds_block)
     return ScanGeom{64, 64, 1, tab + group};
 }
 
+// Launch geometry of a call whose context holds the default one (kDefaultCfg):
+// lanes per point by the amount of work.  A point's solve is a serial run of
+// node passes, so while its call does not fill the chip the time is that of
+// its longest solves, and more lanes per point shorten every pass; once the
+// chip is full, 8 lanes are the most efficient (below 8, the groups' LDS state
+// leaves room for one wavefront per SIMD only).  The chip holds 2^17 lanes at
+// two wavefronts per SIMD; most solves end early, so the best lane count is
+// the largest with points x lanes <= 2^19.  Measured (p 64, t 4, DefaultSeed
+// at xi != 0, max_iter 40, ms at 8 / 16 / 32 / 64 lanes): 1024 points 4.2 /
+// 3.0 / 2.4 / 2.2, 8192 points 4.7 / 4.1 / 3.5 / 3.5, 32768 points 7.7 / 6.8 /
+// 7.0 / 8.0, 131072 points 22.4 / 22.0 / 23.8 / 30.2 (fixed 4 lanes: 34, 37,
+// 38, 56).  MultiSeed's six candidates per point run long: items x lanes <=
+// 2^20 (32768 points at 8 / 16 / 32 lanes: 17.1 / 17.8 / 22.4 ms, 2048 points
+// 5.1 / 3.6 / 2.7).  The later stages hold few, long items (the listed points'
+// MultiSeed candidates): points x lanes <= 2^20, at least 16 (p 64, t 4,
+// xi != 0, stage-2 lanes 16 / 64: 16384 points 5.9 / 4.6 ms, 131072 points
+// 22.0 / 23.4).  A chain is serial over its points: 32 lanes up to 4096 chains
+// (16 x 24 x 8 nodes, 256 chains: 14.8 ms at 8, 8.3 at 32, 8.4 at 64), then
+// 16.
+pnjl_launch_cfg choose_cfg(const pnjl_launch_cfg& c, const pnjl::ScanArgs& A)
+{
+    if (c.lanes_per_point != kDefaultCfg.lanes_per_point || c.chunk != kDefaultCfg.chunk ||
+        c.waves_per_cu != kDefaultCfg.waves_per_cu || c.tail_lanes_per_point != kDefaultCfg.tail_lanes_per_point)
+        return c;
+    auto lanes = [](int64_t items, int64_t total, int least) {
+        int l = 64;
+        while (l > least && items > total / l) l /= 2;
+        return l;
+    };
+    if (A.plan == pnjl::PLAN_CHAINS) return pnjl_launch_cfg{A.n_items <= 4096 ? 32 : 16, 1, 8, 0};
+    const bool many = A.plan == pnjl::PLAN_MULTI;
+    const int l = lanes(A.n_points * A.mult, many ? 1 << 20 : 1 << 19, 8);
+    return pnjl_launch_cfg{l, 1, l > 8 ? 8 : 16, std::max(l, lanes(A.n_points, 1 << 20, 16))};
+}
+
 // Lets every scan_kernel instantiation take `bytes` of dynamic LDS.
 bool allow_scan_lds(int bytes)
 {
@@ -341,7 +376,7 @@ int check_policy(int p)
 // same either way.
 int solve_dev(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const double* xi, const double* seed,
               int policy, int pn, int tn, const pnjl_solve_opts* o, const pnjl_solve_out* out,
-              const pnjl_launch_cfg& cfg, hipStream_t stream, bool fixed = false)
+              const pnjl_launch_cfg& launch, hipStream_t stream, bool fixed = false)
 {
     double* tab = nullptr;
     int rc = fixed ? na_table(ctx, pn, tn, stream, &tab) : get_tab(ctx, pn, tn, &tab);
@@ -392,6 +427,7 @@ int solve_dev(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const
     A.surr_cap = o->surrogate_max_steps;
     A.judge_mode = o->surrogate_judge;
     A.queue = fixed ? (unsigned long long*)(na + kNaQueue) : ctx->queue;
+    const pnjl_launch_cfg cfg = choose_cfg(launch, A);
     A.chunk = std::max(1, cfg.chunk);
     A.bnd = ctx->bnd;
     A.nb = ctx->nb;
@@ -488,7 +524,7 @@ int solve_dev(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const
     S.kind = surr ? pnjl::K_SURR : (multi ? pnjl::K_MPOL : (mr3 ? pnjl::K_MR3 : pnjl::K_PRIMARY));
     launch_scan(ctx, S, G, blocks, stream);
     HIPCHK(ctx, hipGetLastError());
-    // the later stages run on the full persistent grid
+    // the later stages run on the persistent grid
     auto next_stage = [&](int kind, int mult, int k_base, const void* list, int count_word) -> int {
         hipLaunchKernelGGL(pnjl::zero_u64, dim3(1), dim3(64), 0, stream, q + pnjl::Q_HEAD, 1);
         pnjl::ScanArgs L = A;
@@ -498,7 +534,11 @@ int solve_dev(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const
         L.order = nullptr;
         L.item_list = (const int32_t*)list;
         L.item_count = q + count_word;
-        launch_scan(ctx, L, G2, fullblocks, stream);
+        // at most n listed points: no more groups than items (an empty 64-lane
+        // stage of a one-point call costs 33 us on the full grid of 512 blocks)
+        const int64_t groups = (n * mult + A.chunk - 1) / A.chunk;
+        const int64_t most = (groups + G2.groups_per_block - 1) / G2.groups_per_block;
+        launch_scan(ctx, L, G2, (int)std::min<int64_t>(fullblocks, most), stream);
         HIPCHK(ctx, hipGetLastError());
         return PNJL_OK;
     };

@@ -304,6 +304,33 @@ def test_launch_geometry_does_not_change_results(gpu_ctx):
         gpu_ctx.set_launch_cfg(**base_cfg)
 
 
+@pytest.mark.parametrize("policy,n,chain", [(0, 1, 0), (0, 8191, 0), (0, 8193, 0), (0, 16385, 0), (0, 32769, 0), (3, 2731, 0),
+                                            (3, 2730, 0), (5, 3 * 4096, 3), (5, 3 * 4097, 3)])
+def test_default_geometry_picks_lanes(gpu_ctx, policy, n, chain):
+    """The default launch geometry chooses lanes per point by the number of
+    points (here on both sides of its lines): the same roots as a fixed 4-lane
+    geometry.  Both runs stop at |F|_inf < ftol near one root (MultiSeed's may
+    be another candidate's), so they differ by at most 2 ftol |J^-1|_inf to
+    first order; 1e-13 for the rounding of the node sums."""
+    from julia_relaxtime_amd import _lib
+    r = np.random.default_rng(n)
+    T, mu, xi = r.uniform(190, 290, n) / 197.327, r.uniform(5, 390, n) / 197.327, r.choice([0.0, 0.3], n)
+    if chain:
+        T, mu, xi = (np.sort(T.reshape(-1, chain), 1).ravel(), np.repeat(mu[::chain], chain), np.repeat(xi[::chain], chain))
+    opts = _lib.default_opts(ftol=1e-10, xtol=1e-14, max_iter=40, chain_len=chain)
+    assert gpu_ctx.launch_cfg() == dict(lanes_per_point=4, chunk=4, waves_per_cu=8, tail_lanes_per_point=0)
+    a = gpu_ctx.solve_batch(T, mu, xi, policy=policy, p_num=16, t_num=4, opts=opts)
+    try:
+        gpu_ctx.set_launch_cfg(4, 1, 8, 0)
+        b = gpu_ctx.solve_batch(T, mu, xi, policy=policy, p_num=16, t_num=4, opts=opts)
+    finally:
+        gpu_ctx.set_launch_cfg()
+    assert a["converged"].all() and b["converged"].all()
+    J = gpu_ctx.residual_batch(b["x"], T, mu, xi, 16, 4)[1]
+    bound = 2e-10 * np.abs(np.linalg.inv(J)).sum(axis=2).max(axis=1) + 1e-13
+    assert np.all(np.abs(a["x"] - b["x"]).max(axis=1) <= bound)
+
+
 def test_device_pointer_path(gpu_ctx):
     """Inputs already in HBM (torch tensors) give the same results as the host path."""
     import torch
