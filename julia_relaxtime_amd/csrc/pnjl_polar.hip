@@ -1,15 +1,21 @@
 // pnjl_polar.hip -- the anisotropic one-loop polarization Pi(k0, k) on gfx950.
 //
-// One GPU thread evaluates one B0 / B0_correction / polarization value with
-// the reference's fixed quadrature: the same breakpoints (poles of the k = 0
-// integrand, roots of the k > 0 logarithm, imaginary-part intervals), the
-// same 16/32-node power-clustered and 33-node double-exponential rules, the
-// same principal-value subtraction and the same skip-non-finite rule, so the
-// results reproduce the reference's numbers, not the exact integrals.
-// Quadrature tables sit in LDS.  For the grid call, the threads of a
-// wavefront share (point, pair) and take an 8 x 8 tile of (k0, k), so their
-// segment structures differ only smoothly; the propagator batch sorts its
-// work into buckets of similar (pair, mass, lambda, k) for the same reason.
+// One lane, or a group of them, evaluates one B0 / B0_correction /
+// polarization value with the reference's fixed quadrature: the same
+// breakpoints (poles of the k = 0 integrand, roots of the k > 0 logarithm,
+// imaginary-part intervals), the same 16/32-node power-clustered and 33-node
+// double-exponential rules, the same principal-value subtraction and the same
+// skip-non-finite rule, so the results reproduce the reference's numbers, not
+// the exact integrals.  All of it is FP64 arithmetic on tables in LDS, bound
+// by instruction issue: B0's terms that differ only in the distribution's
+// sign are evaluated together, every rule and integrand of an evaluation goes
+// through one node loop, and the nodes' functions are table-driven.  On the
+// 256-point x 3 pairs x 128 k0 x 64 k grid a replay takes 10.4 ms (30.4 ms
+// with one loop per rule, term by term, on the library's functions).  For the
+// grid call, the threads of a wavefront share (point, pair) and take an 8 x 8
+// tile of (k0, k), so their segment structures differ only smoothly; the
+// propagator batch sorts its work into buckets of similar (pair, mass,
+// lambda, k) for the same reason.
 //
 // Follows src/relaxtime/OneLoopIntegrals.jl, OneLoopIntegralsAniso.jl,
 // PolarizationAniso.jl, src/integration/IntervalQuadratureStrategies.jl and
@@ -20,6 +26,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "pnjl_ctx.h"
@@ -41,35 +48,20 @@ constexpr double kEpsSeg = 1.0e-12;     // OneLoopIntegrals.jl:24
 constexpr double kPvGapRel = 1e-6;      // OneLoopIntegrals.jl:35
 constexpr double kAlpha = 0.35;         // IntervalQuadratureStrategies.jl:35
 constexpr double kDeH = 0.15;           // IntervalQuadratureStrategies.jl:36
-constexpr int kTabLen = 354;            // see tab_* offsets below
 
-enum { NONE = 0, LEFT = 1, RIGHT = 2, BOTH = 3 };
-enum { PLUS = 0, MINUS = 1 };           // B0 signs (f+(E), f+(-E) = 1 - f-(E))
-enum { QUARK = 0, ANTIQUARK = 1 };      // first-order anisotropy signs
-
-// table layout: x16 w16 x32 w32 | pl_t16 pl_tp16 pl_t32 pl_tp32 | pr_t16 pr_tp16 pr_t32 pr_tp32 | de_phi de_phip
-struct Tabs {
-    const double *x16, *w16, *x32, *w32;
-    const double *pl_t16, *pl_tp16, *pl_t32, *pl_tp32;
-    const double *pr_t16, *pr_tp16, *pr_t32, *pr_tp32;
-    const double *de_phi, *de_phip;
-};
-
-__device__ __forceinline__ Tabs make_tabs(const double* t)
-{
-    Tabs q;
-    q.x16 = t; q.w16 = t + 16; q.x32 = t + 32; q.w32 = t + 64;
-    q.pl_t16 = t + 96; q.pl_tp16 = t + 112; q.pl_t32 = t + 128; q.pl_tp32 = t + 160;
-    q.pr_t16 = t + 192; q.pr_tp16 = t + 208; q.pr_t32 = t + 224; q.pr_tp32 = t + 256;
-    q.de_phi = t + 288; q.de_phip = t + 321;
-    return q;
-}
-
-// The pole-search kernels' quadrature tables.  Their B0 routine is out of
-// line; it rebuilds its table pointers from this array rather than taking
-// them from the caller, so that it reads the tables with LDS instructions
-// (a pointer passed in would be a generic address: flat loads).
-__shared__ double mass_tab[kTabLen];
+// ---- tables ------------------------------------------------------------------
+// The quadrature kernels' tables in LDS, one array per kernel: addressed from
+// the array itself everywhere (a pointer passed to an out-of-line routine
+// would be generic: flat loads).  Layout: 2^(j/64) [64] (pnjl::exp_tab), pairs
+// (1/c_j, log c_j) [128] (log_p), then the rules, each as nodes t[n] and
+// weights w[n] of sum_i s w_i f(x0 + s t_i).
+constexpr int kPLog = 64;
+constexpr int kPRules = kPLog + 256;
+// power-clustered left / right (x0 = a, s = b - a), double exponential and
+// Gauss-Legendre (x0 = centre, s = half length)
+enum { R_L16 = kPRules, R_L32 = R_L16 + 32, R_R32 = R_L32 + 64, R_DE = R_R32 + 64, R_G16 = R_DE + 66, R_G32 = R_G16 + 32 };
+constexpr int kTabLen = R_G32 + 64;
+__shared__ double ptab[kTabLen];
 
 struct Phys {
     double Lambda, Nc;
@@ -86,264 +78,234 @@ __device__ __forceinline__ double jeps(double x)
 __device__ __forceinline__ double jsign(double x) { return x > 0 ? 1.0 : (x < 0 ? -1.0 : x); }
 __device__ __forceinline__ double clamp_e(double e) { return e < 1e-200 ? 1e-200 : (e > 1e200 ? 1e200 : e); }
 
+// ---- arithmetic of the node loops ----------------------------------------------
+// The quadratures are bound by the FP64 instructions of their nodes (a square
+// root, an exponential, a logarithm and quotients each).  The helpers below
+// round like the library's within a bit, without its scaling and special
+// cases, which the callers' tests cover.
+
+// sqrt(x), NaN for x < 0: v_rsq_f64 estimate, one Goldschmidt step and a
+// residual correction (Markstein, IA-64 and Elementary Functions, 2000)
+__device__ __forceinline__ double sqrt_p(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double e = fma(-g, h, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    g = fma(fma(-g, g, x), h, g);
+    return x == 0.0 ? 0.0 : g;
+}
+
+// 1/d to about 2^-45 (v_rcp_f64 and one Newton step)
+__device__ __forceinline__ double rcp1(double d)
+{
+    const double r = __builtin_amdgcn_rcp(d);
+    return fma(r, fma(-d, r, 1.0), r);
+}
+
+// n/d from r ~ 1/d: the residual correction leaves about half an ulp
+__device__ __forceinline__ double div_r(double n, double d, double r)
+{
+    const double q = n * r;
+    return fma(fma(-d, q, n), r, q);
+}
+__device__ __forceinline__ double div_p(double n, double d) { return div_r(n, d, rcp1(d)); }
+
+// exp(x) as pnjl::exp_tab (Tang's table method, x clamped to [-800, 700]) with
+// the table entry added last: within about 0.6 ulp
+__device__ __forceinline__ double exp_p(double x)
+{
+    x = fmin(fmax(x, -800.0), 700.0);
+    const double nd = rint(x * 0x1.71547652b82fep+6);   // 64 / ln 2
+    double r = fma(nd, -0x1.62e42fee00000p-7, x);       // ln 2 / 64, split
+    r = fma(nd, -0x1.a39ef35793c76p-39, r);
+    const int n = (int)nd;
+    double p = pnjl::fma_k(r, 1.0 / 120.0, 1.0 / 24.0);
+    p = pnjl::fma_k(r, p, 1.0 / 6.0);
+    p = fma(r, p, 0.5);
+    p = fma(r * r, p, r);   // e^r - 1
+    const double t = ptab[pnjl::kExpTab + (n & 63)];
+    return ldexp(fma(t, p, t), n >> 6);
+}
+
+// log(x), x > 0 normal (Tang, ACM TOMS 16(4), 1990, on 128 intervals of [1,
+// 2)): the upper half counts as [1/2, 1) of the next binade and the intervals
+// next to 1 have c_j = 1, so the result keeps its relative accuracy near x = 1.
+__device__ __forceinline__ double log_p(double x)
+{
+    const double ln2_hi = 0x1.62e42fee00000p-1;
+    const double ln2_lo = 0x1.a39ef35793c76p-33;
+    int e;
+    const double m = 2.0 * frexp(x, &e);   // [1, 2)
+    const int j = (int)((uint32_t)(__double2hiint(m)) >> 13) & 127;
+    const double inv = ptab[kPLog + 2 * j], lc = ptab[kPLog + 2 * j + 1];
+    const double r = fma(m, inv, -1.0);
+    double p = pnjl::fma_k(r, -1.0 / 8.0, 1.0 / 7.0);
+    p = pnjl::fma_k(r, p, -1.0 / 6.0);
+    p = pnjl::fma_k(r, p, 1.0 / 5.0);
+    p = pnjl::fma_k(r, p, -0.25);
+    p = pnjl::fma_k(r, p, 1.0 / 3.0);
+    p = fma(r, p, -0.5);
+    const double ed = (double)(e - 1 + (j >> 6));
+    return fma(ed, ln2_hi, lc) + (r + fma(r * r, p, ed * ln2_lo));
+}
+
+// log(x) of any x >= 0 or NaN, subnormal x excepted
+__device__ __forceinline__ double log_c(double x)
+{
+    const double v = log_p(x);
+    return x > 0.0 && x <= 1.7976931348623157e308 ? v : (x == 0.0 ? -__builtin_inf() : x);
+}
+
 // PNJL distributions and their antiderivatives  QuarkDistribution.jl:14-99
-__device__ __forceinline__ double dist_ratio(double e, double c1, double c2)
+// The medium of one evaluation.  joint: |mu|/T < 150, so one exponential
+// serves quark and antiquark (exp(-(E + mu)/T) = exp(-(E - mu)/T) exp(-2
+// mu/T)) without leaving the range; otherwise each has its own.
+struct Medium {
+    double mu, T, beta, K2, Phi, Phib;
+    bool joint;
+};
+
+__device__ __forceinline__ Medium make_medium(double mu, double T, double Phi, double Phib)
 {
-    double e2 = e * e, e3 = e2 * e;
-    return (c1 * e + 2 * c2 * e2 + e3) / (1 + 3 * c1 * e + 3 * c2 * e2 + e3);
+    Medium M{mu, T, 1 / T, 0.0, Phi, Phib, false};
+    M.joint = M.beta > 0.0 && M.beta < 1e300 && fabs(mu) * M.beta < 150.0;
+    M.K2 = exp_p(-2.0 * mu * M.beta);
+    return M;
 }
 
-__device__ __forceinline__ double quark_f(double E, double mu, double T, double Phi, double Phib)
+// exp(-(E - mu)/T) and exp(-(E + mu)/T), clamped to [1e-200, 1e200]
+__device__ __forceinline__ void boltzmann(const Medium& M, double E, double& ep, double& em)
 {
-    return dist_ratio(clamp_e(exp(-(E - mu) * (1 / T))), Phi, Phib);
+    const double x = (M.mu - E) * M.beta;
+    const double t = exp_p(x);
+    ep = clamp_e(t);
+    em = clamp_e(t * M.K2);
+    if (!M.joint) {
+        const double y = -(E + M.mu) * M.beta;
+        em = y != y ? y : clamp_e(exp_p(y));   // a NaN exponent stays one
+        ep = x != x ? x : ep;
+    }
 }
 
-__device__ __forceinline__ double antiquark_f(double E, double mu, double T, double Phi, double Phib)
+// the distributions of both B0 signs, f(E) and 1 - fbar(E) (f+(-E) = 1 - f-(E))
+//   distribution_value_b0  OneLoopIntegrals.jl:68-83
+__device__ __forceinline__ void dist2(const Medium& M, double E, double& dp, double& dm)
 {
-    return dist_ratio(clamp_e(exp(-(E + mu) * (1 / T))), Phib, Phi);
+    double ep, em;
+    boltzmann(M, E, ep, em);
+    const double p2 = ep * ep, p3 = p2 * ep, m2 = em * em, m3 = m2 * em;
+    const double np = M.Phi * ep + 2 * M.Phib * p2 + p3, nm = M.Phib * em + 2 * M.Phi * m2 + m3;
+    const double Dp = 1 + 3 * M.Phi * ep + 3 * M.Phib * p2 + p3, Dm = 1 + 3 * M.Phib * em + 3 * M.Phi * m2 + m3;
+    dp = div_p(np, Dp);
+    dm = 1.0 - div_p(nm, Dm);
 }
 
-__device__ __forceinline__ double anti_deriv(double e, double c1, double c2, double T)
+// antiderivatives of both distributions at E: -T ln(1 + 3 c1 e + 3 c2 e^2 + e^3) / 3
+__device__ __forceinline__ void anti2(const Medium& M, double E, double& ap, double& am)
 {
-    double e2 = e * e, e3 = e2 * e;
-    double d = 1 + 3 * c1 * e + 3 * c2 * e2 + e3;
-    return -T * log(d <= 1e-300 ? 1e-300 : d) / 3;
-}
-
-// distribution_value_b0 / distribution_integral_b0  OneLoopIntegrals.jl:68-104
-__device__ __forceinline__ double dist_b0(int sg, double E, double mu, double T, double Phi, double Phib)
-{
-    return sg == PLUS ? quark_f(E, mu, T, Phi, Phib) : 1.0 - antiquark_f(E, mu, T, Phi, Phib);
-}
-
-__device__ double dist_int_b0(int sg, double a, double b, double mu, double T, double Phi, double Phib)
-{
-    const double beta = 1 / T;
-    if (sg == PLUS)
-        return anti_deriv(clamp_e(exp(-(b - mu) * beta)), Phi, Phib, T) -
-               anti_deriv(clamp_e(exp(-(a - mu) * beta)), Phi, Phib, T);
-    return (b - a) - (anti_deriv(clamp_e(exp(-(b + mu) * beta)), Phib, Phi, T) -
-                      anti_deriv(clamp_e(exp(-(a + mu) * beta)), Phib, Phi, T));
+    double ep, em;
+    boltzmann(M, E, ep, em);
+    const double p2 = ep * ep, m2 = em * em;
+    const double dp = 1 + 3 * M.Phi * ep + 3 * M.Phib * p2 + p2 * ep, dm = 1 + 3 * M.Phib * em + 3 * M.Phi * m2 + m2 * em;
+    ap = -M.T * log_c(dp <= 1e-300 ? 1e-300 : dp) / 3;
+    am = -M.T * log_c(dm <= 1e-300 ? 1e-300 : dm) / 3;
 }
 
 // energy_cutoff / internal_momentum  OneLoopIntegrals.jl:37-48
 __device__ __forceinline__ double e_cut(const Phys& P, double m)
 {
     double mp = m > 0 ? m : 0.0;
-    return sqrt(mp * mp + P.Lambda * P.Lambda);
+    return sqrt_p(mp * mp + P.Lambda * P.Lambda);
 }
 
 __device__ __forceinline__ double p_int(double E, double m)
 {
     double mp = m > 0 ? m : 0.0;
-    return sqrt(E * E - mp * mp);
+    return sqrt_p(E * E - mp * mp);
 }
 
-// Lane-split quadrature (L > 1, the pole search's long tail): the L
-// consecutive lanes of a group each evaluate the nodes i = gl, gl + L, ... of
-// an N-node rule and leave the terms in the group's LDS row, then every lane
-// adds all N terms in the order i = 0 .. N-1 -- the one-thread loop's sum, bit
-// for bit, on every lane.  A skipped (non-finite) node contributes +0.0 there,
-// which leaves any sum the loop can hold unchanged: the sums start at +0.0
-// and so never hold -0.0.  Callers keep the group's control flow uniform
-// (same arguments on every lane of the group); the group's lanes are in one
-// wavefront, whose LDS accesses complete in program order.  L = 1 is the
-// one-thread loop itself.
-constexpr int kQRow = 33;              // terms of the longest rule
-constexpr int kQRows = 256 / 4;        // rows per 256-thread block at 4 lanes per group
-__shared__ double qterms[kQRows][kQRow];
+// A segment of a piecewise rule: sum over the rule's nodes of s w_i f(x0 + s t_i);
+// n = 0 where the segment is empty (integrate_hybrid_interval returns 0 for
+// b <= a and for ends that are not finite).
+struct Seg {
+    double x0, s;
+    int off, n;
+};
+__device__ __forceinline__ Seg seg_power(double a, double b, int off, int n)
+{
+    return Seg{a, b - a, off, (isfinite(a) && isfinite(b) && b > a) ? n : 0};
+}
+// by value: a choice between the objects themselves would keep them in memory
+__device__ __forceinline__ double pick(bool c, double a, double b) { return c ? a : b; }
+__device__ __forceinline__ Seg seg_pick(bool c, Seg a, Seg b)
+{
+    return Seg{pick(c, a.x0, b.x0), pick(c, a.s, b.s), c ? a.off : b.off, c ? a.n : b.n};
+}
+__device__ __forceinline__ Seg seg_mid(double a, double b, int off, int n)
+{
+    return Seg{(a + b) / 2, (b - a) / 2, off, (isfinite(a) && isfinite(b) && b > a) ? n : 0};
+}
+
+// ---- B~0 for both distribution signs ---------------------------------------------
+// One evaluation at (lambda, k, m, m') gives B~0 with f(E) ("plus") and with
+// 1 - fbar(E) ("minus"): the two integrals have the same poles, breakpoints
+// and nodes and share everything but the distribution, and B0 of equal masses
+// (or its average over +-k0) needs both at the same lambda.  The nodes of all
+// of an evaluation's segments run through one loop, whichever rule and
+// integrand a lane has, so the lanes of a wavefront do not wait for each
+// other's branches.
+//
+// L > 1: the L consecutive lanes of a group evaluate the nodes i = q, q + L,
+// ... of a segment (q the lane's number in the group) and leave the terms in
+// the group's LDS row, then every lane adds them in the order of the nodes --
+// the one-lane loop's sums, bit for bit.  Control flow is uniform in a group
+// (same arguments on every lane), and a group's lanes are in one wavefront,
+// whose LDS accesses complete in program order.
+constexpr int kRowTerms = 33;   // terms of the longest rule
 
 template <int L>
-__device__ __forceinline__ int qlane()
+__device__ __forceinline__ double2* term_rows()
 {
-    return L == 1 ? 0 : (int)(threadIdx.x & (L - 1));
+    __shared__ double2 rows[L > 1 ? 256 / L * kRowTerms : 1];
+    return rows + (L > 1 ? threadIdx.x / L * kRowTerms : 0);
 }
 
-template <int L, int N, class Term>
-__device__ __forceinline__ double ordered_sum(double acc, const Term& term)
+// acc += the n terms of the segment, in order, on every lane of the group
+template <int L>
+__device__ __forceinline__ void add_terms(int n, double& ap, double& am)
 {
-    static_assert(L > 1 && (L & (L - 1)) == 0 && 256 / L <= kQRows && N <= kQRow, "lane-split rule shape");
-    double* row = qterms[threadIdx.x / L];
-    const int gl = qlane<L>();
+    const double2* row = term_rows<L>();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    // n = 16, 32 or 33: the loads of four terms issue together
 #pragma unroll 1
-    for (int i = gl; i < N; i += L) row[i] = term(i);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int b = 0; b + 4 <= n; b += 4) {
+        double2 t[4];
 #pragma unroll
-    for (int i = 0; i < N; i++) acc += row[i];   // the loads issue together, the adds keep their order
-    // the row is written again by the group's next rule only after every lane has read it
+        for (int j = 0; j < 4; j++) t[j] = row[b + j];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            ap += t[j].x;
+            am += t[j].y;
+        }
+    }
+    if (n & 1) {
+        ap += row[n - 1].x;
+        am += row[n - 1].y;
+    }
+    // the row is written again only after every lane has read it
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    return acc;
 }
-
-// integrate_hybrid_interval  IntervalQuadratureStrategies.jl:194-310
-template <int L, int N, class F>
-__device__ double rule_power(const F& f, double a, double b, const double* t, const double* tp, const double* W)
-{
-    double len = b - a, total = 0.0;
-    if constexpr (L > 1) {
-        return ordered_sum<L, N>(total, [&](int i) {
-            double x = a + len * t[i];
-            double w = W[i] * len * tp[i];
-            double v = f(x);
-            return isfinite(v) ? w * v : 0.0;
-        });
-    } else {
-        for (int i = 0; i < N; i++) {
-            double x = a + len * t[i];
-            double w = W[i] * len * tp[i];
-            double v = f(x);
-            if (isfinite(v)) total += w * v;
-        }
-        return total;
-    }
-}
-
-template <int L, class F>
-__device__ double hybrid(const F& f, const Tabs& q, double a, double b, int pos, int n)
-{
-    if (!(isfinite(a) && isfinite(b)) || b <= a) return 0.0;
-    if (pos == BOTH) {
-        double half = (b - a) / 2, center = (a + b) / 2, total = 0.0;
-        if constexpr (L > 1) {
-            return ordered_sum<L, 33>(total, [&](int i) {
-                double x = center + half * q.de_phi[i];
-                double w = half * q.de_phip[i];
-                double v = f(x);
-                return isfinite(v) ? w * v : 0.0;
-            });
-        } else {
-            for (int i = 0; i < 33; i++) {
-                double x = center + half * q.de_phi[i];
-                double w = half * q.de_phip[i];
-                double v = f(x);
-                if (isfinite(v)) total += w * v;
-            }
-            return total;
-        }
-    }
-    if (pos == RIGHT)
-        return n == 16 ? rule_power<L, 16>(f, a, b, q.pr_t16, q.pr_tp16, q.w16)
-                       : rule_power<L, 32>(f, a, b, q.pr_t32, q.pr_tp32, q.w32);
-    return n == 16 ? rule_power<L, 16>(f, a, b, q.pl_t16, q.pl_tp16, q.w16)
-                   : rule_power<L, 32>(f, a, b, q.pl_t32, q.pl_tp32, q.w32);
-}
-
-// ---- B~0 at k = 0  OneLoopIntegrals.jl:117-224 ------------------------------
-struct B0K0 {
-    int sg;
-    double lam, m, dterm, mu, T, Phi, Phib;
-    __device__ double operator()(double E) const
-    {
-        double p = p_int(E, m);
-        double dist = dist_b0(sg, E, mu, T, Phi, Phib);
-        double den = lam * E + dterm;
-        if (!isfinite(p) || !isfinite(dist) || !isfinite(den)) return 0.0;
-        if (fabs(den) < kEpsSeg) return 0.0;
-        double v = p * dist / den;
-        return isfinite(v) ? v : 0.0;
-    }
+struct Pair {
+    double rp, ip, rm, im;   // plus: real, imaginary; minus
 };
 
-struct B0Numer {
-    int sg;
-    double m, mu, T, Phi, Phib;
-    __device__ double operator()(double E) const
-    {
-        double p = p_int(E, m);
-        double dist = dist_b0(sg, E, mu, T, Phi, Phib);
-        if (!isfinite(p) || !isfinite(dist)) return 0.0;
-        double v = p * dist;
-        return isfinite(v) ? v : 0.0;
-    }
-};
-
-struct B0Regular {
-    B0Numer num;
-    double E0, f0, Emin, Emax;
-    __device__ double operator()(double E) const
-    {
-        double d = E - E0;
-        if (fabs(d) < 64 * jeps(E0)) {
-            double del = fmax(1e-7 * (Emax - Emin), 64 * jeps(E0));
-            double El = fmax(Emin, E0 - del), Er = fmin(Emax, E0 + del);
-            return Er > El ? (num(Er) - num(El)) / (Er - El) : 0.0;
-        }
-        return (num(E) - f0) / d;
-    }
-};
-
-template <int L>
-__device__ void tilde_B0_k0(const Phys& P, const Tabs& q, int sg, double lam, double m_in, double mp_in, double mu,
-                            double T, double Phi, double Phib, double& re, double& im)
-{
-    const double m = m_in > 0 ? m_in : 0.0, mp = mp_in > 0 ? mp_in : 0.0;
-    const double Emin = m, Emax = e_cut(P, m);
-    const double dterm = (lam * lam + m * m - mp * mp) / 2.0;
-    const B0K0 f{sg, lam, m, dterm, mu, T, Phi, Phib};
-    // singularity_k_zero  :144-157
-    const double E0 = -dterm / lam;
-    bool has = false;
-    if (isfinite(E0)) {
-        double tol = 1e-8 * fmax(1.0, fabs(E0));
-        has = (E0 > Emin - tol) && (E0 < Emax + tol);
-    }
-    if (!has) {
-        re = hybrid<L>(f, q, Emin, Emax, NONE, 16) * 2.0;
-        im = 0.0 / lam;
-        return;
-    }
-    const B0Numer num{sg, m, mu, T, Phi, Phib};
-    const double f0 = num(E0);
-    double pv;
-    const double etol = 1e-10 * fmax(1.0, Emax - Emin);
-    if (fabs(E0 - Emin) <= etol || fabs(Emax - E0) <= etol) {
-        double gap = fmax(kPvGapRel * (Emax - Emin), 64 * jeps(E0));
-        double left_end = fmax(Emin, E0 - gap), right_start = fmin(Emax, E0 + gap);
-        pv = 0.0;
-        if (left_end > Emin) pv += hybrid<L>(f, q, Emin, left_end, NONE, 16);
-        if (right_start < Emax) pv += hybrid<L>(f, q, right_start, Emax, NONE, 16);
-    } else {
-        const B0Regular g{num, E0, f0, Emin, Emax};
-        double regular = hybrid<L>(g, q, Emin, Emax, NONE, 32);
-        double logterm = f0 * (log(fabs(Emax - E0)) - log(fabs(Emin - E0)));
-        pv = (regular + logterm) / lam;
-    }
-    const double p0 = p_int(E0, m);
-    re = pv * 2.0;
-    im = 2.0 * kPi * p0 * dist_b0(sg, E0, mu, T, Phi, Phib) / lam;
-}
-
-// ---- B~0 at k > 0  OneLoopIntegrals.jl:228-476 ------------------------------
-struct B0Kpos {
-    int sg;
-    double lam, k, m, mp, mu, T, Phi, Phib;
-    __device__ double operator()(double E) const
-    {
-        double p = p_int(E, m);
-        double dist = dist_b0(sg, E, mu, T, Phi, Phib);
-        double lpE = lam + E;
-        double common = lpE * lpE - mp * mp;
-        double pmk = p - k, ppk = p + k;
-        double num = common - pmk * pmk;
-        double den = common - ppk * ppk;
-        if (!isfinite(p) || !isfinite(dist) || !isfinite(num) || !isfinite(den)) return 0.0;
-        if (fabs(num) < kEpsSeg && fabs(den) < kEpsSeg) return 0.0;
-        if (fabs(den) < kEpsSeg) den = (den == 0.0) ? kEpsSeg : jsign(den) * kEpsSeg;
-        double ratio = fabs(num / den);
-        if (!isfinite(ratio)) return 0.0;
-        ratio = fmax(ratio, 1e-300);
-        double lt = log(ratio);
-        if (!isfinite(lt)) return 0.0;
-        double v = dist * lt;
-        return isfinite(v) ? v : 0.0;
-    }
-};
-
-// singularity_k_positive  :239-330 -> number of intervals in iv (0..2)
+// singularity_k_positive  OneLoopIntegrals.jl:239-330 -> number of intervals in iv (0..2)
 __device__ int sing_kpos(double lam, double k, double m, double mp, double Emin, double Emax, double iv[2][2])
 {
     int n = 0;
@@ -365,7 +327,7 @@ __device__ int sing_kpos(double lam, double k, double m, double mp, double Emin,
     const double A = lam * lam - k * k + m * m - mp * mp;
     const double disc = A * A + 4.0 * m * m * d0;
     if (disc < 0.0) return 0;
-    const double sq = sqrt(disc);
+    const double sq = sqrt_p(disc);
     double E1 = (lam * A - k * sq) / denom, E2 = (lam * A + k * sq) / denom;
     if (E1 > E2) {
         double t = E1;
@@ -384,175 +346,202 @@ __device__ int sing_kpos(double lam, double k, double m, double mp, double Emin,
         }
         return n;
     }
-    if (E1 > Emin) {
-        double c = fmin(E1, Emax);
-        if (c > Emin) {
-            iv[n][0] = Emin;
-            iv[n][1] = c;
-            n++;
-        }
-    }
-    if (E2 < Emax) {
-        double c = fmax(E2, Emin);
-        if (Emax > c) {
-            iv[n][0] = c;
-            iv[n][1] = Emax;
-            n++;
-        }
-    }
-    return n;
+    // the intervals of this branch are [Emin, c1] and [c2, Emax], stored as such
+    const double c1 = E1 > Emin ? fmin(E1, Emax) : Emin, c2 = E2 < Emax ? fmax(E2, Emin) : Emax;
+    const bool low = c1 > Emin, high = Emax > c2;
+    iv[0][0] = low ? Emin : c2;
+    iv[0][1] = low ? c1 : Emax;
+    iv[1][0] = c2;
+    iv[1][1] = Emax;
+    return (low ? 1 : 0) + (high ? 1 : 0);
 }
 
-// integrate_piecewise_hybrid  :335-421
-template <int L, class F>
-__device__ double piecewise(const F& f, const Tabs& q, double Emin, double Emax, int niv, const double iv[2][2])
-{
-    if (niv == 0) return hybrid<L>(f, q, Emin, Emax, NONE, 16);
-    double E1 = __builtin_nan(""), E2 = __builtin_nan("");
-    if (niv == 1) {
-        E1 = iv[0][0];
-        E2 = iv[0][1];
-    } else {
-        const double a1 = iv[0][0], b1 = iv[0][1], a2 = iv[1][0], b2 = iv[1][1];
-        const double tol = 1e-12 * fmax(1.0, Emax - Emin);
-        if (fabs(a1 - Emin) <= tol) E1 = b1;
-        else if (fabs(a2 - Emin) <= tol) E1 = b2;
-        if (fabs(b1 - Emax) <= tol) E2 = a1;
-        else if (fabs(b2 - Emax) <= tol) E2 = a2;
-    }
-    if (isfinite(E1) && isfinite(E2)) {
-        double total = 0.0;
-        if (E1 > Emin) total += hybrid<L>(f, q, Emin, E1, RIGHT, 32);
-        if (E2 > E1) total += hybrid<L>(f, q, E1, E2, BOTH, 32);
-        if (Emax > E2) total += hybrid<L>(f, q, E2, Emax, LEFT, 16);
-        return total;
-    }
-    // general path: sorted unique breakpoints (insertion sort of <= 6 values)
-    double pts[6];
-    int np = 0;
-    pts[np++] = Emin;
-    for (int i = 0; i < niv; i++) {
-        pts[np++] = iv[i][0];
-        pts[np++] = iv[i][1];
-    }
-    pts[np++] = Emax;
-    for (int i = 1; i < np; i++)
-        for (int j = i; j > 0 && pts[j] < pts[j - 1]; j--) {
-            double t = pts[j];
-            pts[j] = pts[j - 1];
-            pts[j - 1] = t;
-        }
-    int u = 0;
-    for (int i = 0; i < np; i++)
-        if (u == 0 || pts[i] != pts[u - 1]) pts[u++] = pts[i];
-    const int nseg = u - 1;
-    if (nseg <= 0) return 0.0;
-    if (nseg == 1) return hybrid<L>(f, q, pts[0], pts[1], NONE, 16);
-    double total = 0.0;
-    for (int i = 1; i <= nseg; i++) {
-        double a = pts[i - 1], b = pts[i];
-        if (!(isfinite(a) && isfinite(b)) || b <= a) continue;
-        int pos = (i == 1) ? RIGHT : (i == nseg ? LEFT : BOTH);
-        total += hybrid<L>(f, q, a, b, pos, i == nseg ? 16 : 32);
-    }
-    return total;
-}
-
+// lam_m: the minus term's own lambda, equal to lam or to its last bits (lambda
+// = +-k0 + mu1 - mu2 rounds differently for the two signs of k0).  At rest and
+// on a threshold, E0 = m, whether p(E0) exists hangs on those bits (a pole
+// search started there ends or not), so each sign takes its own.
 template <int L>
-__device__ void tilde_B0_kpos(const Phys& P, const Tabs& q, int sg, double lam, double k, double m_in, double mp_in,
-                              double mu, double T, double Phi, double Phib, double& re, double& im)
+__device__ Pair tilde_B0(const Phys& P, const Medium& M, double lam, double lam_m, double k, double m_in, double mp_in,
+                         int q)
 {
     const double m = m_in > 0 ? m_in : 0.0, mp = mp_in > 0 ? mp_in : 0.0;
     const double Emin = m, Emax = e_cut(P, m);
-    double iv[2][2];
-    const int niv = sing_kpos(lam, k, m, mp, Emin, Emax, iv);
-    const B0Kpos f{sg, lam, k, m, mp, mu, T, Phi, Phib};
-    const double real = piecewise<L>(f, q, Emin, Emax, niv, iv);
-    double imag = 0.0;
-    if (niv > 0) {
-        for (int i = 0; i < niv; i++) imag += dist_int_b0(sg, iv[i][0], iv[i][1], mu, T, Phi, Phib);
-        imag *= kPi * jsign(lam);
-    }
-    re = real / k;
-    im = imag / k;
-}
-
-template <int L>
-__device__ void tilde_B0(const Phys& P, const Tabs& q, int sg, double lam, double k, double m, double mp, double mu,
-                         double T, double Phi, double Phib, double& re, double& im)
-{
-    if (fabs(k) < kEpsK) tilde_B0_k0<L>(P, q, sg, lam, m, mp, mu, T, Phi, Phib, re, im);
-    else tilde_B0_kpos<L>(P, q, sg, lam, k, m, mp, mu, T, Phi, Phib, re, im);
-}
-
-// B0  OneLoopIntegrals.jl:489-503: B~+(-l; m1, m2, mu1) - B~-(l; m1, m2, mu1)
-// + B~+(l; m2, m1, mu2) - B~-(-l; m2, m1, mu2), summed in this order.  One
-// loop over the four terms keeps a single copy of tilde_B0 in the kernel.
-template <int L = 1>
-__device__ void B0(const Phys& P, const Tabs& q, double lam, double k, double m1, double mu1, double m2, double mu2,
-                   double T, double Phi, double Phib, double& re, double& im)
-{
-    re = 0.0;
-    im = 0.0;
-#pragma unroll 1
-    for (int t = 0; t < 4; t++) {
-        const bool swap = t >= 2;
-        const double l = (t == 0 || t == 3) ? -lam : lam;
-        double r, i;
-        tilde_B0<L>(P, q, (t & 1) ? MINUS : PLUS, l, k, swap ? m2 : m1, swap ? m1 : m2, swap ? mu2 : mu1, T, Phi, Phib,
-                 r, i);
-        if (t & 1) {
-            re -= r;
-            im -= i;
+    const bool at_rest = fabs(k) < kEpsK;
+    // integrand: RATIO  f(E) ln|num / den| (k > 0); POLE  p f(E) / (lambda E + d);
+    // REGULAR  (p f(E) - f0) / (E - E0), the principal value's regular part
+    enum { RATIO, POLE, REGULAR };
+    int form = RATIO;
+    Seg sg[3] = {};
+    Pair o{0.0, 0.0, 0.0, 0.0};          // what is not a node sum
+    double scale = 1.0;                  // of the node sums
+    double dterm = 0.0, E0 = 0.0, f0p = 0.0, f0m = 0.0, near = 0.0, wnear = 0.0;
+    if (at_rest) {
+        // OneLoopIntegrals.jl:117-224
+        form = POLE;
+        scale = 2.0;
+        dterm = (lam * lam + m * m - mp * mp) / 2.0;
+        E0 = -dterm / lam;
+        bool has = false;
+        if (isfinite(E0)) {   // singularity_k_zero  :144-157
+            const double tol = 1e-8 * fmax(1.0, fabs(E0));
+            has = (E0 > Emin - tol) && (E0 < Emax + tol);
+        }
+        if (!has) {
+            sg[2] = seg_power(Emin, Emax, R_L16, 16);
+            o.ip = o.im = 0.0 / lam;
         } else {
-            re += r;
-            im += i;
+            double dp, dm;
+            dist2(M, E0, dp, dm);
+            const double p0 = p_int(E0, m), ps = isfinite(p0) ? p0 : 0.0;
+            f0p = isfinite(ps * dp) ? ps * dp : 0.0;
+            f0m = isfinite(ps * dm) ? ps * dm : 0.0;
+            const double etol = 1e-10 * fmax(1.0, Emax - Emin);
+            if (fabs(E0 - Emin) <= etol || fabs(Emax - E0) <= etol) {
+                const double gap = fmax(kPvGapRel * (Emax - Emin), 64 * jeps(E0));
+                const double left_end = fmax(Emin, E0 - gap), right_start = fmin(Emax, E0 + gap);
+                if (left_end > Emin) sg[1] = seg_power(Emin, left_end, R_L16, 16);
+                if (right_start < Emax) sg[2] = seg_power(right_start, Emax, R_L16, 16);
+            } else {
+                form = REGULAR;
+                near = 64 * jeps(E0);
+                sg[0] = seg_power(Emin, Emax, R_L32, 32);
+                const double lt = log_c(fabs(Emax - E0)) - log_c(fabs(Emin - E0));
+                scale = 2.0 / lam;
+                o.rp = f0p * lt * scale;
+                o.rm = f0m * lt * scale;
+            }
+            const double E0m = -((lam_m * lam_m + m * m - mp * mp) / 2.0) / lam_m;
+            const double c = 2.0 * kPi / lam;
+            o.ip = c * p0 * dp;
+            o.im = c * p_int(E0m, m) * dm;
+        }
+    } else {
+        // OneLoopIntegrals.jl:228-476: integrate_piecewise_hybrid's breakpoints :335-421
+        double iv[2][2] = {};
+        const int niv = sing_kpos(lam, k, m, mp, Emin, Emax, iv);
+        scale = 1.0 / k;
+        if (niv == 0) {
+            sg[2] = seg_power(Emin, Emax, R_L16, 16);
+        } else {
+            double E1 = iv[0][0], E2 = iv[0][1];
+            if (niv == 2) {
+                const double tol = 1e-12 * fmax(1.0, Emax - Emin);
+                E1 = iv[0][1];
+                E2 = pick(fabs(iv[0][1] - Emax) <= tol, iv[0][0], iv[1][0]);
+            }
+            if (E1 > Emin) sg[0] = seg_power(Emin, E1, R_R32, 32);
+            if (E2 > E1) sg[1] = seg_mid(E1, E2, R_DE, 33);
+            if (Emax > E2) sg[2] = seg_power(E2, Emax, R_L16, 16);
+            double sp = 0.0, sm = 0.0;
+#pragma unroll 1
+            for (int i = 0; i < niv; i++) {
+                const double a = pick(i != 0, iv[1][0], iv[0][0]), b = pick(i != 0, iv[1][1], iv[0][1]);
+                double apa, ama, apb, amb;
+                anti2(M, a, apa, ama);
+                anti2(M, b, apb, amb);
+                sp += apb - apa;
+                sm += (b - a) - (amb - ama);
+            }
+            const double c = kPi * jsign(lam);
+            o.ip = sp * c / k;
+            o.im = sm * c / k;
         }
     }
+    double accp = 0.0, accm = 0.0;
+#pragma unroll 1
+    for (int g = 0; g < 3; g++) {
+        const Seg S = seg_pick(g == 0, sg[0], seg_pick(g == 1, sg[1], sg[2]));
+#pragma unroll 1
+        for (int i = q; i < S.n; i += L) {
+            const double E = S.x0 + S.s * ptab[S.off + i];
+            const double w = S.s * ptab[S.off + S.n + i];
+            const double p = p_int(E, m);
+            double dp, dm, vp, vm;
+            dist2(M, E, dp, dm);
+            if (form == RATIO) {
+                const double lpE = lam + E;
+                const double common = lpE * lpE - mp * mp;
+                const double pmk = p - k, ppk = p + k;
+                const double num = common - pmk * pmk;
+                double den = common - ppk * ppk;
+                const bool tiny = fabs(den) < kEpsSeg;
+                const bool ok = isfinite(num) && isfinite(den) && !(tiny && fabs(num) < kEpsSeg);
+                if (tiny) den = (den == 0.0) ? kEpsSeg : jsign(den) * kEpsSeg;
+                const double ratio = fabs(div_p(num, den));
+                const double lt = (ok && isfinite(ratio)) ? log_p(fmax(ratio, 1e-300)) : 0.0;
+                vp = dp * lt;
+                vm = dm * lt;
+            } else {
+                vp = p * dp;
+                vm = p * dm;
+                double d = lam * E + dterm;
+                if (form == REGULAR) {
+                    d = E - E0;
+                    vp = (isfinite(vp) ? vp : 0.0) - f0p;
+                    vm = (isfinite(vm) ? vm : 0.0) - f0m;
+                    if (fabs(d) < near) {   // takes the difference quotient, below
+                        wnear += w;
+                        vp = vm = 0.0;
+                        d = 1.0;
+                    }
+                } else if (!isfinite(d) || fabs(d) < kEpsSeg) {
+                    vp = vm = 0.0;
+                    d = 1.0;
+                }
+                const double r = rcp1(d);
+                vp = div_r(vp, d, r);
+                vm = div_r(vm, d, r);
+            }
+            const double tp = isfinite(vp) ? w * vp : 0.0, tm = isfinite(vm) ? w * vm : 0.0;
+            if constexpr (L > 1) {
+                term_rows<L>()[i] = double2{tp, tm};
+            } else {
+                accp += tp;
+                accm += tm;
+            }
+        }
+        if constexpr (L > 1) add_terms<L>(S.n, accp, accm);
+    }
+    if (form == REGULAR) {
+        // nodes next to E0: the difference quotient across it
+        if constexpr (L > 1)
+            for (int d = 1; d < L; d *= 2) wnear += __shfl_xor(wnear, d, L);
+        if (wnear != 0.0) {
+            const double del = fmax(1e-7 * (Emax - Emin), near);
+            const double El = fmax(Emin, E0 - del), Er = fmin(Emax, E0 + del);
+            double lp, lm, rp, rm;
+            dist2(M, El, lp, lm);
+            dist2(M, Er, rp, rm);
+            const double pl = p_int(El, m), pr = p_int(Er, m), r = Er > El ? wnear / (Er - El) : 0.0;
+            accp += r * (pr * rp - pl * lp);
+            accm += r * (pr * rm - pl * lm);
+        }
+    }
+    o.rp += accp * scale;
+    o.rm += accm * scale;
+    return o;
 }
 
 // ---- first-order anisotropy  OneLoopIntegralsAniso.jl ---------------------
-// quark_df_dE / antiquark_df_dE / correction_cos_theta_coefficient
-//   QuarkDistribution_Aniso.jl:14-86
-__device__ double corr_coef(int sg, double p, double m, double mu, double T, double Phi, double Phib, double xi)
+// correction_cos_theta_coefficient (QuarkDistribution_Aniso.jl:14-86) of quark
+// and antiquark at (p, E): xi p^2 / (2 E) df/dE
+__device__ __forceinline__ void corr2(const Medium& M, double p, double E, double xi, double& cq, double& ca)
 {
-    const double E = sqrt(p * p + m * m);
-    const double coeff = 0.5 * xi * (p * p) / E;
-    const double beta = 1 / T;
-    const double c1 = sg == QUARK ? Phi : Phib, c2 = sg == QUARK ? Phib : Phi;
-    const double arg = sg == QUARK ? -(E - mu) * beta : -(E + mu) * beta;
-    const double e = clamp_e(exp(arg));
-    const double e2 = e * e, e3 = e2 * e;
-    const double num = c1 * e + 2 * c2 * e2 + e3;
-    const double den = 1 + 3 * c1 * e + 3 * c2 * e2 + e3;
-    const double dnum = -(c1 * e + 4 * c2 * e2 + 3 * e3);
-    const double dden = -(3 * c1 * e + 6 * c2 * e2 + 3 * e3);
-    double dfdx = dnum * den - num * dden;
-    dfdx /= den * den;
-    return coeff * (beta * dfdx);
+    double ep, em;
+    boltzmann(M, E, ep, em);
+    const double c = div_p(0.5 * xi * (p * p), E) * M.beta;
+    auto slope = [&](double e, double c1, double c2) {
+        const double e2 = e * e, e3 = e2 * e;
+        const double num = c1 * e + 2 * c2 * e2 + e3;
+        const double den = 1 + 3 * c1 * e + 3 * c2 * e2 + e3;
+        const double dnum = -(c1 * e + 4 * c2 * e2 + 3 * e3);
+        const double dden = -(3 * c1 * e + 6 * c2 * e2 + 3 * e3);
+        const double t = dnum * den - num * dden, dd = den * den;
+        return div_p(t, dd);
+    };
+    cq = c * slope(ep, M.Phi, M.Phib);
+    ca = c * slope(em, M.Phib, M.Phi);
 }
-
-// compute_coefficients  OneLoopIntegralsAniso.jl:50-61 (k > 0 branch)
-struct BcKpos {
-    int sg;
-    double lam, k, m, mp, mu, T, Phi, Phib, xi;
-    bool imag;
-    __device__ double operator()(double E) const
-    {
-        const double dc = lam * lam + 2 * lam * E + m * m - mp * mp - k * k;
-        const double p = p_int(E, m);
-        const double cx = 2 * p * k;
-        double tool;
-        if (imag) {
-            tool = kPi * dc * dc / (cx * cx * cx);
-        } else {
-            double t1 = -2 * dc / (cx * cx);
-            double t2 = dc * dc / (cx * cx * cx);
-            tool = t1 + t2 * log(fabs((cx + dc) / (cx - dc)));
-        }
-        return 2.0 * p * tool * corr_coef(sg, p, m, mu, T, Phi, Phib, xi);
-    }
-};
 
 // find_roots_AB  :207-272 -> number of roots (ascending, unique)
 __device__ int roots_AB(double lam, double k, double m, double mp, double Emin, double Emax, double r[2])
@@ -563,7 +552,7 @@ __device__ int roots_AB(double lam, double k, double m, double mp, double Emin, 
         if (fabs(b) < 1e-14) return 0;
         double E = -c / b;
         if (E >= Emin && E <= Emax && E >= m) {
-            double p = sqrt(fmax(0.0, E * E - m * m));
+            double p = sqrt_p(fmax(0.0, E * E - m * m));
             double A = 2 * k * p, B = lam * lam + 2 * lam * E + m * m - mp * mp - k * k;
             if (fabs(A + B) < 1e-10 || fabs(A - B) < 1e-10) {
                 r[0] = E;
@@ -574,195 +563,195 @@ __device__ int roots_AB(double lam, double k, double m, double mp, double Emin, 
     }
     const double D = b * b - 4 * a * c;
     if (D < 0) return 0;
-    const double sD = sqrt(D);
+    const double sD = sqrt_p(D);
     const double E12[2] = {(-b - sD) / (2 * a), (-b + sD) / (2 * a)};
-    int n = 0;
+    bool ok[2];
+#pragma unroll
     for (int i = 0; i < 2; i++) {
-        double E = E12[i];
-        if (E >= m && E >= Emin && E <= Emax) {
-            double p = sqrt(E * E - m * m);
-            double A = 2 * k * p, B = lam * lam + 2 * lam * E + m * m - mp * mp - k * k;
-            if (fabs(A + B) < 1e-10 || fabs(A - B) < 1e-10) r[n++] = E;
-        }
+        const double E = E12[i];
+        const double p = sqrt_p(E * E - m * m);
+        const double A = 2 * k * p, B = lam * lam + 2 * lam * E + m * m - mp * mp - k * k;
+        ok[i] = E >= m && E >= Emin && E <= Emax && (fabs(A + B) < 1e-10 || fabs(A - B) < 1e-10);
     }
-    if (n == 2) {
-        if (r[0] > r[1]) {
-            double t = r[0];
-            r[0] = r[1];
-            r[1] = t;
-        }
-        if (r[0] == r[1]) n = 1;
+    if (ok[0] && ok[1]) {
+        r[0] = fmin(E12[0], E12[1]);
+        r[1] = fmax(E12[0], E12[1]);
+        return r[0] == r[1] ? 1 : 2;
     }
-    return n;
+    r[0] = pick(ok[0], E12[0], E12[1]);
+    return (ok[0] || ok[1]) ? 1 : 0;
 }
 
-// tilde_B0_correction_k_zero  :133-190
+// tilde_B0_correction for the quark (plus) and antiquark (minus) coefficient:
+// k = 0 :133-190, k > 0 :307-375
 template <int L>
-__device__ void tilde_Bc_k0(const Phys& P, const Tabs& q, int sg, double lam, double m, double mp, double mu, double T,
-                            double Phi, double Phib, double xi, double& re, double& im)
+__device__ Pair tilde_Bc(const Phys& P, const Medium& M, double lam, double k, double m, double mp, double xi, int q)
 {
     const double Emin = m, Emax = e_cut(P, m);
-    const double cE = 2.0 * lam;
-    const double dc = lam * lam + m * m - mp * mp;
-    bool has = false;
-    double E0 = 0.0;
-    if (cE != 0.0) {
-        double v = -dc / cE;
-        if (isfinite(v) && v >= Emin && v <= Emax) {
-            has = true;
-            E0 = v;
+    const bool at_rest = !(k > kEpsK);
+    Seg sg[5] = {};              // 3, 4: the imaginary part's
+    Pair o{0.0, 0.0, 0.0, 0.0};
+    double A0p = 0.0, A0m = 0.0;
+    const double cE = 2.0 * lam, dc0 = lam * lam + m * m - mp * mp;
+    // sqrt(p^2 + m^2): the node energy, but for a negative mass, whose momentum is clamped (p_int)
+    auto energy = [&](double E, double p) { return m >= 0.0 ? E : sqrt_p(p * p + m * m); };
+    if (at_rest) {
+        const double E0 = -dc0 / cE;
+        if (cE != 0.0 && isfinite(E0) && E0 >= Emin && E0 <= Emax) {
+            const double p0 = p_int(E0, m);
+            corr2(M, p0, energy(E0, p0), xi, A0p, A0m);
+            A0p *= (4.0 / 3.0) * p0;
+            A0m *= (4.0 / 3.0) * p0;
+            const double lt = (log_c(fabs(cE * Emax + dc0)) - log_c(fabs(cE * Emin + dc0))) / cE;
+            o.rp = A0p * lt;
+            o.rm = A0m * lt;
+            // imag_integrand_k_zero  :98-112
+            const double c = kPi / cE;
+            o.ip = c * A0p;
+            o.im = c * A0m;
         }
-    }
-    auto numer = [&](double E) {
-        double p = p_int(E, m);
-        return (4.0 / 3.0) * p * corr_coef(sg, p, m, mu, T, Phi, Phib, xi);
-    };
-    double sum = 0.0;
-    const double A0 = has ? numer(E0) : 0.0;
-    auto term = [&](int i) {
-        double E = ((Emax - Emin) * q.x32[i] + (Emax + Emin)) / 2.0;
-        double w = q.w32[i] * (Emax - Emin) / 2.0;
-        double den = cE * E + dc;
-        double v = numer(E) - A0;
-        return w * ((isfinite(den) && isfinite(v)) ? v / den : 0.0);
-    };
-    if constexpr (L > 1)
-        sum = ordered_sum<L, 32>(sum, term);
-    else
-        for (int i = 0; i < 32; i++) sum += term(i);
-    if (has) sum += A0 / cE * (log(fabs(cE * Emax + dc)) - log(fabs(cE * Emin + dc)));
-    re = sum;
-    // imag_integrand_k_zero  :98-112
-    const double Ep = -dc / cE;
-    if (!(Ep >= m && Ep <= e_cut(P, m))) {
-        im = 0.0;
+        sg[0] = Seg{(Emax + Emin) / 2.0, (Emax - Emin) / 2.0, R_G32, 32};
     } else {
-        const double pp = p_int(Ep, m);
-        im = kPi * (4.0 / 3.0) * pp / cE * corr_coef(sg, pp, m, mu, T, Phi, Phib, xi);
-    }
-}
-
-// tilde_B0_correction_k_positive  :307-375
-template <int L>
-__device__ void tilde_Bc_kpos(const Phys& P, const Tabs& q, int sg, double lam, double k, double m, double mp,
-                              double mu, double T, double Phi, double Phib, double xi, double& re, double& im)
-{
-    const double Emin = m, Emax = e_cut(P, m);
-    double ivi[2][2];
-    const int nimag = sing_kpos(lam, k, m, mp, Emin, Emax, ivi);
-    double roots[2];
-    const int nr = roots_AB(lam, k, m, mp, Emin, Emax, roots);
-    // build_intervals_from_roots  :275-292
-    const double del = fmax(1e-10, 1e-8 * (Emax - Emin));
-    double ep[6];
-    int ne = 0;
-    ep[ne++] = Emin;
-    for (int i = 0; i < nr; i++) {
-        ep[ne++] = roots[i] - del;
-        ep[ne++] = roots[i] + del;
-    }
-    ep[ne++] = Emax;
-    double iv[3][2];
-    int niv = 0;
-    for (int i = 0; i + 1 < ne; i += 2)
-        if (ep[i + 1] > ep[i] + 1e-16) {
-            iv[niv][0] = ep[i];
-            iv[niv][1] = ep[i + 1];
-            niv++;
+        double iv[2][2] = {}, r[2] = {};
+        const int ni = sing_kpos(lam, k, m, mp, Emin, Emax, iv);
+        const int nr = roots_AB(lam, k, m, mp, Emin, Emax, r);
+        // build_intervals_from_roots  :275-292
+        const double del = fmax(1e-10, 1e-8 * (Emax - Emin));
+        const double b0 = nr >= 1 ? r[0] - del : Emax, a1 = r[0] + del, b1 = nr == 2 ? r[1] - del : Emax, a2 = r[1] + del;
+        const bool v0 = b0 > Emin + 1e-16, v1 = nr >= 1 && b1 > a1 + 1e-16, v2 = nr == 2 && Emax > a2 + 1e-16;
+        if (nr == 0) {
+            if (v0) sg[2] = seg_power(Emin, Emax, R_L16, 16);
+        } else {
+            // the first of several intervals clusters to its right end, the last to its left, others to both
+            const int nv = (v0 ? 1 : 0) + (v1 ? 1 : 0) + (v2 ? 1 : 0);
+            if (v0) sg[0] = nv == 1 ? seg_mid(Emin, b0, R_DE, 33) : seg_power(Emin, b0, R_R32, 32);
+            if (v1) sg[1] = (nv == 1 || (v0 && v2)) ? seg_mid(a1, b1, R_DE, 33)
+                          : (v0 ? seg_power(a1, b1, R_L16, 16) : seg_power(a1, b1, R_R32, 32));
+            if (v2) sg[2] = nv == 1 ? seg_mid(a2, Emax, R_DE, 33) : seg_power(a2, Emax, R_L16, 16);
         }
-    const BcKpos fr{sg, lam, k, m, mp, mu, T, Phi, Phib, xi, false};
-    double real = 0.0;
-    for (int i = 0; i < niv; i++) {
-        int pos;
-        if (niv == 1) pos = nr == 0 ? NONE : BOTH;
-        else if (i == 0) pos = RIGHT;
-        else if (i == niv - 1) pos = LEFT;
-        else pos = BOTH;
-        const int n = (nr == 0) ? 16 : (pos == LEFT ? 16 : 32);
-        real += hybrid<L>(fr, q, iv[i][0], iv[i][1], pos, n);
+        if (ni > 0) sg[3] = Seg{(iv[0][0] + iv[0][1]) / 2, (iv[0][1] - iv[0][0]) / 2, R_G16, 16};
+        if (ni > 1) sg[4] = Seg{(iv[1][0] + iv[1][1]) / 2, (iv[1][1] - iv[1][0]) / 2, R_G16, 16};
     }
-    double imag = 0.0;
-    if (nimag > 0) {
-        const BcKpos fi{sg, lam, k, m, mp, mu, T, Phi, Phib, xi, true};
-        for (int j = 0; j < nimag; j++) {
-            const double E1 = ivi[j][0], E2 = ivi[j][1];
-            const double half = (E2 - E1) / 2, center = (E1 + E2) / 2;
-            if constexpr (L > 1) {
-                imag = ordered_sum<L, 16>(imag, [&](int i) {
-                    double x = center + half * q.x16[i];
-                    double w = q.w16[i] * half;
-                    double v = fi(x);
-                    return isfinite(v) ? w * v : 0.0;
-                });
+    double sp = 0.0, sm = 0.0;
+#pragma unroll 1
+    for (int g = 0; g < 5; g++) {
+        const Seg S = seg_pick(g == 0, sg[0], seg_pick(g == 1, sg[1], seg_pick(g == 2, sg[2], seg_pick(g == 3, sg[3], sg[4]))));
+#pragma unroll 1
+        for (int i = q; i < S.n; i += L) {
+            const double E = S.x0 + S.s * ptab[S.off + i];
+            const double w = S.s * ptab[S.off + S.n + i];
+            const double p = p_int(E, m);
+            double vp, vm, tp, tm;
+            corr2(M, p, energy(E, p), xi, vp, vm);
+            if (at_rest) {
+                const double den = cE * E + dc0;
+                vp = (4.0 / 3.0) * p * vp - A0p;
+                vm = (4.0 / 3.0) * p * vm - A0m;
+                // a zero denominator (lambda = 0, equal masses) stays infinite
+                const double r = rcp1(den);
+                const double up = den == 0.0 ? vp * __builtin_inf() : div_r(vp, den, r);
+                const double um = den == 0.0 ? vm * __builtin_inf() : div_r(vm, den, r);
+                tp = w * ((isfinite(den) && isfinite(vp)) ? up : 0.0);
+                tm = w * ((isfinite(den) && isfinite(vm)) ? um : 0.0);
             } else {
-                for (int i = 0; i < 16; i++) {
-                    double x = center + half * q.x16[i];
-                    double w = q.w16[i] * half;
-                    double v = fi(x);
-                    if (isfinite(v)) imag += w * v;
+                // compute_coefficients, real_integral_tool, imag_integral_tool  :26-61
+                const double dc = lam * lam + 2 * lam * E + m * m - mp * mp - k * k;
+                const double cx = 2 * p * k, ic = rcp1(cx), ic2 = ic * ic;
+                const double t2 = div_r(dc * dc, cx * cx * cx, ic2 * ic);
+                double tool = kPi * t2;
+                if (g < 3) {
+                    const double ratio = fabs(div_p(cx + dc, cx - dc));
+                    const bool ok = ratio > 0.0 && isfinite(ratio);
+                    tool = ok ? div_r(-2 * dc, cx * cx, ic2) + t2 * log_p(ok ? ratio : 1.0) : __builtin_nan("");
                 }
+                tool *= 2.0 * p;
+                vp *= tool;
+                vm *= tool;
+                tp = isfinite(vp) ? w * vp : 0.0;
+                tm = isfinite(vm) ? w * vm : 0.0;
+            }
+            if constexpr (L > 1) {
+                term_rows<L>()[i] = double2{tp, tm};
+            } else {
+                sp += tp;
+                sm += tm;
             }
         }
-        imag *= jsign(lam);
-    }
-    re = real;
-    im = imag;
-}
-
-template <int L>
-__device__ void tilde_Bc(const Phys& P, const Tabs& q, int sg, double lam, double k, double m, double mp, double mu,
-                         double T, double Phi, double Phib, double xi, double& re, double& im)
-{
-    if (k > kEpsK) tilde_Bc_kpos<L>(P, q, sg, lam, k, m, mp, mu, T, Phi, Phib, xi, re, im);
-    else tilde_Bc_k0<L>(P, q, sg, lam, m, mp, mu, T, Phi, Phib, xi, re, im);
-}
-
-// B0_correction  OneLoopIntegralsAniso.jl:396-413 (all four terms added):
-// dB~q(-l; m1, m2, mu1) + dB~qbar(l; m1, m2, mu1) + dB~q(l; m2, m1, mu2)
-// + dB~qbar(-l; m2, m1, mu2).
-template <int L = 1>
-__device__ void B0_corr(const Phys& P, const Tabs& q, double lam, double k, double m1, double m2, double mu1,
-                        double mu2, double T, double Phi, double Phib, double xi, double& re, double& im)
-{
-    re = 0.0;
-    im = 0.0;
-#pragma unroll 1
-    for (int t = 0; t < 4; t++) {
-        const bool swap = t >= 2;
-        const double l = (t == 0 || t == 3) ? -lam : lam;
-        double r, i;
-        tilde_Bc<L>(P, q, (t & 1) ? ANTIQUARK : QUARK, l, k, swap ? m2 : m1, swap ? m1 : m2, swap ? mu2 : mu1, T, Phi,
-                 Phib, xi, r, i);
-        re += r;
-        im += i;
-    }
-}
-
-// The symmetrised B0 (+ B0_correction) of polarization_aniso
-//   PolarizationAniso.jl:29-54
-template <int L = 1>
-__device__ void b0_total(const Phys& P, const Tabs& q, double k0, double k, double m1, double m2, double mu1,
-                         double mu2, double T, double Phi, double Phib, double xi, int num_s, double& br, double& bi)
-{
-    // lambda = k0 + mu1 - mu2; num_s = 1 averages with lambda' = -k0 + mu1 - mu2
-    const int nv = num_s == 1 ? 2 : 1;
-    double vr[2], vi[2];
-#pragma unroll 1
-    for (int v = 0; v < nv; v++) {
-        const double l = (v == 0 ? k0 : -k0) + mu1 - mu2;
-        B0<L>(P, q, l, k, m1, mu1, m2, mu2, T, Phi, Phib, vr[v], vi[v]);
-    }
-    br = nv == 2 ? 0.5 * (vr[0] + vr[1]) : vr[0];
-    bi = nv == 2 ? 0.5 * (vi[0] + vi[1]) : vi[0];
-    if (fabs(xi) > kEpsSeg) {
-#pragma unroll 1
-        for (int v = 0; v < nv; v++) {
-            const double l = (v == 0 ? k0 : -k0) + mu1 - mu2;
-            B0_corr<L>(P, q, l, k, m1, m2, mu1, mu2, T, Phi, Phib, xi, vr[v], vi[v]);
+        if constexpr (L > 1) add_terms<L>(S.n, sp, sm);
+        if (g == 2) {
+            o.rp += sp;
+            o.rm += sm;
+            sp = sm = 0.0;
         }
-        br += nv == 2 ? 0.5 * (vr[0] + vr[1]) : vr[0];
-        bi += nv == 2 ? 0.5 * (vi[0] + vi[1]) : vi[0];
     }
+    const double s = jsign(lam);
+    o.ip += sp * s;
+    o.im += sm * s;
+    return o;
+}
+
+// B0 (part 1), B0_correction (part 2) or both summed (part 3), symmetrised
+// over +-k0 for num_s = 1:
+//   B0  OneLoopIntegrals.jl:489-503: B~+(-l; m1, m2, mu1) - B~-(l; m1, m2, mu1)
+//       + B~+(l; m2, m1, mu2) - B~-(-l; m2, m1, mu2)
+//   B0_correction  OneLoopIntegralsAniso.jl:396-413: the same arguments with
+//       the quark / antiquark coefficients, all four added
+//   polarization_aniso  PolarizationAniso.jl:29-54: l = k0 + mu1 - mu2, averaged with l' = -k0 + mu1 - mu2
+// With mu1 = mu2 the plus and minus terms pair up at equal (lambda, m): two
+// evaluations for equal masses, four for the average, instead of four and
+// eight.  A group of L x S lanes gives every evaluation L lanes and runs S of
+// them at once; the evaluations are summed in their order in every lane.
+template <int L = 1, int S = 1>
+__device__ void b0_sum(const Phys& P, int part, double l0, double l1, double k, double m1, double m2, double mu1,
+                       double mu2, double T, double Phi, double Phib, double xi, int nv, double& br, double& bi)
+{
+    const int gl = (int)(threadIdx.x & (L * S - 1)), q = gl & (L - 1);
+    const bool eqmu = mu1 == mu2, two = eqmu && m1 == m2 && nv == 1;
+    const bool four = !two && eqmu && nv == 2;
+    const int ne = two ? 2 : (four ? 4 : 4 * nv);
+    const double wgt = nv == 2 ? 0.5 : 1.0;
+    double r = 0.0, i = 0.0;
+#pragma unroll 1
+    for (int e0 = 0; e0 < ne; e0 += S) {
+        const int e = e0 + gl / L, t = e & 3;
+        const bool swap = t >= 2, neg = t == 0 || t == 3;
+        // the plus and the minus term's l; with four, l1 = -l0 to the last bits
+        const double l = pick(e >= 4, l1, l0), lp = four && (t & 1) ? -l1 : l, lm = four && !(t & 1) ? -l1 : l;
+        const bool both = two || four;
+        const bool plus = both || !(t & 1), minus = both || (t & 1);
+        double br0 = 0.0, bi0 = 0.0, br1 = 0.0, bi1 = 0.0;
+        if (S == 1 || e < ne) {
+            const Medium M = make_medium(swap ? mu2 : mu1, T, Phi, Phib);
+            const double lam = neg ? -lp : lp, lam_m = neg ? -lm : lm, ma = swap ? m2 : m1, mb = swap ? m1 : m2;
+            if (part & 1) {
+                const Pair b = tilde_B0<L>(P, M, lam, both ? lam_m : lam, k, ma, mb, q);
+                br0 = wgt * ((plus ? b.rp : 0.0) - (minus ? b.rm : 0.0));
+                bi0 = wgt * ((plus ? b.ip : 0.0) - (minus ? b.im : 0.0));
+            }
+            if (part & 2) {
+                const Pair b = tilde_Bc<L>(P, M, lam, k, ma, mb, xi, q);
+                br1 = wgt * ((plus ? b.rp : 0.0) + (minus ? b.rm : 0.0));
+                bi1 = wgt * ((plus ? b.ip : 0.0) + (minus ? b.im : 0.0));
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < S; j++) {
+            r += S > 1 ? __shfl(br0, j * L, L * S) : br0;
+            i += S > 1 ? __shfl(bi0, j * L, L * S) : bi0;
+            r += S > 1 ? __shfl(br1, j * L, L * S) : br1;
+            i += S > 1 ? __shfl(bi1, j * L, L * S) : bi1;
+        }
+    }
+    br = r;
+    bi = i;
+}
+
+template <int L = 1, int S = 1>
+__device__ void b0_total(const Phys& P, double k0, double k, double m1, double m2, double mu1, double mu2, double T,
+                         double Phi, double Phib, double xi, int num_s, double& br, double& bi)
+{
+    b0_sum<L, S>(P, fabs(xi) > kEpsSeg ? 3 : 1, k0 + mu1 - mu2, -k0 + mu1 - mu2, k, m1, m2, mu1, mu2, T, Phi, Phib, xi, num_s == 1 ? 2 : 1, br,
+                 bi);
 }
 
 // polarization_aniso / polarization_with_width  PolarizationAniso.jl:22-118
@@ -783,6 +772,23 @@ __device__ void pi_value(const Phys& P, int channel, int width, double k0, doubl
     }
     re = factor * real;
     im = factor * imag;
+}
+
+// PNJL distributions  QuarkDistribution.jl:14-60
+__device__ __forceinline__ double dist_ratio(double e, double c1, double c2)
+{
+    double e2 = e * e, e3 = e2 * e;
+    return (c1 * e + 2 * c2 * e2 + e3) / (1 + 3 * c1 * e + 3 * c2 * e2 + e3);
+}
+
+__device__ __forceinline__ double quark_f(double E, double mu, double T, double Phi, double Phib)
+{
+    return dist_ratio(clamp_e(exp(-(E - mu) * (1 / T))), Phi, Phib);
+}
+
+__device__ __forceinline__ double antiquark_f(double E, double mu, double T, double Phi, double Phib)
+{
+    return dist_ratio(clamp_e(exp(-(E + mu) * (1 / T))), Phib, Phi);
 }
 
 // A / A_aniso  OneLoopIntegrals.jl:507-543, OneLoopIntegralsAniso.jl:446-467
@@ -822,49 +828,47 @@ __device__ double A_value(const Phys& P, double m, double mu, double T, double P
 }
 
 // ---- kernels -----------------------------------------------------------------
-__device__ __forceinline__ void load_tabs(double* lds, const double* tab)
+__device__ __forceinline__ void load_tabs(const double* tab)
 {
-    for (int i = threadIdx.x; i < kTabLen; i += blockDim.x) lds[i] = tab[i];
+    for (int i = threadIdx.x; i < kTabLen; i += blockDim.x) ptab[i] = tab[i];
     __syncthreads();
 }
 
-// query i = thread / stride (stride 1, or 64: one query per wavefront)
+// query i = thread / (L S stride): L x S lanes per query (stride 1), or one
+// query per wavefront on one lane (stride 64, for counting FLOPs)
+template <int L, int S>
 __global__ void __launch_bounds__(256, 3) query_kernel(Phys P, const double* tab, int64_t n, const pnjl_pol_query* qs,
                                                     double* re, double* im, int stride)
 {
-    __shared__ double lds[kTabLen];
-    load_tabs(lds, tab);
+    load_tabs(tab);
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t % stride) return;
-    const int64_t i = t / stride;
+    const int64_t i = t / (L * S * stride);
     if (i >= n) return;
-    const Tabs q = make_tabs(lds);
     const pnjl_pol_query a = qs[i];
-    if (a.channel != PNJL_CHANNEL_P && a.channel != PNJL_CHANNEL_S) {
-        re[i] = im[i] = __builtin_nan("");   // unsupported channel
-        return;
+    double r = __builtin_nan(""), m = __builtin_nan("");   // unsupported channel
+    if (a.channel == PNJL_CHANNEL_P || a.channel == PNJL_CHANNEL_S) {
+        double br, bi;
+        b0_total<L, S>(P, a.k0, a.k, a.m1, a.m2, a.mu1, a.mu2, a.T, a.Phi, a.Phib, a.xi, a.num_s, br, bi);
+        pi_value(P, a.channel, a.width, a.k0, a.gamma, a.k, a.m1, a.m2, a.k0 + a.mu1 - a.mu2, a.A1 + a.A2, br, bi, r,
+                 m);
     }
-    double br, bi;
-    b0_total(P, q, a.k0, a.k, a.m1, a.m2, a.mu1, a.mu2, a.T, a.Phi, a.Phib, a.xi, a.num_s, br, bi);
-    pi_value(P, a.channel, a.width, a.k0, a.gamma, a.k, a.m1, a.m2, a.k0 + a.mu1 - a.mu2, a.A1 + a.A2, br, bi, re[i],
-             im[i]);
+    if (threadIdx.x % (L * S) == 0) {
+        re[i] = r;
+        im[i] = m;
+    }
 }
 
 __global__ void __launch_bounds__(256, 3) b0_kernel(Phys P, const double* tab, int64_t n, const double* args, int corr,
                                                  double* re, double* im)
 {
-    __shared__ double lds[kTabLen];
-    load_tabs(lds, tab);
+    load_tabs(tab);
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const Tabs q = make_tabs(lds);
-    if (!corr) {
-        const double* a = args + i * 9;
-        B0(P, q, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], re[i], im[i]);
-    } else {
-        const double* a = args + i * 10;
-        B0_corr(P, q, a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9], re[i], im[i]);
-    }
+    // B0(lambda, k, m1, mu1, m2, mu2, T, Phi, Phib), B0_correction(lambda, k, m1, m2, mu1, mu2, T, Phi, Phib, xi)
+    const double* a = args + i * (corr ? 10 : 9);
+    b0_sum(P, corr ? 2 : 1, a[0], a[0], a[1], a[2], corr ? a[3] : a[4], corr ? a[4] : a[3], a[5], a[6], a[7], a[8],
+           corr ? a[9] : 0.0, 1, re[i], im[i]);
 }
 
 __global__ void __launch_bounds__(256) a_kernel(Phys P, int64_t n, const double* args, int np, const double* xp,
@@ -897,23 +901,22 @@ __global__ void __launch_bounds__(256) grid_a_kernel(Phys P, int npts, const pnj
 #ifndef PNJL_GRID_TILE_K
 #define PNJL_GRID_TILE_K 8
 #endif
-// grid: one thread per (point, pair, k0, k); both channels written.
-// The quadrature kernels are held to 3 waves per SIMD (168 VGPRs, a few
-// spills): latency hiding pays more than the spill traffic costs.
+// grid: L x S lanes per (point, pair, k0, k); both channels written.
+// The quadrature kernels are held to 3 waves per SIMD (168 VGPRs): latency
+// hiding pays more than a few spills cost.
+template <int L, int S>
 __global__ void __launch_bounds__(256, 3) grid_pi_kernel(Phys P, const double* tab, int npts, const pnjl_pol_point* pts,
                                                       const double* A, int nk0, const double* k0s, int nk,
                                                       const double* ks, double* re, double* im)
 {
-    __shared__ double lds[kTabLen];
-    load_tabs(lds, tab);
-    const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    load_tabs(tab);
+    const int64_t tid = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / (L * S);
     const int64_t plane = (int64_t)nk0 * nk;
     if (tid >= (int64_t)npts * 3 * plane) return;
-    const Tabs q = make_tabs(lds);
     int64_t j, i0;
     int pair, pt;
     constexpr int TK = PNJL_GRID_TILE_K, T0 = 64 / TK;
-    if (TK < 64 && nk % TK == 0 && nk0 % T0 == 0) {
+    if (L * S == 1 && TK < 64 && nk % TK == 0 && nk0 % T0 == 0) {
         // a wavefront takes a T0 (k0) x TK (k) tile of one (point, pair) plane
         const int64_t lane = tid & 63, tile = tid >> 6;
         const int64_t ntk = nk / TK, tiles = ntk * (nk0 / T0);
@@ -932,7 +935,8 @@ __global__ void __launch_bounds__(256, 3) grid_pi_kernel(Phys P, const double* t
     const double A12 = A[pt * 2 + (pair == 2 ? 1 : 0)] + A[pt * 2 + (pair == 0 ? 0 : 1)];
     const double k0 = k0s[i0], k = ks[j];
     double br, bi;
-    b0_total(P, q, k0, k, m1, m2, s.mu, s.mu, s.T, s.Phi, s.Phib, s.xi, pair, br, bi);
+    b0_total<L, S>(P, k0, k, m1, m2, s.mu, s.mu, s.T, s.Phi, s.Phib, s.xi, pair, br, bi);
+    if (threadIdx.x % (L * S)) return;
     const int64_t base = ((int64_t)pt * 3 + pair) * 2 * plane + i0 * nk + j;
     for (int c = 0; c < 2; c++) {
         double r, m;
@@ -1112,28 +1116,31 @@ __global__ void __launch_bounds__(256) prop_scatter_kernel(int64_t n, const pnjl
 // pair.  pib[i*12 + 2*slot] as in pnjl_polarization_grid's order.  Threads
 // past the worklist's length (offs[kPropBuckets]) exit; stride 64 puts one
 // item per wavefront, for counting FLOPs.
+template <int L, int S>
 __global__ void __launch_bounds__(256, 3) prop_pi_kernel(Phys P, const double* tab, const pnjl_prop_query* qs,
                                                       const unsigned* items, const unsigned* offs, double* pib,
                                                       int stride)
 {
-    __shared__ double lds[kTabLen];
-    load_tabs(lds, tab);
+    const int64_t per = (int64_t)L * S * stride;   // threads per item
+    const int64_t total = (int64_t)offs[kPropBuckets];
+    if ((int64_t)blockIdx.x * blockDim.x >= total * per) return;   // uniform per block
+    load_tabs(tab);
     const int64_t ts = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (ts % stride) return;
-    const int64_t t = ts / stride;
-    if (t >= (int64_t)offs[kPropBuckets]) return;
+    const int64_t t = ts / per;
+    if (t >= total) return;
     const unsigned code = items[t];
     const int pair = (int)(code % 3u);
     const int64_t i = code / 3u;
     const pnjl_prop_query a = qs[i];
     const unsigned need = item_need(a, pair);
     double* o = pib + i * 12 + 4 * pair;
-    const Tabs q = make_tabs(lds);
     const double m1 = pair == 2 ? a.m_s : a.m_u, m2 = pair == 0 ? a.m_u : a.m_s;
     const double mu1 = pair == 2 ? a.mu_s : a.mu_u, mu2 = pair == 0 ? a.mu_u : a.mu_s;
     const double A1 = pair == 2 ? a.A_s : a.A_u, A2 = pair == 0 ? a.A_u : a.A_s;
     double br, bi;
-    b0_total(P, q, a.k0, a.k, m1, m2, mu1, mu2, a.T, a.Phi, a.Phib, a.xi, pair, br, bi);
+    b0_total<L, S>(P, a.k0, a.k, m1, m2, mu1, mu2, a.T, a.Phi, a.Phib, a.xi, pair, br, bi);
+    if (threadIdx.x % (L * S)) return;
     for (int c = 0; c < 2; c++) {
         if (need & (1u << c))
             pi_value(P, c == 0 ? PNJL_CHANNEL_P : PNJL_CHANNEL_S, 0, a.k0, 0.0, a.k, m1, m2, a.k0 + mu1 - mu2, A1 + A2,
@@ -1210,17 +1217,16 @@ __device__ __forceinline__ int mass_pairs(int m, int* pairs)
 
 // B0 (symmetrised for u sbar, + correction) of the meson's pairs at k0
 //   MesonMass.jl:34-60, :222-231 (MesonMass passes num_s 0 for s sbar, equivalent to 2)
-template <int L = 1>
-__device__ __noinline__ void mass_b0(const Phys& P, const Tabs&, const pnjl_mass_query& a, double k0, MassB0& B)
+template <int L>
+__device__ __forceinline__ void mass_b0(const Phys& P, const pnjl_mass_query& a, double k0, MassB0& B)
 {
-    const Tabs T = make_tabs(mass_tab);
     int pairs[2];
     const int np = mass_pairs(a.meson, pairs);
 #pragma unroll 1
     for (int j = 0; j < np; j++) {
         double m1, m2, mu1, mu2, A12;
         mass_pair(a, pairs[j], m1, m2, mu1, mu2, A12);
-        b0_total<L>(P, T, k0, a.k, m1, m2, mu1, mu2, a.T, a.Phi, a.Phib, a.xi, pairs[j] == 1 ? 1 : 0, B.r[j], B.i[j]);
+        b0_total<L>(P, k0, a.k, m1, m2, mu1, mu2, a.T, a.Phi, a.Phib, a.xi, pairs[j] == 1 ? 1 : 0, B.r[j], B.i[j]);
     }
 }
 
@@ -1265,29 +1271,8 @@ __device__ void mass_residual(const Phys& P, const pnjl_mass_query& a, const mes
     f[1] = res.i;
 }
 
-// central finite differences (FiniteDiff): J[:, j] = (f(x + e_j h) - f(x - e_j h)) / 2h;
-// Bx holds B0 at x[0] (the gamma column needs no new B0)
-__device__ void mass_jac(const Phys& P, const Tabs& T, const pnjl_mass_query& a, const meson::KCoef& k,
-                         const double* x, const MassB0& Bx, double J[2][2])
-{
-    for (int j = 0; j < 2; j++) {
-        const double h = fmax(kFdStep * fabs(x[j]), kFdStep);
-        double xp[2] = {x[0], x[1]}, xm[2] = {x[0], x[1]}, fp[2], fm[2];
-        xp[j] = x[j] + h;
-        xm[j] = x[j] - h;
-        if (j == 0) {
-            MassB0 Bp, Bm;
-            mass_b0(P, T, a, xp[0], Bp);
-            mass_b0(P, T, a, xm[0], Bm);
-            mass_residual(P, a, k, Bp, xp[0], xp[1], fp);
-            mass_residual(P, a, k, Bm, xm[0], xm[1], fm);
-        } else {
-            mass_residual(P, a, k, Bx, xp[0], xp[1], fp);
-            mass_residual(P, a, k, Bx, xm[0], xm[1], fm);
-        }
-        for (int i = 0; i < 2; i++) J[i][j] = (fp[i] - fm[i]) / (2.0 * h);
-    }
-}
+// step of the central finite differences (FiniteDiff) at x
+__device__ __forceinline__ double fd_step(double x) { return fmax(kFdStep * fabs(x), kFdStep); }
 
 __device__ __forceinline__ double wnorm2(const double* d, const double* v)
 {
@@ -1350,7 +1335,7 @@ struct MassState {
 };
 
 // solve_meson_mass  MesonMass.jl:241-276 with NLsolve's trust region (dogleg,
-// autoscale, factor 1) and a central-difference Jacobian; one thread per query.
+// autoscale, factor 1) and a central-difference Jacobian.
 // out[i*6] = (mass, gamma, residual_norm (inf), converged, iterations, exception)
 //
 // The queries run in phases of growing iteration budgets (16, 16, 32, ...,
@@ -1359,85 +1344,152 @@ struct MassState {
 // phase.  The searches differ by orders of magnitude in length (most stop in
 // a few dozen iterations, some run NLsolve's full 1000), so one launch would
 // hold every wavefront for its longest query; the phases keep the long ones
-// packed together.  A query's arithmetic is the same as in one uninterrupted
-// loop.  stride 64 puts one query per wavefront, for counting FLOPs.
-// 3 waves per SIMD (168 VGPRs, some spilled): the extra waves hide the
-// quadratures' latency (1.5x over 256 VGPRs at 1 wave).
-__global__ void __launch_bounds__(256, 3) mass_kernel(Phys P, const double* tab, int64_t n,
-                                                   const pnjl_mass_query* qs, const double* kc, double G, double K,
+// packed together.
+//
+// G lanes per query.  An iteration needs B0 at the trial k0 and at k0 +- h for
+// the Jacobian's k0 column: with 16 or 64 lanes, four sub-groups evaluate the
+// three at once (the fourth repeats the first), each splitting its nodes over
+// G/4 lanes; one lane (for counting FLOPs, stride 64: one query per wavefront)
+// takes them one after the other.  Every lane runs the same control logic on
+// the same values, so a query's arithmetic does not depend on G.  The time is
+// that of the longest searches (NLsolve's 1000 iterations), so the residual
+// code is inlined into one trip loop: nothing of it goes through memory.
+// 18 432 queries (48 x 48 points, 8 mesons): 65.6 -> 13.0 ms; 524 288: 168 ->
+// 98 ms.  Giving sub-groups several evaluations at once instead of all their
+// lanes to one (8 x 2, 4 x 4 of 16 lanes) took 14.7 and 24.3 ms.
+// The residual f at x and the Jacobian J there by central finite differences
+// (FiniteDiff): J[:, j] = (f(x + e_j h) - f(x - e_j h)) / 2h, from B0 at x[0]
+// and x[0] +- h (the gamma column needs no new B0).  A group's sub-groups
+// evaluate B0 at the three, then the lanes of each eight take one of the five
+// residuals each (x, x[0] +- h, x[1] +- h; the rest repeat the first), and the
+// group exchanges them.
+template <int G>
+__device__ __forceinline__ void mass_group(const Phys& P, const pnjl_mass_query& a, const meson::KCoef& k,
+                                           const double* x, double* f, double J[2][2])
+{
+    constexpr int kSub = G == 1 ? 1 : G / 4;   // lanes per B0
+    const double h0 = fd_step(x[0]), h1 = fd_step(x[1]);
+    if constexpr (G == 1) {
+        MassB0 Bx;
+        double s[2];
+#pragma unroll 1
+        for (int w = 0; w < 5; w++) {
+            const double k0 = w == 1 ? x[0] + h0 : (w == 2 ? x[0] - h0 : x[0]);
+            const double ga = w == 3 ? x[1] + h1 : (w == 4 ? x[1] - h1 : x[1]);
+            MassB0 B = Bx;
+            if (w < 3) mass_b0<1>(P, a, k0, B);
+            if (w == 0) Bx = B;
+            double g[2];
+            mass_residual(P, a, k, B, k0, ga, g);
+            for (int i = 0; i < 2; i++) {
+                if (w == 0) f[i] = g[i];
+                else if (w == 1 || w == 3) s[i] = g[i];
+                else if (w == 2) J[i][0] = (s[i] - g[i]) / (2.0 * h0);
+                else J[i][1] = (s[i] - g[i]) / (2.0 * h1);
+            }
+        }
+    } else {
+        const int gl = (int)(threadIdx.x % G), sub = gl / kSub, w = gl & 7;
+        MassB0 B;
+        mass_b0<kSub>(P, a, sub == 1 ? x[0] + h0 : (sub == 2 ? x[0] - h0 : x[0]), B);
+        const int from = w == 1 ? kSub : (w == 2 ? 2 * kSub : 0);
+        for (int j = 0; j < 2; j++) {
+            B.r[j] = __shfl(B.r[j], from, G);
+            B.i[j] = __shfl(B.i[j], from, G);
+        }
+        double g[2];
+        mass_residual(P, a, k, B, w == 1 ? x[0] + h0 : (w == 2 ? x[0] - h0 : x[0]),
+                      w == 3 ? x[1] + h1 : (w == 4 ? x[1] - h1 : x[1]), g);
+        for (int i = 0; i < 2; i++) {
+            f[i] = __shfl(g[i], 0, G);
+            J[i][0] = (__shfl(g[i], 1, G) - __shfl(g[i], 2, G)) / (2.0 * h0);
+            J[i][1] = (__shfl(g[i], 3, G) - __shfl(g[i], 4, G)) / (2.0 * h1);
+        }
+    }
+}
+
+template <int G>
+__global__ void __launch_bounds__(256, G == 1 ? 3 : 2) mass_kernel(Phys P, const double* tab, int64_t n,
+                                                   const pnjl_mass_query* qs, const double* kc, double Gc, double K,
                                                    int Nc, double* out, int stride, MassState* states,
                                                    const int32_t* in_list, const unsigned* in_count,
                                                    int32_t* out_list, unsigned* out_count, int budget)
 {
-    double* const lds = mass_tab;
-    load_tabs(lds, tab);
+    const bool first = (in_list == nullptr);
+    const int64_t count = first ? n : (int64_t)*in_count, per = (int64_t)G * stride;
+    // blocks past the list leave before the table load (uniform per block)
+    if ((int64_t)blockIdx.x * blockDim.x >= count * per) return;
+    load_tabs(tab);
     const int64_t ts = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (ts % stride) return;
-    const int64_t slot = ts / stride;
-    const bool first = (in_list == nullptr);
-    if (first ? slot >= n : slot >= (int64_t)*in_count) return;
+    const int64_t slot = ts / per;
+    if (slot >= count) return;   // whole groups leave together
+    const bool lead = G == 1 || threadIdx.x % G == 0;
     const int64_t i = first ? slot : (int64_t)in_list[slot];
-    const Tabs T = make_tabs(lds);
     const pnjl_mass_query a = qs[i];
     double* o = out + i * 6;
     const meson::KCoef k = kc ? load_kc(kc + i * 12)
-                              : meson::couplings(G, K, meson::G_from_A(a.A_u, a.m_u, Nc),
+                              : meson::couplings(Gc, K, meson::G_from_A(a.A_u, a.m_u, Nc),
                                                  meson::G_from_A(a.A_s, a.m_s, Nc));
-    double x[2], r[2], J[2][2], d[2], delta;
-    int it;
-    bool conv, stopped;
+    double x[2], r[2], J[2][2], d[2], p[2], xold[2], delta;
+    int it = 0;
+    bool conv = false, stopped = false, fresh = first;
     if (first) {
         if (a.meson < 0 || a.meson >= PNJL_MESON_ID_COUNT || a.max_iter < 0) {
-            for (int j = 0; j < 6; j++) o[j] = __builtin_nan("");
+            if (lead)
+                for (int j = 0; j < 6; j++) o[j] = __builtin_nan("");
             return;
         }
         x[0] = isnan(a.mass0) ? mass_guess(a) : a.mass0;
         x[1] = a.gamma0;
-        MassB0 B;
-        mass_b0(P, T, a, x[0], B);
-        mass_residual(P, a, k, B, x[0], x[1], r);
-        if (!isfinite(r[0]) || !isfinite(r[1])) {   // NLsolve's IsFiniteException at the start
-            o[0] = x[0], o[1] = x[1], o[2] = __builtin_nan(""), o[3] = 0.0, o[4] = 0.0, o[5] = 1.0;
-            return;
-        }
-        mass_jac(P, T, a, k, x, B, J);
-        it = 0;
-        conv = fmax(fabs(r[0]), fabs(r[1])) < a.ftol;
-        stopped = isnan(x[0]) || isnan(x[1]) || isnan(r[0]) || isnan(r[1]);
-        d[0] = d[1] = delta = 0.0;
-        if (!conv) {
-            for (int j = 0; j < 2; j++) {
-                d[j] = sqrt(J[0][j] * J[0][j] + J[1][j] * J[1][j]);
-                if (d[j] == 0.0) d[j] = 1.0;
-            }
-            delta = 1.0 * wnorm2(d, x);
-            if (delta == 0.0) delta = 1.0;
-        }
     } else {
         const MassState& S = states[i];
         x[0] = S.x[0], x[1] = S.x[1], r[0] = S.r[0], r[1] = S.r[1];
         J[0][0] = S.J[0][0], J[0][1] = S.J[0][1], J[1][0] = S.J[1][0], J[1][1] = S.J[1][1];
         d[0] = S.d[0], d[1] = S.d[1], delta = S.delta;
-        it = S.it, conv = S.conv != 0, stopped = S.stopped != 0;
+        it = S.it;
     }
-    int spent = 0;
-    while (!stopped && !conv && it < a.max_iter && (budget < 0 || spent < budget)) {
-        it++;
-        spent++;
-        double p[2], fn[2];
-        dogleg2(p, r, d, J, delta);
-        const double xold[2] = {x[0], x[1]};
-        x[0] += p[0], x[1] += p[1];
-        MassB0 Bn;
-        mass_b0(P, T, a, x[0], Bn);
-        mass_residual(P, a, k, Bn, x[0], x[1], fn);
+    // one trip: the step to the trial point (none on a fresh search), the
+    // residual and Jacobian there, and the trust region's decision
+    for (int spent = 0;; spent++) {
+        if (!fresh) {
+            if (stopped || conv || it >= a.max_iter || (budget >= 0 && spent >= budget)) break;
+            it++;
+            dogleg2(p, r, d, J, delta);
+            xold[0] = x[0], xold[1] = x[1];
+            x[0] += p[0], x[1] += p[1];
+        }
+        double fn[2], Jn[2][2];
+        mass_group<G>(P, a, k, x, fn, Jn);
+        if (fresh) {
+            fresh = false;
+            spent--;
+            r[0] = fn[0], r[1] = fn[1];
+            if (!isfinite(r[0]) || !isfinite(r[1])) {   // NLsolve's IsFiniteException at the start
+                if (lead) o[0] = x[0], o[1] = x[1], o[2] = __builtin_nan(""), o[3] = 0.0, o[4] = 0.0, o[5] = 1.0;
+                return;
+            }
+            for (int q = 0; q < 2; q++) J[q][0] = Jn[q][0], J[q][1] = Jn[q][1];
+            conv = fmax(fabs(r[0]), fabs(r[1])) < a.ftol;
+            stopped = isnan(x[0]) || isnan(x[1]) || isnan(r[0]) || isnan(r[1]);
+            d[0] = d[1] = delta = 0.0;
+            if (!conv) {
+                for (int j = 0; j < 2; j++) {
+                    d[j] = sqrt(J[0][j] * J[0][j] + J[1][j] * J[1][j]);
+                    if (d[j] == 0.0) d[j] = 1.0;
+                }
+                delta = 1.0 * wnorm2(d, x);
+                if (delta == 0.0) delta = 1.0;
+            }
+            continue;
+        }
         double rp[2];
         for (int q = 0; q < 2; q++) rp[q] = J[q][0] * p[0] + J[q][1] * p[1] + r[q];
         const double ssr = r[0] * r[0] + r[1] * r[1];
         const double rho = (ssr - (fn[0] * fn[0] + fn[1] * fn[1])) / (ssr - (rp[0] * rp[0] + rp[1] * rp[1]));
         if (rho > 1e-4) {
             r[0] = fn[0], r[1] = fn[1];
-            mass_jac(P, T, a, k, x, Bn, J);
+            for (int q = 0; q < 2; q++) J[q][0] = Jn[q][0], J[q][1] = Jn[q][1];
             for (int j = 0; j < 2; j++) d[j] = fmax(0.1 * d[j], sqrt(J[0][j] * J[0][j] + J[1][j] * J[1][j]));
             const bool xc = fmax(fabs(x[0] - xold[0]), fabs(x[1] - xold[1])) < a.xtol;
             conv = xc || fmax(fabs(r[0]), fabs(r[1])) < a.ftol;
@@ -1453,6 +1505,7 @@ __global__ void __launch_bounds__(256, 3) mass_kernel(Phys P, const double* tab,
             delta = fmax(delta, 2.0 * wnorm2(d, p));
         stopped = isnan(x[0]) || isnan(x[1]) || isnan(fn[0]) || isnan(fn[1]);
     }
+    if (!lead) return;
     if (!stopped && !conv && it < a.max_iter) {
         // budget spent: save the state for the next phase
         MassState& S = states[i];
@@ -1463,127 +1516,6 @@ __global__ void __launch_bounds__(256, 3) mass_kernel(Phys P, const double* tab,
         out_list[atomicAdd(out_count, 1u)] = (int32_t)i;
         return;
     }
-    o[0] = x[0], o[1] = x[1], o[2] = fmax(fabs(r[0]), fabs(r[1])), o[3] = conv ? 1.0 : 0.0, o[4] = (double)it;
-    o[5] = 0.0;
-}
-
-// The long tail of the pole searches (the phases after the first two: a few
-// percent of the queries, most of them running NLsolve's full 1000
-// iterations) with 16 lanes per query, four sub-groups of four: every
-// trust-region iteration needs B0 at the trial k0 and, when the step is
-// accepted, at k0 +- h for the Jacobian's k0 column; sub-groups 0, 1, 2
-// evaluate the three at once (sub-group 3 repeats sub-group 0), each with its
-// quadrature rules split over its four lanes and summed in the one-thread
-// order (ordered_sum), and the group exchanges them.  So an iteration costs a
-// quarter of one B0 evaluation of latency instead of three evaluations, the
-// phase runs 16x more lanes to hide it, and every lane runs the same control
-// logic on the same values, bit for bit, as the one-thread loop of
-// mass_kernel.  (Splitting a mixed meson's two quark pairs over sub-groups
-// as well was slower: the pairs' masses differ, so their quadrature branches
-// diverge within the wavefront.)  2 waves per SIMD: the 256 VGPRs spill less
-// than 168 at 3 waves, 8 % faster.
-constexpr int kMassLanes = 16;
-constexpr int kMassQLanes = 4;   // quadrature lanes per B0 evaluation
-
-__device__ __forceinline__ void shfl_b0(MassB0& dst, const MassB0& src, int lane)
-{
-    for (int j = 0; j < 2; j++) {
-        dst.r[j] = __shfl(src.r[j], lane, kMassLanes);
-        dst.i[j] = __shfl(src.i[j], lane, kMassLanes);
-    }
-}
-
-__global__ void __launch_bounds__(256, 2) mass_tail_kernel(Phys P, const double* tab, const pnjl_mass_query* qs,
-                                                        const double* kc, double G, double K, int Nc, double* out,
-                                                        MassState* states, const int32_t* in_list,
-                                                        const unsigned* in_count, int32_t* out_list,
-                                                        unsigned* out_count, int budget)
-{
-    // blocks past the list leave before the table load (uniform per block)
-    if ((int64_t)blockIdx.x * (blockDim.x / kMassLanes) >= (int64_t)*in_count) return;
-    double* const lds = mass_tab;
-    load_tabs(lds, tab);
-    const int64_t ts = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t slot = ts / kMassLanes;
-    const int gl = (int)(ts % kMassLanes);
-    const int sub = gl / kMassQLanes;
-    if (slot >= (int64_t)*in_count) return;   // whole groups leave together
-    const int64_t i = (int64_t)in_list[slot];
-    const Tabs T = make_tabs(lds);
-    const pnjl_mass_query a = qs[i];
-    const meson::KCoef k = kc ? load_kc(kc + i * 12)
-                              : meson::couplings(G, K, meson::G_from_A(a.A_u, a.m_u, Nc),
-                                                 meson::G_from_A(a.A_s, a.m_s, Nc));
-    const MassState& S = states[i];
-    double x[2] = {S.x[0], S.x[1]}, r[2] = {S.r[0], S.r[1]};
-    double J[2][2] = {{S.J[0][0], S.J[0][1]}, {S.J[1][0], S.J[1][1]}};
-    double d[2] = {S.d[0], S.d[1]}, delta = S.delta;
-    int it = S.it;
-    bool conv = S.conv != 0, stopped = S.stopped != 0;
-    int spent = 0;
-    while (!stopped && !conv && it < a.max_iter && (budget < 0 || spent < budget)) {
-        it++;
-        spent++;
-        double p[2], fn[2];
-        dogleg2(p, r, d, J, delta);
-        const double xold[2] = {x[0], x[1]};
-        x[0] += p[0], x[1] += p[1];
-        // B0 at the trial k0 (sub-groups 0, 3) and at k0 +- h (sub-groups 1, 2), h as mass_jac's k0 column
-        const double h = fmax(kFdStep * fabs(x[0]), kFdStep);
-        const double k0 = sub == 1 ? x[0] + h : (sub == 2 ? x[0] - h : x[0]);
-        MassB0 Bl, Bn, Bp, Bm;
-        mass_b0<kMassQLanes>(P, T, a, k0, Bl);
-        shfl_b0(Bn, Bl, 0);   // lanes of the query's group (__shfl's lane is relative to its width)
-        shfl_b0(Bp, Bl, kMassQLanes);
-        shfl_b0(Bm, Bl, 2 * kMassQLanes);
-        mass_residual(P, a, k, Bn, x[0], x[1], fn);
-        double rp[2];
-        for (int q = 0; q < 2; q++) rp[q] = J[q][0] * p[0] + J[q][1] * p[1] + r[q];
-        const double ssr = r[0] * r[0] + r[1] * r[1];
-        const double rho = (ssr - (fn[0] * fn[0] + fn[1] * fn[1])) / (ssr - (rp[0] * rp[0] + rp[1] * rp[1]));
-        if (rho > 1e-4) {
-            r[0] = fn[0], r[1] = fn[1];
-            // mass_jac with its three B0 sets already at hand
-            for (int j = 0; j < 2; j++) {
-                const double hj = fmax(kFdStep * fabs(x[j]), kFdStep);
-                double xp[2] = {x[0], x[1]}, xm[2] = {x[0], x[1]}, fp[2], fm[2];
-                xp[j] = x[j] + hj;
-                xm[j] = x[j] - hj;
-                if (j == 0) {
-                    mass_residual(P, a, k, Bp, xp[0], xp[1], fp);
-                    mass_residual(P, a, k, Bm, xm[0], xm[1], fm);
-                } else {
-                    mass_residual(P, a, k, Bn, xp[0], xp[1], fp);
-                    mass_residual(P, a, k, Bn, xm[0], xm[1], fm);
-                }
-                for (int q = 0; q < 2; q++) J[q][j] = (fp[q] - fm[q]) / (2.0 * hj);
-            }
-            for (int j = 0; j < 2; j++) d[j] = fmax(0.1 * d[j], sqrt(J[0][j] * J[0][j] + J[1][j] * J[1][j]));
-            const bool xc = fmax(fabs(x[0] - xold[0]), fabs(x[1] - xold[1])) < a.xtol;
-            conv = xc || fmax(fabs(r[0]), fabs(r[1])) < a.ftol;
-        } else {
-            x[0] -= p[0], x[1] -= p[1];
-            conv = false;
-        }
-        if (rho < 0.1)
-            delta = delta / 2.0;
-        else if (rho >= 0.9)
-            delta = 2.0 * wnorm2(d, p);
-        else if (rho >= 0.5)
-            delta = fmax(delta, 2.0 * wnorm2(d, p));
-        stopped = isnan(x[0]) || isnan(x[1]) || isnan(fn[0]) || isnan(fn[1]);
-    }
-    if (gl != 0) return;
-    if (!stopped && !conv && it < a.max_iter) {
-        MassState& W = states[i];
-        W.x[0] = x[0], W.x[1] = x[1], W.r[0] = r[0], W.r[1] = r[1];
-        W.J[0][0] = J[0][0], W.J[0][1] = J[0][1], W.J[1][0] = J[1][0], W.J[1][1] = J[1][1];
-        W.d[0] = d[0], W.d[1] = d[1], W.delta = delta;
-        W.it = it, W.conv = 0, W.stopped = 0;
-        out_list[atomicAdd(out_count, 1u)] = (int32_t)i;
-        return;
-    }
-    double* o = out + i * 6;
     o[0] = x[0], o[1] = x[1], o[2] = fmax(fabs(r[0]), fabs(r[1])), o[3] = conv ? 1.0 : 0.0, o[4] = (double)it;
     o[5] = 0.0;
 }
@@ -1627,57 +1559,74 @@ namespace {
 
 polar::Phys phys(const pnjl_ctx* c) { return polar::Phys{c->params.Lambda, (double)c->params.N_color}; }
 
-// x16 w16 x32 w32 | power-left 16/32 (t, t') | power-right 16/32 | DE 33 (phi, phi')
-//   IntervalQuadratureStrategies.jl:56-85
+// the quadrature kernels' tables (layout: polar::ptab)
+//   rules: IntervalQuadratureStrategies.jl:56-85
 int polar_tab(pnjl_ctx* ctx, double** out)
 {
     if (!ctx->polar_tab) {
-        std::vector<double> t(polar::kTabLen), x, w;
-        double* o = t.data();
-        std::vector<double> x16, w16, x32, w32;
+        std::vector<double> t(polar::kTabLen), x16, w16, x32, w32;
+        for (int j = 0; j < 64; j++) t[pnjl::kExpTab + j] = (double)exp2l((long double)j / 64.0L);
+        for (int j = 0; j < 128; j++) {
+            // the first and last intervals take c = 1 and c = 2: log(1) = 0 there
+            const long double c = j == 0 ? 1.0L : (j == 127 ? 2.0L : 1.0L + ((long double)j + 0.5L) / 128.0L);
+            const double inv = (double)(1.0L / c);
+            t[polar::kPLog + 2 * j] = inv;
+            t[polar::kPLog + 2 * j + 1] = (double)(-logl((j >= 64 ? 2.0L : 1.0L) * (long double)inv));
+        }
         gl_rule(16, x16, w16);
         gl_rule(32, x32, w32);
-        auto put = [&](const std::vector<double>& v) {
-            memcpy(o, v.data(), v.size() * sizeof(double));
-            o += v.size();
-        };
-        put(x16);
-        put(w16);
-        put(x32);
-        put(w32);
         const double ia = 1.0 / polar::kAlpha;
-        for (int side = 0; side < 2; side++)
-            for (const std::vector<double>* xs : {&x16, &x32}) {
-                const size_t n = xs->size();
-                std::vector<double> tt(n), tp(n);
-                for (size_t i = 0; i < n; i++) {
-                    double u = ((*xs)[i] + 1) / 2;
-                    if (side == 0) {
-                        tt[i] = pow(u, ia);
-                        tp[i] = ia * pow(u, ia - 1) / 2;
-                    } else {
-                        tt[i] = 1 - pow(1 - u, ia);
-                        tp[i] = ia * pow(1 - u, ia - 1) / 2;
-                    }
-                }
-                put(tt);
-                put(tp);
-            }
-        std::vector<double> phi(33), phip(33);
+        auto put = [&](int off, int i, int n, double node, double weight) {
+            t[off + i] = node;
+            t[off + n + i] = weight;
+        };
+        for (int i = 0; i < 16; i++) {
+            const double u = (x16[i] + 1) / 2;
+            put(polar::R_L16, i, 16, pow(u, ia), w16[i] * (ia * pow(u, ia - 1) / 2));
+            put(polar::R_G16, i, 16, x16[i], w16[i]);
+        }
+        for (int i = 0; i < 32; i++) {
+            const double u = (x32[i] + 1) / 2;
+            put(polar::R_L32, i, 32, pow(u, ia), w32[i] * (ia * pow(u, ia - 1) / 2));
+            put(polar::R_R32, i, 32, 1 - pow(1 - u, ia), w32[i] * (ia * pow(1 - u, ia - 1) / 2));
+            put(polar::R_G32, i, 32, x32[i], w32[i]);
+        }
         for (int k = -16; k <= 16; k++) {
             double tk = k * polar::kDeH;
             double s = polar::kPi / 2 * sinh(tk);
             double sech = 1.0 / cosh(s);
-            phi[k + 16] = tanh(s);
-            phip[k + 16] = polar::kDeH * (polar::kPi / 2) * cosh(tk) * (sech * sech);
+            put(polar::R_DE, k + 16, 33, tanh(s), polar::kDeH * (polar::kPi / 2) * cosh(tk) * (sech * sech));
         }
-        put(phi);
-        put(phip);
         HIPCHK(ctx, hipMalloc(&ctx->polar_tab, t.size() * sizeof(double)));
         HIPCHK(ctx, hipMemcpy(ctx->polar_tab, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
     }
     *out = ctx->polar_tab;
     return PNJL_OK;
+}
+
+// Lanes per item of the quadrature kernels (an item is a Pi query, a grid cell
+// or a propagator query's quark pair, about two per query): one lane walks
+// the ~60 to 320 nodes of an item alone, which is the cheapest use of the
+// chip but leaves it idle below its ~2 x 10^5 resident lanes, so smaller calls
+// split each item over more lanes.  Measured, ms at 1 / 4 / 16 / 64 lanes: Pi
+// queries 1000: 0.62 / 0.36 / 0.19 / 0.16, 10 000: 0.74 / 0.35 / 0.26 / 0.32,
+// 60 000: 0.98 / 0.93 / 0.93, 200 000: 2.90 / 2.90 / 3.07; grid cells 81 000:
+// 0.72 / 0.56 / 0.63 / 1.20, 307 200: 1.17 / 1.25 / 1.70; propagator queries
+// 1000: 0.48 / 0.22 / 0.11 / 0.09, 5000: 0.48 / 0.22 / 0.13 / 0.18, 65 536:
+// 0.55 / 0.43 / 0.70, 131 072: 0.71 / 0.71 / 1.30.
+int item_lanes(int64_t items) { return items <= 4096 ? 64 : (items <= 32768 ? 16 : (items <= 196608 ? 4 : 1)); }
+
+// f(L, S) with the kernels' compile-time split of `lanes`: L lanes per evaluation, S evaluations at once
+template <class F>
+void launch_lanes(int lanes, const F& f)
+{
+    using std::integral_constant;
+    switch (lanes) {
+    case 64: f(integral_constant<int, 16>(), integral_constant<int, 4>()); break;
+    case 16: f(integral_constant<int, 4>(), integral_constant<int, 4>()); break;
+    case 4: f(integral_constant<int, 4>(), integral_constant<int, 1>()); break;
+    default: f(integral_constant<int, 1>(), integral_constant<int, 1>()); break;
+    }
 }
 
 int blocks_for(int64_t n) { return (int)((n + 255) / 256); }
@@ -1716,8 +1665,11 @@ int pnjl_polarization_batch(pnjl_ctx* ctx, int64_t n, const pnjl_pol_query* q, d
     }
     HIPCHK(ctx, hipEventRecord(ctx->ev0, st));
     const int stride = (flags & PNJL_FLAG_ONE_PER_WAVE) ? 64 : 1;
-    hipLaunchKernelGGL(polar::query_kernel, dim3(blocks_for(n * stride)), dim3(256), 0, st, phys(ctx), tab, n, dq, dre,
-                       dim, stride);
+    const int lanes = stride > 1 ? 1 : item_lanes(n);
+    launch_lanes(lanes, [&](auto L, auto S) {
+        hipLaunchKernelGGL((polar::query_kernel<L(), S()>), dim3(blocks_for(n * stride * lanes)), dim3(256), 0, st,
+                           phys(ctx), tab, n, dq, dre, dim, stride);
+    });
     HIPCHK(ctx, hipGetLastError());
     HIPCHK(ctx, hipEventRecord(ctx->ev1, st));
     if (!dev) {
@@ -1846,9 +1798,12 @@ int pnjl_polarization_grid(pnjl_ctx* ctx, int npts, const pnjl_pol_point* pts, i
         hipLaunchKernelGGL(polar::grid_a_kernel, dim3(blocks_for(2 * (int64_t)npts)), dim3(256), 0, g->cap,
                            phys(ctx), npts, (const pnjl_pol_point*)g->pts, np, g->nodes, g->nodes + np, nc,
                            g->nodes + 2 * np, g->nodes + 2 * np + nc, g->A);
-        hipLaunchKernelGGL(polar::grid_pi_kernel, dim3(blocks_for(nout / 2)), dim3(256), 0, g->cap, phys(ctx), tab,
-                           npts, (const pnjl_pol_point*)g->pts, (const double*)g->A, nk0, (const double*)g->k0, nk,
-                           (const double*)g->k, g->re, g->im);
+        const int lanes = item_lanes(nout / 2);
+        launch_lanes(lanes, [&](auto L, auto S) {
+            hipLaunchKernelGGL((polar::grid_pi_kernel<L(), S()>), dim3(blocks_for(nout / 2 * lanes)), dim3(256), 0,
+                               g->cap, phys(ctx), tab, npts, (const pnjl_pol_point*)g->pts, (const double*)g->A, nk0,
+                               (const double*)g->k0, nk, (const double*)g->k, g->re, g->im);
+        });
         HIPCHK(ctx, hipStreamEndCapture(g->cap, &g->graph));
         HIPCHK(ctx, hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0));
     }
@@ -1966,8 +1921,12 @@ int pnjl_propagator_by_channel_batch(pnjl_ctx* ctx, int64_t n, const pnjl_prop_q
     hipLaunchKernelGGL(polar::prop_scan_kernel, dim3(1), dim3(256), 0, st, (const unsigned*)counts, offs);
     hipLaunchKernelGGL(polar::prop_scatter_kernel, dim3(blocks_for(3 * n)), dim3(256), 0, st, n, dq,
                        (const unsigned*)offs, cursor, (unsigned*)items);
-    hipLaunchKernelGGL(polar::prop_pi_kernel, dim3(blocks_for(3 * n * stride)), dim3(256), 0, st, phys(ctx), tab, dq,
-                       (const unsigned*)items, (const unsigned*)offs, (double*)pib, stride);
+    const int lanes = stride > 1 ? 1 : item_lanes(2 * n);
+    launch_lanes(lanes, [&](auto L, auto S) {
+        hipLaunchKernelGGL((polar::prop_pi_kernel<L(), S()>), dim3(blocks_for(3 * n * stride * lanes)), dim3(256), 0,
+                           st, phys(ctx), tab, dq, (const unsigned*)items, (const unsigned*)offs, (double*)pib,
+                           stride);
+    });
     HIPCHK(ctx, hipGetLastError());
     hipLaunchKernelGGL(polar::prop_compose_kernel, dim3(blocks_for(n)), dim3(256), 0, st, n, dq, dkc, ctx->params.G,
                        ctx->params.K, ctx->params.N_color, (const double*)pib, dout);
@@ -2030,21 +1989,25 @@ int pnjl_meson_mass_batch(pnjl_ctx* ctx, int64_t n, const pnjl_mass_query* q, co
     HIPCHK(ctx, hipEventRecord(ctx->ev0, st));
     hipLaunchKernelGGL(polar::zero_u32, dim3(1), dim3(64), 0, st, cnt, kPhases);
     const int stride = (flags & PNJL_FLAG_ONE_PER_WAVE) ? 64 : 1;
-    // the tail phases (from kTailPhase on: few queries, hundreds of
-    // iterations each) run kMassLanes lanes per query; the
-    // one-query-per-wavefront FLOP count keeps one thread per query throughout
+    // from kTailPhase on: few queries, hundreds of iterations each.  16 lanes
+    // for every other phase (524 288 queries: 111 ms, with one lane in the
+    // first two phases 153), 64 in the tail while the longest searches set the
+    // time (tail at 16 / 64 lanes: 18 432 queries 21.7 / 13.0 ms, 131 072
+    // queries 50 / 43); one lane past the launch limit of 2^32 threads.
     constexpr int kTailPhase = 2;
+    const int head = stride > 1 || n > ((int64_t)1 << 27) ? 1 : 16, tail = (head > 1 && n <= 131072) ? 64 : head;
     for (int ph = 0; ph < kPhases; ph++) {
         const int32_t* in_list = ph == 0 ? nullptr : lists[(ph - 1) & 1];
         const unsigned* in_count = ph == 0 ? nullptr : cnt + ph - 1;
-        if (ph >= kTailPhase && stride == 1)
-            hipLaunchKernelGGL(polar::mass_tail_kernel, dim3(blocks_for(n * polar::kMassLanes)), dim3(256), 0, st,
-                               phys(ctx), tab, dq, dkc, ctx->params.G, ctx->params.K, ctx->params.N_color, dout,
+        const int lanes = ph >= kTailPhase ? tail : head;
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(blocks_for(n * stride * lanes)), dim3(256), 0, st, phys(ctx), tab, n, dq,
+                               dkc, ctx->params.G, ctx->params.K, ctx->params.N_color, dout, stride,
                                (polar::MassState*)vs, in_list, in_count, lists[ph & 1], cnt + ph, budgets[ph]);
-        else
-            hipLaunchKernelGGL(polar::mass_kernel, dim3(blocks_for(n * stride)), dim3(256), 0, st, phys(ctx), tab, n,
-                               dq, dkc, ctx->params.G, ctx->params.K, ctx->params.N_color, dout, stride,
-                               (polar::MassState*)vs, in_list, in_count, lists[ph & 1], cnt + ph, budgets[ph]);
+        };
+        if (lanes == 64) launch(polar::mass_kernel<64>);
+        else if (lanes == 16) launch(polar::mass_kernel<16>);
+        else launch(polar::mass_kernel<1>);
         HIPCHK(ctx, hipGetLastError());
     }
     HIPCHK(ctx, hipEventRecord(ctx->ev1, st));

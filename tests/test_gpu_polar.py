@@ -54,6 +54,28 @@ def test_polarization_batch_matches_oracle(gpu_ctx, oracle):
     assert np.isfinite(ore).mean() > 0.99
 
 
+@pytest.mark.parametrize("n", [1, 2, 4096, 4097, 32769, 196609])
+def test_lane_split_does_not_change_results(gpu_ctx, n):
+    """A value does not depend on how many lanes its batch gives it: the lanes
+    of a group add their terms in the one-lane order, bit for bit (sizes on
+    both sides of each change of the split; 196 609 queries run on one lane
+    each).  Queries of all forms, k = 0 and k > 0, equal and unequal masses and
+    chemical potentials, and one with NaN and one with infinite inputs."""
+    from julia_relaxtime_amd import polarization as P
+    cols = _queries(512, 3)
+    q = np.zeros(512, dtype=P.QUERY_DTYPE)
+    for f, v in cols.items():
+        q[f] = v
+    q["mu1"][7] = np.nan
+    q["k0"][9] = np.inf
+    q["T"][11] = 1e-3
+    ref = P.polarization_batch(np.resize(q, 200000))
+    re, im = P.polarization_batch(np.resize(q, n))
+    for g, r in ((re, ref[0]), (im, ref[1])):
+        assert np.array_equal(g.view(np.int64), np.resize(r[:512], n).view(np.int64)) or \
+            np.array_equal(g, np.resize(r[:512], n), equal_nan=True)
+
+
 def test_B0_and_correction_batches_match_oracle(gpu_ctx, oracle):
     from julia_relaxtime_amd import polarization as P
     rng = np.random.default_rng(4)
