@@ -9,10 +9,15 @@
 // of the node terms ln F(a), ln F(b), a = (mu - E)/T, b = -(E + mu)/T: the
 // Hessian of the gap solve extended by the rows and columns of T and mu.
 //
-// One thread per root: this pass runs once per point after the solve, so it
-// keeps the node loop simple -- every node and sign through the shifted
-// per-sign evaluation of the 1e-16 floor (lnF_slow), table-driven exp/log.
+// NL lanes per root (by the number of roots): the lanes split the nodes, and
+// each adds some of the sums over all of them in node order (NodeSums), so the
+// results are those of one lane, bit for bit; the rest runs on every lane
+// alike.  The pass runs once per point after the solve, so it keeps the node
+// loop simple -- every node and sign through the shifted per-sign evaluation
+// of the 1e-16 floor (lnF_slow), table-driven exp/log.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "pnjl_ctx.h"
 
@@ -34,94 +39,200 @@ struct FlavD {
     double Smu, ST, Smumu, SmuT, STT, SMmu, SMT, SPmu, SPbmu, SPT, SPbT;
 };
 
-__device__ void flavour_d(const double* tab, int pn, int tn, double M, double mu, double T, double xi, double Phi,
+// The sums over the p x t mesh of NC terms per node, each a number of NP parts
+// (term c, part p at t[c NP + p]).  One lane adds its terms as they come.  The
+// lanes of a group (within one wavefront) take the nodes l pn + j = gl, gl +
+// NL, ... in rounds of NL, leave their terms in the group's LDS rows one part
+// at a time, and lane k adds the terms k, k + NL, ... of the round's nodes in
+// order: a term's sum is the one-lane sum.  (At low T derivatives are small
+// differences of such sums, and another order moves them by 1e-9.)
+template <int NL, int NC, int NP>
+struct NodeSums {
+    static constexpr int kOwn = (NC + NL - 1) / NL;
+    double own[NP][kOwn] = {};
+    double* rows;
+
+    __device__ __forceinline__ explicit NodeSums(double* lds_rows) : rows(lds_rows + threadIdx.x / NL * (NL * NC)) {}
+
+    __device__ __forceinline__ static void fence()
+    {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    // t: this lane's terms; m: nodes of the round
+    __device__ __forceinline__ void add(const double* t, int m)
+    {
+        const int gl = (int)(threadIdx.x % NL);
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            if (gl < m)
+#pragma unroll
+                for (int c = 0; c < NC; c++) rows[gl * NC + c] = t[c * NP + p];
+            fence();
+#pragma unroll
+            for (int i = 0; i < kOwn; i++) {
+                const int c = gl + i * NL;
+                if (c < NC) {
+                    double a = own[p][i];
+                    if (m == NL) {
+#pragma unroll 8
+                        for (int n = 0; n < NL; n++) a += rows[n * NC + c];
+                    } else {
+                        for (int n = 0; n < m; n++) a += rows[n * NC + c];
+                    }
+                    own[p][i] = a;
+                }
+            }
+            fence();
+        }
+    }
+    // every lane gets all sums
+    __device__ __forceinline__ void take(double* o)
+    {
+        const int gl = (int)(threadIdx.x % NL);
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+#pragma unroll
+            for (int i = 0; i < kOwn; i++)
+                if (gl + i * NL < NC) rows[gl + i * NL] = own[p][i];
+            fence();
+#pragma unroll
+            for (int c = 0; c < NC; c++) o[c * NP + p] = rows[c];
+            fence();
+        }
+    }
+};
+
+// f(l, j, t) leaves the terms of node (l, j) in t; o gets their sums over the mesh
+template <int NL, int NC, int NP, class F>
+__device__ __forceinline__ void node_sums(double* lds_rows, int pn, int tn, double* o, const F& f)
+{
+    double t[NC * NP];
+    if constexpr (NL == 1) {
+#pragma unroll
+        for (int i = 0; i < NC * NP; i++) o[i] = 0.0;
+#pragma unroll 1
+        for (int l = 0; l < tn; l++)
+#pragma unroll 1
+            for (int j = 0; j < pn; j++) {
+                f(l, j, t);
+#pragma unroll
+                for (int i = 0; i < NC * NP; i++) o[i] += t[i];
+            }
+    } else {
+        NodeSums<NL, NC, NP> sums(lds_rows);
+        const int total = pn * tn;
+        int l = 0, j = (int)(threadIdx.x % NL);
+#pragma unroll 1
+        for (int e = 0; e < total; e += NL, j += NL) {
+            while (j >= pn) {
+                j -= pn;
+                l++;
+            }
+            if (l < tn) f(l, j, t);
+            sums.add(t, total - e < NL ? total - e : NL);
+        }
+        sums.take(o);
+    }
+}
+
+template <int NL>
+__device__ void flavour_d(const double* tab, double* rows, int pn, int tn, double M, double mu, double T, double xi, double Phi,
                           double Phib, FlavD& o)
 {
-    o = FlavD{};
     const double* pp = tab + pnjl::kMathTab;
     const double* cc = pp + pn;
     const double* Cm = pp + pn + tn;
     const double invT = 1.0 / T, invT2 = invT * invT, M2 = M * M;
-    for (int l = 0; l < tn; l++) {
+    node_sums<NL, sizeof(FlavD) / sizeof(double), 1>(rows, pn, tn, &o.S, [&](int l, int j, double* t) {
+        FlavD& n = *reinterpret_cast<FlavD*>(t);
         const double xc = xi * cc[l];
-        for (int j = 0; j < pn; j++) {
-            const double C = Cm[l * pn + j];
-            double E, invE;
-            pnjl::rsqrt_sqrt(fma(xc, pp[j], pp[j]) + M2, invE, E);
-            const double a = (mu - E) * invT, b = -(E + mu) * invT;
-            pnjl::Sign1 sp, sm;
-            pnjl::lnF_slow(tab, a, Phi, Phib, sp);
-            pnjl::lnF_slow(tab, b, Phib, Phi, sm);
-            // derivatives of ln F in its own argument and loop parameters
-            const double gp = 3.0 * sp.gq, gm = 3.0 * sm.gq;
-            const double hp = 3.0 * sp.h, hm = 3.0 * sm.h;
-            const double ac1p = 3.0 * sp.k1, ac2p = 3.0 * sp.k2, ac1m = 3.0 * sm.k1, ac2m = 3.0 * sm.k2;
-            const double Q = sp.v + sm.v;
-            const double QE = -(gp + gm) * invT, QEE = (hp + hm) * invT2;
-            const double QP = 3.0 * (sp.r1 + sm.r2), QPb = 3.0 * (sp.r2 + sm.r1);
-            const double QEP = -(ac1p + ac2m) * invT, QEPb = -(ac2p + ac1m) * invT;
-            const double EM = M * invE, EMM = (1.0 - EM * EM) * invE;
-            o.S += C * Q;
-            o.SM += C * (QE * EM);
-            o.SP += C * QP;
-            o.SPb += C * QPb;
-            o.SMM += C * (QEE * EM * EM + QE * EMM);
-            o.SMP += C * (QEP * EM);
-            o.SMPb += C * (QEPb * EM);
-            o.SPP += C * (-9.0 * (sp.r1 * sp.r1 + sm.r2 * sm.r2));
-            o.SPPb += C * (-9.0 * (sp.r1 * sp.r2 + sm.r1 * sm.r2));
-            o.SPbPb += C * (-9.0 * (sp.r2 * sp.r2 + sm.r1 * sm.r1));
-            // da/dmu = 1/T, db/dmu = -1/T, da/dT = -a/T, db/dT = -b/T, da/dE = db/dE = -1/T
-            o.Smu += C * (gp - gm) * invT;
-            o.ST += C * (-(gp * a + gm * b) * invT);
-            o.Smumu += C * (hp + hm) * invT2;
-            o.SmuT += C * (-(gp - gm) - (hp * a - hm * b)) * invT2;
-            o.STT += C * (2.0 * (gp * a + gm * b) + hp * a * a + hm * b * b) * invT2;
-            o.SMmu += C * (-(hp - hm) * invT2) * EM;
-            o.SMT += C * ((gp + gm + hp * a + hm * b) * invT2) * EM;
-            o.SPmu += C * (ac1p - ac2m) * invT;
-            o.SPbmu += C * (ac2p - ac1m) * invT;
-            o.SPT += C * (-(ac1p * a + ac2m * b) * invT);
-            o.SPbT += C * (-(ac2p * a + ac1m * b) * invT);
-        }
-    }
+        const double C = Cm[l * pn + j];
+        double E, invE;
+        pnjl::rsqrt_sqrt(fma(xc, pp[j], pp[j]) + M2, invE, E);
+        const double a = (mu - E) * invT, b = -(E + mu) * invT;
+        pnjl::Sign1 sp, sm;
+        pnjl::lnF_slow(tab, a, Phi, Phib, sp);
+        pnjl::lnF_slow(tab, b, Phib, Phi, sm);
+        // derivatives of ln F in its own argument and loop parameters
+        const double gp = 3.0 * sp.gq, gm = 3.0 * sm.gq;
+        const double hp = 3.0 * sp.h, hm = 3.0 * sm.h;
+        const double ac1p = 3.0 * sp.k1, ac2p = 3.0 * sp.k2, ac1m = 3.0 * sm.k1, ac2m = 3.0 * sm.k2;
+        const double Q = sp.v + sm.v;
+        const double QE = -(gp + gm) * invT, QEE = (hp + hm) * invT2;
+        const double QP = 3.0 * (sp.r1 + sm.r2), QPb = 3.0 * (sp.r2 + sm.r1);
+        const double QEP = -(ac1p + ac2m) * invT, QEPb = -(ac2p + ac1m) * invT;
+        const double EM = M * invE, EMM = (1.0 - EM * EM) * invE;
+        n.S = C * Q;
+        n.SM = C * (QE * EM);
+        n.SP = C * QP;
+        n.SPb = C * QPb;
+        n.SMM = C * (QEE * EM * EM + QE * EMM);
+        n.SMP = C * (QEP * EM);
+        n.SMPb = C * (QEPb * EM);
+        n.SPP = C * (-9.0 * (sp.r1 * sp.r1 + sm.r2 * sm.r2));
+        n.SPPb = C * (-9.0 * (sp.r1 * sp.r2 + sm.r1 * sm.r2));
+        n.SPbPb = C * (-9.0 * (sp.r2 * sp.r2 + sm.r1 * sm.r1));
+        // da/dmu = 1/T, db/dmu = -1/T, da/dT = -a/T, db/dT = -b/T, da/dE = db/dE = -1/T
+        n.Smu = C * (gp - gm) * invT;
+        n.ST = C * (-(gp * a + gm * b) * invT);
+        n.Smumu = C * (hp + hm) * invT2;
+        n.SmuT = C * (-(gp - gm) - (hp * a - hm * b)) * invT2;
+        n.STT = C * (2.0 * (gp * a + gm * b) + hp * a * a + hm * b * b) * invT2;
+        n.SMmu = C * (-(hp - hm) * invT2) * EM;
+        n.SMT = C * ((gp + gm + hp * a + hm * b) * invT2) * EM;
+        n.SPmu = C * (ac1p - ac2m) * invT;
+        n.SPbmu = C * (ac2p - ac1m) * invT;
+        n.SPT = C * (-(ac1p * a + ac2m * b) * invT);
+        n.SPbT = C * (-(ac2p * a + ac1m * b) * invT);
+    });
 }
 
-// LU with partial pivoting of a 5x5 system with two right-hand sides;
-// returns false on an exactly zero pivot
-__device__ bool lu5_solve2(double A[5][5], double b1[5], double b2[5])
+// LU with partial pivoting (largest |pivot|, first on ties) of a 5x5 system
+// with two right-hand sides, fully unrolled with row exchanges by selects, so
+// the matrix stays in registers; returns false on an exactly zero pivot
+__device__ __forceinline__ bool lu5_solve2(double A[5][5], double b1[5], double b2[5])
 {
+    bool sing = false;
+#pragma unroll
     for (int k = 0; k < 5; k++) {
         int p = k;
         double best = fabs(A[k][k]);
-        for (int i = k + 1; i < 5; i++)
-            if (fabs(A[i][k]) > best) {
-                best = fabs(A[i][k]);
-                p = i;
-            }
-        if (A[p][k] == 0.0) return false;
-        if (p != k) {
-            for (int j = 0; j < 5; j++) {
-                double t = A[k][j];
-                A[k][j] = A[p][j];
-                A[p][j] = t;
-            }
-            double t = b1[k];
-            b1[k] = b1[p];
-            b1[p] = t;
-            t = b2[k];
-            b2[k] = b2[p];
-            b2[p] = t;
+#pragma unroll
+        for (int i = k + 1; i < 5; i++) {
+            const bool gt = fabs(A[i][k]) > best;
+            best = gt ? fabs(A[i][k]) : best;
+            p = gt ? i : p;
         }
+#pragma unroll
+        for (int i = k + 1; i < 5; i++) {
+            const bool sw = p == i;
+            auto swap = [&](double& u, double& v) {
+                const double t = u;
+                u = sw ? v : t;
+                v = sw ? t : v;
+            };
+#pragma unroll
+            for (int j = 0; j < 5; j++)
+                if (j >= k) swap(A[k][j], A[i][j]);
+            swap(b1[k], b1[i]);
+            swap(b2[k], b2[i]);
+        }
+        sing = sing || A[k][k] == 0.0;
+#pragma unroll
         for (int i = k + 1; i < 5; i++) {
             const double l = A[i][k] / A[k][k];
+#pragma unroll
             for (int j = k + 1; j < 5; j++) A[i][j] -= l * A[k][j];
             b1[i] -= l * b1[k];
             b2[i] -= l * b2[k];
         }
     }
+#pragma unroll
     for (int i = 4; i >= 0; i--) {
         double s1 = b1[i], s2 = b2[i];
+#pragma unroll
         for (int j = i + 1; j < 5; j++) {
             s1 -= A[i][j] * b1[j];
             s2 -= A[i][j] * b2[j];
@@ -129,7 +240,7 @@ __device__ bool lu5_solve2(double A[5][5], double b1[5], double b2[5])
         b1[i] = s1 / A[i][i];
         b2[i] = s2 / A[i][i];
     }
-    return true;
+    return !sing;
 }
 
 struct DerivArgs {
@@ -141,13 +252,14 @@ struct DerivArgs {
     double* out;   // n * PNJL_THERMO_DERIV_FIELDS
 };
 
+template <int NL>
 __global__ void __launch_bounds__(256) deriv_kernel(DerivArgs A)
 {
     extern __shared__ double lds[];
     const int tab_len = pnjl::kMathTab + A.pn + A.tn + A.pn * A.tn + A.pn;
     for (int i = threadIdx.x; i < tab_len; i += blockDim.x) lds[i] = A.tab[i];
     __syncthreads();
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t g = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / NL;
     if (g >= A.n) return;
     const DevParams& P = A.P;
     const double T = A.T[g], mu = A.mu[g], xi = A.xi[g];
@@ -170,10 +282,10 @@ __global__ void __launch_bounds__(256) deriv_kernel(DerivArgs A)
     };
     // node sums: u, s, and d unless phi_d == phi_u
     FlavD f[3];
-    flavour_d(lds, A.pn, A.tn, M[0], mu, T, xi, Phi, Phib, f[0]);
-    flavour_d(lds, A.pn, A.tn, M[2], mu, T, xi, Phi, Phib, f[2]);
+    flavour_d<NL>(lds, lds + tab_len, A.pn, A.tn, M[0], mu, T, xi, Phi, Phib, f[0]);
+    flavour_d<NL>(lds, lds + tab_len, A.pn, A.tn, M[2], mu, T, xi, Phi, Phib, f[2]);
     if (pd == pu) f[1] = f[0];
-    else flavour_d(lds, A.pn, A.tn, M[1], mu, T, xi, Phi, Phib, f[1]);
+    else flavour_d<NL>(lds, lds + tab_len, A.pn, A.tn, M[1], mu, T, xi, Phi, Phib, f[1]);
 
     // chiral term, vacuum term, Polyakov potential (Thermodynamics.jl:112-160)
     const double chi = 2.0 * G * (pu * pu + pd * pd + ps * ps) - 4.0 * K * pu * pd * ps;
@@ -274,6 +386,7 @@ __global__ void __launch_bounds__(256) deriv_kernel(DerivArgs A)
         dxdT[a] = -Om_xT[a];
         dxdmu[a] = -Om_xmu[a];
     }
+    if (NL > 1 && threadIdx.x % NL) return;
     if (!lu5_solve2(H, dxdT, dxdmu)) {
         for (int k = 0; k < PNJL_THERMO_DERIV_FIELDS; k++) out[k] = __builtin_nan("");
         return;
@@ -373,6 +486,8 @@ __device__ inline double val(double x) { return x; }
 __device__ inline double val(const D2& x) { return x.v; }
 __device__ inline bool same(double a, double b) { return a == b; }
 __device__ inline bool same(const D2& a, const D2& b) { return a.v == b.v && a.t == b.t && a.m == b.m; }
+__device__ inline double choose(bool c, double a, double b) { return c ? a : b; }
+__device__ inline D2 choose(bool c, D2 a, D2 b) { return D2{c ? a.v : b.v, c ? a.t : b.t, c ? a.m : b.m}; }
 template <class R> __device__ inline R cst(double c);
 template <> __device__ inline double cst<double>(double c) { return c; }
 template <> __device__ inline D2 cst<D2>(double c) { return D2{c, 0.0, 0.0}; }
@@ -441,48 +556,47 @@ struct FlavR {
     R SM, SP, SPb, SMM, SMP, SMPb, SPP, SPPb, SPbPb, SMmu, SMT, SPmu, SPbmu, SPT, SPbT;
 };
 
-template <class R>
-__device__ void flavour_r(const double* tab, int pn, int tn, R M, R mu, R T, double xi, R Phi, R Phib, FlavR<R>& o)
+template <int NL, class R>
+__device__ void flavour_r(const double* tab, double* rows, int pn, int tn, R M, R mu, R T, double xi, R Phi, R Phib, FlavR<R>& o)
 {
-    const R z = cst<R>(0.0);
-    o = FlavR<R>{z, z, z, z, z, z, z, z, z, z, z, z, z, z, z};
     const double* pp = tab + pnjl::kMathTab;
     const double* cc = pp + pn;
     const double* Cm = pp + pn + tn;
     const R invT = 1.0 / T, invT2 = invT * invT, M2 = M * M;
-    for (int l = 0; l < tn; l++) {
+    constexpr int kParts = sizeof(R) / sizeof(double);
+    node_sums<NL, sizeof(FlavR<R>) / sizeof(R), kParts>(rows, pn, tn, reinterpret_cast<double*>(&o), [&](int l, int j,
+                                                                                                       double* t) {
+        FlavR<R>& n = *reinterpret_cast<FlavR<R>*>(t);
         const double xc = xi * cc[l];
-        for (int j = 0; j < pn; j++) {
-            const double C = Cm[l * pn + j];
-            R E, invE;
-            r_rsqrt_sqrt(fma(xc, pp[j], pp[j]) + M2, invE, E);
-            const R a = (mu - E) * invT, b = -(E + mu) * invT;
-            SignR<R> sp, sm;
-            lnF_r(tab, a, Phi, Phib, sp);
-            lnF_r(tab, b, Phib, Phi, sm);
-            const R gp = 3.0 * sp.gq, gm = 3.0 * sm.gq;
-            const R hp = 3.0 * sp.h, hm = 3.0 * sm.h;
-            const R ac1p = 3.0 * sp.k1, ac2p = 3.0 * sp.k2, ac1m = 3.0 * sm.k1, ac2m = 3.0 * sm.k2;
-            const R QE = -(gp + gm) * invT, QEE = (hp + hm) * invT2;
-            const R QEP = -(ac1p + ac2m) * invT, QEPb = -(ac2p + ac1m) * invT;
-            const R EM = M * invE, EMM = (1.0 - EM * EM) * invE;
-            o.SM += C * (QE * EM);
-            o.SP += C * (3.0 * (sp.r1 + sm.r2));
-            o.SPb += C * (3.0 * (sp.r2 + sm.r1));
-            o.SMM += C * (QEE * EM * EM + QE * EMM);
-            o.SMP += C * (QEP * EM);
-            o.SMPb += C * (QEPb * EM);
-            o.SPP += C * (-9.0 * (sp.r1 * sp.r1 + sm.r2 * sm.r2));
-            o.SPPb += C * (-9.0 * (sp.r1 * sp.r2 + sm.r1 * sm.r2));
-            o.SPbPb += C * (-9.0 * (sp.r2 * sp.r2 + sm.r1 * sm.r1));
-            o.SMmu += C * (-(hp - hm) * invT2) * EM;
-            o.SMT += C * ((gp + gm + hp * a + hm * b) * invT2) * EM;
-            o.SPmu += C * (ac1p - ac2m) * invT;
-            o.SPbmu += C * (ac2p - ac1m) * invT;
-            o.SPT += C * (-(ac1p * a + ac2m * b) * invT);
-            o.SPbT += C * (-(ac2p * a + ac1m * b) * invT);
-        }
-    }
+        const double C = Cm[l * pn + j];
+        R E, invE;
+        r_rsqrt_sqrt(fma(xc, pp[j], pp[j]) + M2, invE, E);
+        const R a = (mu - E) * invT, b = -(E + mu) * invT;
+        SignR<R> sp, sm;
+        lnF_r(tab, a, Phi, Phib, sp);
+        lnF_r(tab, b, Phib, Phi, sm);
+        const R gp = 3.0 * sp.gq, gm = 3.0 * sm.gq;
+        const R hp = 3.0 * sp.h, hm = 3.0 * sm.h;
+        const R ac1p = 3.0 * sp.k1, ac2p = 3.0 * sp.k2, ac1m = 3.0 * sm.k1, ac2m = 3.0 * sm.k2;
+        const R QE = -(gp + gm) * invT, QEE = (hp + hm) * invT2;
+        const R QEP = -(ac1p + ac2m) * invT, QEPb = -(ac2p + ac1m) * invT;
+        const R EM = M * invE, EMM = (1.0 - EM * EM) * invE;
+        n.SM = C * (QE * EM);
+        n.SP = C * (3.0 * (sp.r1 + sm.r2));
+        n.SPb = C * (3.0 * (sp.r2 + sm.r1));
+        n.SMM = C * (QEE * EM * EM + QE * EMM);
+        n.SMP = C * (QEP * EM);
+        n.SMPb = C * (QEPb * EM);
+        n.SPP = C * (-9.0 * (sp.r1 * sp.r1 + sm.r2 * sm.r2));
+        n.SPPb = C * (-9.0 * (sp.r1 * sp.r2 + sm.r1 * sm.r2));
+        n.SPbPb = C * (-9.0 * (sp.r2 * sp.r2 + sm.r1 * sm.r1));
+        n.SMmu = C * (-(hp - hm) * invT2) * EM;
+        n.SMT = C * ((gp + gm + hp * a + hm * b) * invT2) * EM;
+        n.SPmu = C * (ac1p - ac2m) * invT;
+        n.SPbmu = C * (ac2p - ac1m) * invT;
+        n.SPT = C * (-(ac1p * a + ac2m * b) * invT);
+        n.SPbT = C * (-(ac2p * a + ac1m * b) * invT);
+    });
 }
 
 // dI/dM and d2I/dM2 of the vacuum term (pnjl::vacuum_I)
@@ -501,8 +615,8 @@ __device__ void vacuum_r(const DevParams& P, R M, R& dI, R& d2I)
 
 // H = d2 Omega/dx2, FT = d2 Omega/dx dT, Fmu = d2 Omega/dx dmu at (x, T, mu)
 // (the formulas of deriv_kernel)
-template <class R>
-__device__ void hess_theta(const DevParams& P, const double* tab, int pn, int tn, const R* x, R T, R mu, double xi,
+template <int NL, class R>
+__device__ void hess_theta(const DevParams& P, const double* tab, double* rows, int pn, int tn, const R* x, R T, R mu, double xi,
                            R H[5][5], R FT[5], R Fmu[5])
 {
     const double G = P.G, K = P.K;
@@ -510,10 +624,10 @@ __device__ void hess_theta(const DevParams& P, const double* tab, int pn, int tn
     const R M[3] = {P.m_ud0 - 4.0 * G * pu + 2.0 * K * pd * ps, P.m_ud0 - 4.0 * G * pd + 2.0 * K * pu * ps,
                     P.m_s0 - 4.0 * G * ps + 2.0 * K * pu * pd};
     const R c4G = cst<R>(-4.0 * G);
-    const R dM[3][3] = {{c4G, 2.0 * K * ps, 2.0 * K * pd}, {2.0 * K * ps, c4G, 2.0 * K * pu},
-                        {2.0 * K * pd, 2.0 * K * pu, c4G}};
     const R z = cst<R>(0.0);
+#pragma unroll
     for (int a = 0; a < 5; a++) {
+#pragma unroll
         for (int b = 0; b < 5; b++) H[a][b] = z;
         FT[a] = Fmu[a] = z;
     }
@@ -522,37 +636,46 @@ __device__ void hess_theta(const DevParams& P, const double* tab, int pn, int tn
     H[0][2] = H[2][0] = -4.0 * K * pd;
     H[1][2] = H[2][1] = -4.0 * K * pu;
     R SPP = z, SPPb = z, SPbPb = z;
-    FlavR<R> fu;
+    FlavR<R> fu, f;
+    // one copy of the node loop; flavour i's mass and derivatives are picked by
+    // value, so that nothing is indexed in memory
+#pragma unroll 1
     for (int i = 0; i < 3; i++) {
-        FlavR<R> fo;
-        const FlavR<R>* f = &fo;
+        const R Mi = choose(i == 0, M[0], choose(i == 1, M[1], M[2]));
+        const R two_ps = 2.0 * K * ps, two_pd = 2.0 * K * pd, two_pu = 2.0 * K * pu;
+        const R dM[3] = {choose(i == 0, c4G, choose(i == 1, two_ps, two_pd)),
+                         choose(i == 1, c4G, choose(i == 0, two_ps, two_pu)),
+                         choose(i == 2, c4G, choose(i == 0, two_pd, two_pu))};
         if (i == 1 && same(M[1], M[0]))   // phi_d == phi_u: d aliases u
-            f = &fu;
+            f = fu;
         else
-            flavour_r(tab, pn, tn, M[i], mu, T, xi, Phi, Phib, fo);
-        if (i == 0) fu = fo;
+            flavour_r<NL>(tab, rows, pn, tn, Mi, mu, T, xi, Phi, Phib, f);
+        if (i == 0) fu = f;
         R dI, d2I;
-        vacuum_r(P, M[i], dI, d2I);
-        const R gM = -2.0 * P.Nc * dI - 2.0 * T * f->SM, hM = -2.0 * P.Nc * d2I - 2.0 * T * f->SMM;
+        vacuum_r(P, Mi, dI, d2I);
+        const R gM = -2.0 * P.Nc * dI - 2.0 * T * f.SM, hM = -2.0 * P.Nc * d2I - 2.0 * T * f.SMM;
+#pragma unroll
         for (int a = 0; a < 3; a++) {
+#pragma unroll
             for (int b = 0; b < 3; b++) {
-                R h = hM * dM[i][a] * dM[i][b];
+                R h = hM * dM[a] * dM[b];
                 if (a != b && a != i && b != i) h += gM * (2.0 * K);   // d2M_i / dphi_a dphi_b
                 H[a][b] += h;
             }
-            H[a][3] += -2.0 * T * f->SMP * dM[i][a];
-            H[a][4] += -2.0 * T * f->SMPb * dM[i][a];
-            Fmu[a] += dM[i][a] * (-2.0 * T * f->SMmu);
-            FT[a] += dM[i][a] * (-2.0 * f->SM - 2.0 * T * f->SMT);
+            H[a][3] += -2.0 * T * f.SMP * dM[a];
+            H[a][4] += -2.0 * T * f.SMPb * dM[a];
+            Fmu[a] += dM[a] * (-2.0 * T * f.SMmu);
+            FT[a] += dM[a] * (-2.0 * f.SM - 2.0 * T * f.SMT);
         }
-        Fmu[3] += -2.0 * T * f->SPmu;
-        Fmu[4] += -2.0 * T * f->SPbmu;
-        FT[3] += -2.0 * f->SP - 2.0 * T * f->SPT;
-        FT[4] += -2.0 * f->SPb - 2.0 * T * f->SPbT;
-        SPP += f->SPP;
-        SPPb += f->SPPb;
-        SPbPb += f->SPbPb;
+        Fmu[3] += -2.0 * T * f.SPmu;
+        Fmu[4] += -2.0 * T * f.SPbmu;
+        FT[3] += -2.0 * f.SP - 2.0 * T * f.SPT;
+        FT[4] += -2.0 * f.SPb - 2.0 * T * f.SPbT;
+        SPP += f.SPP;
+        SPPb += f.SPPb;
+        SPbPb += f.SPbPb;
     }
+#pragma unroll
     for (int a = 0; a < 3; a++) {
         H[3][a] = H[a][3];
         H[4][a] = H[a][4];
@@ -589,25 +712,29 @@ struct Deriv2Args {
     double* out;   // n * PNJL_IMPLICIT2_FIELDS
 };
 
+template <int NL>
 __global__ void __launch_bounds__(256) deriv2_kernel(Deriv2Args A)
 {
     extern __shared__ double lds[];
     const int tab_len = pnjl::kMathTab + A.pn + A.tn + A.pn * A.tn + A.pn;
     for (int i = threadIdx.x; i < tab_len; i += blockDim.x) lds[i] = A.tab[i];
     __syncthreads();
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t g = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / NL;
     if (g >= A.n) return;
     const DevParams& P = A.P;
     const double T = A.T[g], mu = A.mu[g], xi = A.xi[g];
     double x[5];
+#pragma unroll
     for (int i = 0; i < 5; i++) x[i] = A.x[g * 5 + i];
     double* out = A.out + g * PNJL_IMPLICIT2_FIELDS;
     // first order: x_T, x_mu
     double H[5][5], FT[5], Fmu[5], L[5][5], xT[5], xmu[5];
-    hess_theta<double>(P, lds, A.pn, A.tn, x, T, mu, xi, H, FT, Fmu);
+    hess_theta<NL, double>(P, lds, lds + tab_len, A.pn, A.tn, x, T, mu, xi, H, FT, Fmu);
+#pragma unroll
     for (int a = 0; a < 5; a++) {
         xT[a] = -FT[a];
         xmu[a] = -Fmu[a];
+#pragma unroll
         for (int b = 0; b < 5; b++) L[a][b] = H[a][b];
     }
     bool ok = lu5_solve2(L, xT, xmu);
@@ -615,11 +742,14 @@ __global__ void __launch_bounds__(256) deriv2_kernel(Deriv2Args A)
     double x2[3][5];
     if (ok) {
         D2 xd[5], Hd[5][5], FTd[5], Fmud[5];
+#pragma unroll
         for (int a = 0; a < 5; a++) xd[a] = D2{x[a], xT[a], xmu[a]};
-        hess_theta<D2>(P, lds, A.pn, A.tn, xd, D2{T, 1.0, 0.0}, D2{mu, 0.0, 1.0}, xi, Hd, FTd, Fmud);
+        hess_theta<NL, D2>(P, lds, lds + tab_len, A.pn, A.tn, xd, D2{T, 1.0, 0.0}, D2{mu, 0.0, 1.0}, xi, Hd, FTd, Fmud);
         double r2[5];
+#pragma unroll
         for (int a = 0; a < 5; a++) {
             double tt = FTd[a].t, tm = FTd[a].m, mm = Fmud[a].m;
+#pragma unroll
             for (int b = 0; b < 5; b++) {
                 tt += Hd[a][b].t * xT[b];
                 tm += Hd[a][b].m * xT[b];
@@ -630,17 +760,23 @@ __global__ void __launch_bounds__(256) deriv2_kernel(Deriv2Args A)
             x2[2][a] = -mm;
             r2[a] = 0.0;
         }
+#pragma unroll
         for (int a = 0; a < 5; a++)
+#pragma unroll
             for (int b = 0; b < 5; b++) L[a][b] = H[a][b];
         ok = lu5_solve2(L, x2[0], x2[1]);
+#pragma unroll
         for (int a = 0; a < 5; a++)
+#pragma unroll
             for (int b = 0; b < 5; b++) L[a][b] = H[a][b];
         ok = ok && lu5_solve2(L, x2[2], r2);
     }
+    if (NL > 1 && threadIdx.x % NL) return;
     if (!ok) {
         for (int k = 0; k < PNJL_IMPLICIT2_FIELDS; k++) out[k] = __builtin_nan("");
         return;
     }
+#pragma unroll
     for (int a = 0; a < 5; a++) {
         out[a] = x[a];
         out[5 + a] = xT[a];
@@ -652,12 +788,14 @@ __global__ void __launch_bounds__(256) deriv2_kernel(Deriv2Args A)
     // masses as ThermoDerivatives.jl:111-121 writes them (bare 5.5 and 140.0
     // MeV): M_i = m_i0 - 4 G phi_i + 2 K phi_j phi_k, (j, k) the other two
     const double G = P.G, K = P.K;
+#pragma unroll
     for (int i = 0; i < 3; i++) {
         const int j = (i == 0) ? 1 : 0, k = (i == 2) ? 1 : 2;
         const double m0 = (i == 2) ? 0.140 / 0.197327 : 0.0055 / 0.197327;
         out[30 + i] = m0 - 4.0 * G * x[i] + 2.0 * K * x[j] * x[k];
         out[33 + i] = -4.0 * G * xT[i] + 2.0 * K * (xT[j] * x[k] + x[j] * xT[k]);
         out[36 + i] = -4.0 * G * xmu[i] + 2.0 * K * (xmu[j] * x[k] + x[j] * xmu[k]);
+#pragma unroll
         for (int q = 0; q < 3; q++) {
             const double* va = (q == 2) ? xmu : xT;   // (T, T), (T, mu), (mu, mu)
             const double* vb = (q == 0) ? xT : xmu;
@@ -668,6 +806,27 @@ __global__ void __launch_bounds__(256) deriv2_kernel(Deriv2Args A)
 }
 
 }  // namespace pnjl_deriv
+
+namespace {
+
+// f(NL) with the lanes per root of a batch of n.  One lane per root uses the
+// chip best but walks the mesh alone and leaves the chip idle below some 10^4
+// roots.  Measured (kernel ms, first / second order, p 64): 5000 roots, t 4,
+// at 1 / 16 / 32 / 64 lanes 0.42 / 0.09 / 0.08 / 0.09 and 1.62 / 0.40 / 0.40 /
+// 0.49; 40 000 roots, t 6: 0.67 / 0.56 / 0.59 / 0.76 and 2.56 / 3.00 / 3.75 /
+// 5.46; both calls together at 10 roots 2.25 / 0.43 / 0.34 / 0.30 ms, at
+// 20 000 (t 6) 5.3 ms with 1 and 4.1 with 16.
+template <class F>
+void launch_lanes(int64_t n, const F& f)
+{
+    using std::integral_constant;
+    if (n <= 1024) f(integral_constant<int, 64>());
+    else if (n <= 8192) f(integral_constant<int, 32>());
+    else if (n <= 24576) f(integral_constant<int, 16>());
+    else f(integral_constant<int, 1>());
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -715,7 +874,12 @@ int pnjl_thermo_derivatives_batch(pnjl_ctx* ctx, int64_t n, const double* T, con
     A.out = dout;
     const size_t lds = sizeof(double) * (pnjl::kMathTab + (size_t)p_num + t_num + (size_t)p_num * t_num + p_num);
     HIPCHK(ctx, hipEventRecord(ctx->ev0, st));
-    hipLaunchKernelGGL(pnjl_deriv::deriv_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), lds, st, A);
+    const size_t rows = 256 * sizeof(pnjl_deriv::FlavD);
+    // a node table that leaves no room for the rows: one lane
+    launch_lanes(lds + rows <= 64 * 1024 ? n : INT64_MAX, [&](auto NL) {
+        hipLaunchKernelGGL(pnjl_deriv::deriv_kernel<NL()>, dim3((unsigned)((n * NL() + 255) / 256)), dim3(256),
+                           NL() > 1 ? lds + rows : lds, st, A);
+    });
     HIPCHK(ctx, hipGetLastError());
     HIPCHK(ctx, hipEventRecord(ctx->ev1, st));
     if (!dev)
@@ -772,7 +936,11 @@ int pnjl_implicit_derivatives2_batch(pnjl_ctx* ctx, int64_t n, const double* T, 
     A.out = dout;
     const size_t lds = sizeof(double) * (pnjl::kMathTab + (size_t)p_num + t_num + (size_t)p_num * t_num + p_num);
     HIPCHK(ctx, hipEventRecord(ctx->ev0, st));
-    hipLaunchKernelGGL(pnjl_deriv::deriv2_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), lds, st, A);
+    const size_t rows = 256 * sizeof(pnjl_deriv::FlavR<double>);
+    launch_lanes(lds + rows <= 64 * 1024 ? n : INT64_MAX, [&](auto NL) {
+        hipLaunchKernelGGL(pnjl_deriv::deriv2_kernel<NL()>, dim3((unsigned)((n * NL() + 255) / 256)), dim3(256),
+                           NL() > 1 ? lds + rows : lds, st, A);
+    });
     HIPCHK(ctx, hipGetLastError());
     HIPCHK(ctx, hipEventRecord(ctx->ev1, st));
     if (!dev)

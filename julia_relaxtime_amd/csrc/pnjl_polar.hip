@@ -896,8 +896,8 @@ __global__ void __launch_bounds__(256) grid_a_kernel(Phys P, int npts, const pnj
 
 // k extent of a wavefront's (k0, k) tile: 8 x 8 tiles keep the lanes of a
 // wavefront closer in both momenta than a 1 x 64 row (measured on the 256 x
-// 128 x 64 grid: 31.1 ms per replay against 42.7 ms for 1 x 64 rows, 31.1
-// for 4 x 16, 32.1 for 16 x 4, 35.1 for 2 x 32).
+// 128 x 64 grid: 10.5 ms per call against 12.8 ms for 1 x 64 rows, 10.6 for
+// 4 x 16, 10.8 for 16 x 4, 11.3 for 32 x 2).
 #ifndef PNJL_GRID_TILE_K
 #define PNJL_GRID_TILE_K 8
 #endif

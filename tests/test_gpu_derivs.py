@@ -166,3 +166,25 @@ def test_second_order_derivatives_match_oracle(gpu_ctx, oracle, pn, tn):
         assert np.all(err <= tol), (k, np.flatnonzero(err > tol)[:5], err.max())
     print(f"[deriv2 p{pn} t{tn}] {len(T)} roots ({int(stiff.sum())} next to a spinodal); worst relative "
           f"difference per block: " + ", ".join(f"{k} {v:.1e}" for k, v in worst.items()), flush=True)
+
+
+@pytest.mark.parametrize("n,pn,tn", [(1, 64, 4), (1024, 24, 4), (1025, 24, 4), (8193, 7, 3), (24576, 5, 1), (300, 1, 3),
+                                     (40, 64, 64), (3, 1024, 4)])
+def test_lane_split_does_not_change_results(gpu_ctx, n, pn, tn):
+    """The derivatives of a root are the same bits whatever lanes its batch
+    gives it (sizes on both sides of each change of the split, meshes that do
+    not fill a round, a node table that leaves no room for the rows)."""
+    rng = np.random.default_rng(3)
+    m = 64
+    T, mu = rng.uniform(0.2, 1.4, m), rng.uniform(0.0, 2.0, m)
+    xi = rng.choice([0.0, 0.2, -0.3], m)
+    x = np.stack([rng.uniform(-1.8, -0.1, m), rng.uniform(-1.8, -0.1, m), rng.uniform(-2.2, -0.4, m),
+                  rng.uniform(0.01, 0.9, m), rng.uniform(0.01, 0.9, m)], 1)
+    x[::2, 1] = x[::2, 0]
+    rep = lambda k: [np.resize(a, (k,) + a.shape[1:]) for a in (x, T, mu, xi)]  # noqa: E731
+    for f in (gpu_ctx.thermo_derivatives_batch, gpu_ctx.implicit_derivatives2_batch):
+        one = f(*rep(24577), pn, tn)   # one lane each
+        got = f(*rep(n), pn, tn)
+        for k in got:
+            want = np.resize(np.asarray(one[k])[:m], (n,) + np.asarray(one[k]).shape[1:])
+            assert np.array_equal(got[k], want, equal_nan=True), k
