@@ -237,17 +237,17 @@ ScanGeom scan_geom(int lpp, int pn, int tn, size_t lds_block)
 // leaves room for one wavefront per SIMD only).  The chip holds 2^17 lanes at
 // two wavefronts per SIMD; most solves end early, so the best lane count is
 // the largest with points x lanes <= 2^19.  Measured (p 64, t 4, DefaultSeed
-// at xi != 0, max_iter 40, ms at 8 / 16 / 32 / 64 lanes): 1024 points 4.2 /
-// 3.0 / 2.4 / 2.2, 8192 points 4.7 / 4.1 / 3.5 / 3.5, 32768 points 7.7 / 6.8 /
-// 7.0 / 8.0, 131072 points 22.4 / 22.0 / 23.8 / 30.2 (fixed 4 lanes: 34, 37,
+// at xi != 0, max_iter 40, ms at 8 / 16 / 32 / 64 lanes): 1024 points 3.8 /
+// 2.5 / 1.9 / 1.6, 8192 points 4.4 / 3.6 / 2.9 / 2.7, 32768 points 6.9 / 6.2 /
+// 6.0 / 6.3, 131072 points 22.4 / 22.7 / 23.1 / 24.9 (fixed 4 lanes: 34, 37,
 // 38, 56).  MultiSeed's six candidates per point run long: items x lanes <=
-// 2^20 (32768 points at 8 / 16 / 32 lanes: 17.1 / 17.8 / 22.4 ms, 2048 points
-// 5.1 / 3.6 / 2.7).  The later stages hold few, long items (the listed points'
+// 2^20 (32768 points at 8 / 16 / 32 lanes: 16.7 / 17.2 / 19.3 ms, 2048 points
+// 5.0 / 3.5 / 2.3).  The later stages hold few, long items (the listed points'
 // MultiSeed candidates): points x lanes <= 2^20, at least 16 (p 64, t 4,
-// xi != 0, stage-2 lanes 16 / 64: 16384 points 5.9 / 4.6 ms, 131072 points
-// 22.0 / 23.4).  A chain is serial over its points: 32 lanes up to 4096 chains
-// (16 x 24 x 8 nodes, 256 chains: 14.8 ms at 8, 8.3 at 32, 8.4 at 64), then
-// 16.
+// xi != 0, stage-2 lanes 16 / 64: 16384 points 7.0 / 5.6 ms, 131072 points
+// 22.4 / 23.0).  A chain is serial over its points: 64 lanes up to 2048 chains
+// (16 points x 24 x 8 nodes, 256 chains: 14.2 ms at 8, 5.7 at 32, 4.3 at 64),
+// then 32 (12 x 6 nodes, 4096 chains: 5.7 ms at 64, 5.3 at 32).
 pnjl_launch_cfg choose_cfg(const pnjl_launch_cfg& c, const pnjl::ScanArgs& A)
 {
     if (c.lanes_per_point != kDefaultCfg.lanes_per_point || c.chunk != kDefaultCfg.chunk ||
@@ -258,7 +258,7 @@ pnjl_launch_cfg choose_cfg(const pnjl_launch_cfg& c, const pnjl::ScanArgs& A)
         while (l > least && items > total / l) l /= 2;
         return l;
     };
-    if (A.plan == pnjl::PLAN_CHAINS) return pnjl_launch_cfg{A.n_items <= 4096 ? 32 : 16, 1, 8, 0};
+    if (A.plan == pnjl::PLAN_CHAINS) return pnjl_launch_cfg{A.n_items <= 2048 ? 64 : 32, 1, 8, 0};
     const bool many = A.plan == pnjl::PLAN_MULTI;
     const int l = lanes(A.n_points * A.mult, many ? 1 << 20 : 1 << 19, 8);
     return pnjl_launch_cfg{l, 1, l > 8 ? 8 : 16, std::max(l, lanes(A.n_points, 1 << 20, 16))};

@@ -398,10 +398,141 @@ __device__ __forceinline__ void flavour_sums(const double* lds, int pn, int tn, 
     flav_finish(acc, invT);
 }
 
+// ---- the pass of 32- and 64-lane groups ------------------------------------
+// These groups serve calls that leave the chip idle: a pass is a chain of
+// dependent FP64 instructions of one or two wavefronts per SIMD, and its time
+// is the solve's.  So the u and s flavours run side by side through one walk
+// over the whole p x t mesh (two independent chains per lane; the lanes take
+// the mesh's nodes in one sequence, so a last round is the only ragged one),
+// and all 26 sums are reduced together, each step halving the registers that
+// hold them: v_permlane32_swap and v_permlane16_swap put two sums' halves into
+// one register, so one add serves two sums, and no step goes through LDS.  A
+// pass of a 64-lane group, by the clock: 64 nodes 11.0e3 -> 4.6e3 cycles, 12 x
+// 6 nodes 18.7e3 -> 5.3e3, 64 x 8 nodes 24.1e3 -> 14.0e3.
+// a's upper lanes of each pair of kRow-lane rows exchanged with b's lower ones
+template <int kRow>
+__device__ __forceinline__ void swap_rows(double& a, double& b)
+{
+    const unsigned long long ua = __builtin_bit_cast(unsigned long long, a), ub = __builtin_bit_cast(unsigned long long, b);
+    unsigned long long ra, rb;
+    if constexpr (kRow == 32) {
+        const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)ua, (unsigned)ub, false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+        ra = ((unsigned long long)hi[0] << 32) | lo[0];
+        rb = ((unsigned long long)hi[1] << 32) | lo[1];
+    } else {
+        const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)ua, (unsigned)ub, false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+        ra = ((unsigned long long)hi[0] << 32) | lo[0];
+        rb = ((unsigned long long)hi[1] << 32) | lo[1];
+    }
+    a = __builtin_bit_cast(double, ra);
+    b = __builtin_bit_cast(double, rb);
+}
+
+// Sums v[0..NV) over the group's lanes and stores them to the group's state
+// at f.  After the row steps, register m holds sum 4 m + {0, 2, 1, 3} (64
+// lanes) or 2 m + {0, 1} (32 lanes) in the rows of the group, a partial per
+// lane; the steps within a row are the butterfly of group_sum.
+template <int LPP, int NV>
+__device__ __forceinline__ void reduce_store(double* v, const Scr& s, int f, int gl)
+{
+    static_assert(LPP == 32 || LPP == 64, "whole rows of a wavefront");
+    constexpr int n1 = LPP == 64 ? (NV + 1) / 2 : NV, n2 = (n1 + 1) / 2;
+    if constexpr (LPP == 64) {
+#pragma unroll
+        for (int k = 0; k < n1; k++) {
+            double a = v[2 * k], b = 2 * k + 1 < NV ? v[2 * k + 1] : 0.0;
+            swap_rows<32>(a, b);
+            v[k] = a + b;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < n2; k++) {
+        double a = v[2 * k], b = 2 * k + 1 < n1 ? v[2 * k + 1] : 0.0;
+        swap_rows<16>(a, b);
+        v[k] = a + b;
+    }
+#pragma unroll
+    for (int k = 0; k < n2; k++) v[k] += dpp_f64<DPP_ROW_MIRROR>(v[k]);
+#pragma unroll
+    for (int k = 0; k < n2; k++) v[k] += dpp_f64<DPP_ROW_HALF_MIRROR>(v[k]);
+#pragma unroll
+    for (int k = 0; k < n2; k++) v[k] += dpp_f64<DPP_QUAD_XOR1>(v[k]);
+#pragma unroll
+    for (int k = 0; k < n2; k++) v[k] += dpp_f64<DPP_QUAD_XOR2>(v[k]);
+    const int row = gl >> 4;
+    const int sub = LPP == 64 ? ((row & 1) << 1 | (row >> 1)) : row;
+    constexpr int per = LPP / 16;
+#pragma unroll
+    for (int k = 0; k < n2; k++)
+        if (per * k + per <= NV || per * k + sub < NV) s.at(f + per * k + sub) = v[k];
+    // other lanes read them (one wavefront: LDS accesses complete in order)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// this lane's share of the node sums of NF flavours: nodes e = gl, gl + LPP,
+// ... of the mesh e = l pn + j (of the pn momentum nodes at xi = 0)
+template <int LPP, int NF, bool kChecked>
+__device__ __forceinline__ void node_loop_wide(const double* lds, int pn, int tn, unsigned div, const double* M2,
+                                               double muT, double invT, double K2mu, double xi, double Phi, double Phib,
+                                               int gl, FlavSums* acc)
+{
+    const double* pp = lds + kMathTab;
+    const double* cc = pp + pn;
+    const double* Cm = pp + pn + tn;
+    const bool iso = xi == 0.0;
+    const double* C = iso ? Cm + pn * tn : Cm;
+    const int total = iso ? pn : pn * tn;
+#pragma unroll 1
+    for (int e = gl; e < total; e += LPP) {
+        double q;
+        if (iso) {
+            q = pp[e];
+        } else {
+            const int l = div ? (int)__umulhi((unsigned)e, div) : e, j = e - l * pn;
+            q = fma(xi * cc[l], pp[j], pp[j]);
+        }
+        const double Ce = C[e];
+#pragma unroll
+        for (int f = 0; f < NF; f++) node_accumulate<kChecked>(lds, q, Ce, M2[f], muT, invT, K2mu, Phi, Phib, acc[f]);
+    }
+}
+
+template <int LPP, int NF>
+__device__ __forceinline__ void flavours_wide(const double* lds, int pn, int tn, unsigned div, const double* M, double invT,
+                                              double muT, double K2mu, double xi, double Phi, double Phib, int gl,
+                                              const Scr& s, int f)
+{
+    FlavSums acc[NF];
+    double M2[NF];
+#pragma unroll
+    for (int i = 0; i < NF; i++) {
+        M2[i] = M[i] * M[i];
+        flav_zero(acc[i]);
+    }
+    if (__any(!nodes_all_fast(Phi, Phib, muT)))
+        node_loop_wide<LPP, NF, true>(lds, pn, tn, div, M2, muT, invT, K2mu, xi, Phi, Phib, gl, acc);
+    else
+        node_loop_wide<LPP, NF, false>(lds, pn, tn, div, M2, muT, invT, K2mu, xi, Phi, Phib, gl, acc);
+    double v[13 * NF];
+#pragma unroll
+    for (int i = 0; i < NF; i++) {
+        flav_finish(acc[i], invT);
+        const FlavSums& a = acc[i];
+        const double t[13] = {a.S, a.A1, a.A2, a.SP, a.SPb, a.B1, a.B2, a.SPP, a.SPPb, a.SPbPb, a.Sfp, a.Sfm, a.Sfab};
+#pragma unroll
+        for (int k = 0; k < 13; k++) v[13 * i + k] = t[k];
+    }
+    reduce_store<LPP, 13 * NF>(v, s, SB_SUMS + 13 * f, gl);
+}
+
 // Node pass at state x: u, s, and d unless M_d == M_u (then d aliases u);
-// the reduced sums go to the group's LDS state.
+// the reduced sums go to the group's LDS state.  div: see node_div.
 template <int LPP>
-__device__ __forceinline__ void node_pass(const DevParams& P, const double* lds, int pn, int tn, const Scr& s,
+__device__ __forceinline__ void node_pass(const DevParams& P, const double* lds, int pn, int tn, unsigned div, const Scr& s,
                                           const double* x, double T, double mu, double xi, bool sym, int gl)
 {
     double M[3];
@@ -410,15 +541,24 @@ __device__ __forceinline__ void node_pass(const DevParams& P, const double* lds,
     const double invT = 1.0 / T;
     const double muT = mu * invT;
     const double K2mu = exp(-2.0 * muT);
-    const int nf = sym ? 2 : 3;
+    if constexpr (LPP >= 32) {
+        const double Mus[2] = {M[0], M[2]};
+        flavours_wide<LPP, 2>(lds, pn, tn, div, Mus, invT, muT, K2mu, xi, x[3], x[4], gl, s, 0);
+        if (!sym) flavours_wide<LPP, 1>(lds, pn, tn, div, M + 1, invT, muT, K2mu, xi, x[3], x[4], gl, s, 2);
+    } else {
+        const int nf = sym ? 2 : 3;
 #pragma unroll 1
-    for (int f = 0; f < nf; f++) {
-        double Mf = (f == 0) ? M[0] : ((f == 1) ? M[2] : M[1]);
-        FlavSums acc;
-        flavour_sums<LPP>(lds, pn, tn, Mf, invT, muT, K2mu, xi, x[3], x[4], gl, acc);
-        store_flav(s, f, acc);
+        for (int f = 0; f < nf; f++) {
+            double Mf = (f == 0) ? M[0] : ((f == 1) ? M[2] : M[1]);
+            FlavSums acc;
+            flavour_sums<LPP>(lds, pn, tn, Mf, invT, muT, K2mu, xi, x[3], x[4], gl, acc);
+            store_flav(s, f, acc);
+        }
     }
 }
+
+// e / pn = umulhi(e, node_div(pn)) for the mesh's e <= 4096 (0: pn = 1)
+__device__ __forceinline__ unsigned node_div(int pn) { return pn > 1 ? 0xffffffffu / (unsigned)pn + 1u : 0u; }
 
 // scratch slot holding the sums of mass index i (0 u, 1 d, 2 s)
 __device__ __forceinline__ int slot_of(int i, bool sym) { return i == 0 ? 0 : (i == 2 ? 1 : (sym ? 0 : 2)); }
@@ -534,16 +674,46 @@ __device__ __forceinline__ void assemble_core(const DevParams& P, const Scr& s, 
     Jp[sidx(4, 4)] = -(T4 * (Tb * lPbPb) + m2T * SPbPb);
 }
 
-// Candidate record at x: thermodynamics (calculate_thermo + densities, in
-// closed form from the sums) and the physicality gate
-// (_default_is_physical_solution + _all_finite_thermo, ImplicitSolver.jl:50-64).
+// A candidate record is made in two steps.  raw_rec notes the state, Omega, the
+// residual and the node sums the thermodynamics needs (in fields that
+// finish_rec fills); finish_rec computes the rest in place, once, when the
+// attempt ends: the trust region accepts a point on most of its up to 1000
+// steps, and only the last one's record is used (a step of a 64-lane group,
+// control only: 11.2e3 -> 9.1e3 cycles).
 // x is the group's current state st.x, read here from LDS.
-__device__ __noinline__ void put_rec(Scr s, int blk, double mu, double T, bool sym,
-                        double phi_tol, double omega, double res, int it, bool fconv, bool xconv)
+enum RawField { RW_FAB = RF_P, RW_S = RF_M, RW_FP = RF_NQ, RW_FM = RF_NQB };   // one per quark
+
+__device__ __forceinline__ void raw_rec(const Scr& s, int blk, bool sym, double omega, double res, int it, bool fconv,
+                                        bool xconv)
 {
     const double* x = s.st().x;
+#pragma unroll
+    for (int i = 0; i < 5; i++) s.rec(blk + RF_X + i) = x[i];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const int b = SB_SUMS + 13 * slot_of(i, sym);
+        s.rec(blk + RW_S + i) = s.at(b + SF_S);
+        s.rec(blk + RW_FP + i) = s.at(b + SF_Sfp);
+        s.rec(blk + RW_FM + i) = s.at(b + SF_Sfm);
+        s.rec(blk + RW_FAB + i) = s.at(b + SF_Sfab);
+    }
+    s.rec(blk + RF_OMEGA) = omega;
+    s.rec(blk + RF_RES) = res;
+    s.rec(blk + RF_IT) = (double)it;
+    s.rec(blk + RF_FCONV) = fconv ? 1.0 : 0.0;
+    s.rec(blk + RF_XCONV) = xconv ? 1.0 : 0.0;
+}
+
+// Thermodynamics of a raw record (calculate_thermo + densities, in closed form
+// from the sums) and the physicality gate (_default_is_physical_solution +
+// _all_finite_thermo, ImplicitSolver.jl:50-64).
+__device__ __noinline__ void finish_rec(Scr s, int blk, double mu, double T, double phi_tol)
+{
     const DevParams& P = cold_args.P;
-    double M[3];
+    double x[5], M[3];
+#pragma unroll
+    for (int i = 0; i < 5; i++) x[i] = s.rec(blk + RF_X + i);
+    const double omega = s.rec(blk + RF_OMEGA);
     mass_vec(P, x, M);
     const double Phi = x[3], Phib = x[4];
     double Tr = P.T0 / T;
@@ -560,11 +730,10 @@ __device__ __noinline__ void put_rec(Scr s, int blk, double mu, double T, bool s
     const double twoNc = 2.0 * P.Nc;
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        const int b = SB_SUMS + 13 * slot_of(i, sym);
-        double sfp = s.at(b + SF_Sfp), sfm = s.at(b + SF_Sfm);
+        const double sfp = s.rec(blk + RW_FP + i), sfm = s.rec(blk + RW_FM + i);
         rsum += 6.0 * (sfp - sfm);
-        Sab += s.at(b + SF_Sfab);
-        Ssum += s.at(b + SF_S);
+        Sab += s.rec(blk + RW_FAB + i);
+        Ssum += s.rec(blk + RW_S + i);
         s.rec(blk + RF_NQ + i) = twoNc * sfp;
         s.rec(blk + RF_NQB + i) = twoNc * sfm;
         s.rec(blk + RF_M + i) = M[i];
@@ -578,17 +747,10 @@ __device__ __noinline__ void put_rec(Scr s, int blk, double mu, double T, bool s
 #pragma unroll
     for (int i = 0; i < 3; i++) ph = ph && isfinite(M[i]) && (M[i] > 0.0);
     ph = ph && isfinite(omega) && isfinite(pressure) && isfinite(rho_norm) && isfinite(entropy) && isfinite(energy);
-#pragma unroll
-    for (int i = 0; i < 5; i++) s.rec(blk + RF_X + i) = x[i];
-    s.rec(blk + RF_OMEGA) = omega;
     s.rec(blk + RF_P) = pressure;
     s.rec(blk + RF_RHO) = rho_norm;
     s.rec(blk + RF_S) = entropy;
     s.rec(blk + RF_E) = energy;
-    s.rec(blk + RF_RES) = res;
-    s.rec(blk + RF_IT) = (double)it;
-    s.rec(blk + RF_FCONV) = fconv ? 1.0 : 0.0;
-    s.rec(blk + RF_XCONV) = xconv ? 1.0 : 0.0;
     s.rec(blk + RF_PHYS) = ph ? 1.0 : 0.0;
     s.rec(blk + RF_EXC) = 0.0;
     s.rec(blk + RF_FLAGS) = 0.0;
@@ -632,7 +794,9 @@ __device__ __forceinline__ void unpack5(const double Jp[15], double A[5][5])
 
 // In-place LU with partial pivoting (largest |pivot|, first on ties), then
 // solves A x = b (b is overwritten by x).  Returns true when a pivot is
-// exactly zero (Julia's SingularException).
+// exactly zero (Julia's SingularException).  A row exchange is skipped where no
+// lane of the wavefront needs it (200 selects on a chain of dependent
+// operations that a small call waits for on every step).
 __device__ __forceinline__ bool lu_solve5(double A[5][5], double b[5])
 {
     bool sing = false;
@@ -649,16 +813,18 @@ __device__ __forceinline__ bool lu_solve5(double A[5][5], double b[5])
         }
 #pragma unroll
         for (int i = k + 1; i < 5; i++) {
-            bool sw = (p == i);
+            const bool sw = (p == i);
+            if (__any(sw)) {
 #pragma unroll
-            for (int j = k; j < 5; j++) {
-                double t = A[k][j];
-                A[k][j] = sw ? A[i][j] : t;
-                A[i][j] = sw ? t : A[i][j];
+                for (int j = k; j < 5; j++) {
+                    double t = A[k][j];
+                    A[k][j] = sw ? A[i][j] : t;
+                    A[i][j] = sw ? t : A[i][j];
+                }
+                double t = b[k];
+                b[k] = sw ? b[i] : t;
+                b[i] = sw ? t : b[i];
             }
-            double t = b[k];
-            b[k] = sw ? b[i] : t;
-            b[i] = sw ? t : b[i];
         }
         sing = sing || (A[k][k] == 0.0);
         double ip = 1.0 / A[k][k];
@@ -1410,7 +1576,7 @@ __device__ __noinline__ bool tr_step(Scr s, St&, double omega)
     if (st.fresh) {
         st.fresh = false;
         bool fconv = norm_inf5(F) < A.ftol;
-        put_rec(s, SB_TRC, st.mu, st.T, st.sym, A.phi_tol, omega, norm_inf5(F), 0, fconv, false);
+        raw_rec(s, SB_TRC, st.sym, omega, norm_inf5(F), 0, fconv, false);
 #pragma unroll
         for (int i = 0; i < 5; i++) r[i] = F[i];
 #pragma unroll
@@ -1475,7 +1641,7 @@ __device__ __noinline__ bool tr_step(Scr s, St&, double omega)
             bool xconv = !xnan && cheb < A.xtol;
             bool fconv = norm_inf5(r) < A.ftol;
             converged = xconv || fconv;
-            put_rec(s, SB_TRC, st.mu, st.T, st.sym, A.phi_tol, omega, norm_inf5(r), st.it, fconv, xconv);
+            raw_rec(s, SB_TRC, st.sym, omega, norm_inf5(r), st.it, fconv, xconv);
         } else {
 #pragma unroll
             for (int i = 0; i < 5; i++) st.x[i] = s.at(SB_XOLD + i);
@@ -1506,6 +1672,7 @@ __device__ __noinline__ bool tr_step(Scr s, St&, double omega)
         if (st.sym) st.x[1] = st.x[0];
         return true;
     }
+    finish_rec(s, SB_TRC, st.mu, st.T, A.phi_tol);
     s.rec(SB_TRC + RF_IT) = (double)st.it;
     return false;
 }
@@ -1558,7 +1725,8 @@ __device__ __forceinline__ void control_step(const ScanArgs& A, const Scr& s, St
         }
         // Newton finished: candidate at x
         double res = norm_inf5(F);
-        put_rec(s, SB_PRIM, st.mu, st.T, st.sym, A.phi_tol, omega, res, st.it, fconv, xconv);
+        raw_rec(s, SB_PRIM, st.sym, omega, res, st.it, fconv, xconv);
+        finish_rec(s, SB_PRIM, st.mu, st.T, A.phi_tol);
         bool good = rec_good(s, SB_PRIM, A.resmax);
         if (A.tr_fb && !good && st.attempt != ATT_SURR) {
             st.phase = PH_TR;
@@ -1614,6 +1782,7 @@ __global__ void __launch_bounds__(256, 2) scan_kernel(ScanArgs A)
     const int gl = threadIdx.x % LPP;
     const Scr s{(int)(tab_len + (threadIdx.x / LPP) * STATE_STRIDE)};
     const bool chains = (A.plan == PLAN_CHAINS);
+    const unsigned div = node_div(A.pn);
     St& st = s.st();
     st.phase = PH_IDLE;
     st.item = 0;
@@ -1644,7 +1813,7 @@ __global__ void __launch_bounds__(256, 2) scan_kernel(ScanArgs A)
             double x[5];
 #pragma unroll
             for (int i = 0; i < 5; i++) x[i] = st.x[i];
-            node_pass<LPP>(A.P, lds, A.pn, A.tn, s, x, st.T, st.mu, st.xi, st.sym, gl);
+            node_pass<LPP>(A.P, lds, A.pn, A.tn, div, s, x, st.T, st.mu, st.xi, st.sym, gl);
             st.passes += st.sym ? 2 : 3;
         }
         control_step<LPP>(A, s, st, gl);
@@ -1741,7 +1910,7 @@ __global__ void __launch_bounds__(256, 3) residual_kernel(ResArgs R)
 #pragma unroll
     for (int i = 0; i < 5; i++) x[i] = R.x[g * 5 + i];
     bool sym = (x[0] == x[1]);
-    node_pass<LPP>(R.P, lds, R.pn, R.tn, s, x, R.T[g], R.mu[g], R.xi[g], sym, gl);
+    node_pass<LPP>(R.P, lds, R.pn, R.tn, node_div(R.pn), s, x, R.T[g], R.mu[g], R.xi[g], sym, gl);
     double omega, F[5], Jp[15];
     assemble_core<LPP>(R.P, s, x, R.T[g], sym, omega, F, Jp, gl);
     if (gl == 0) {

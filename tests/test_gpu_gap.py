@@ -305,7 +305,7 @@ def test_launch_geometry_does_not_change_results(gpu_ctx):
 
 
 @pytest.mark.parametrize("policy,n,chain", [(0, 1, 0), (0, 8191, 0), (0, 8193, 0), (0, 16385, 0), (0, 32769, 0), (3, 2731, 0),
-                                            (3, 2730, 0), (5, 3 * 4096, 3), (5, 3 * 4097, 3)])
+                                            (3, 2730, 0), (5, 3 * 2048, 3), (5, 3 * 2049, 3)])
 def test_default_geometry_picks_lanes(gpu_ctx, policy, n, chain):
     """The default launch geometry chooses lanes per point by the number of
     points (here on both sides of its lines): the same roots as a fixed 4-lane
@@ -329,6 +329,36 @@ def test_default_geometry_picks_lanes(gpu_ctx, policy, n, chain):
     J = gpu_ctx.residual_batch(b["x"], T, mu, xi, 16, 4)[1]
     bound = 2e-10 * np.abs(np.linalg.inv(J)).sum(axis=2).max(axis=1) + 1e-13
     assert np.all(np.abs(a["x"] - b["x"]).max(axis=1) <= bound)
+
+
+@pytest.mark.parametrize("lpp", [32, 64])
+@pytest.mark.parametrize("pn,tn,xi", [(64, 4, 0.0), (65, 3, 0.0), (1, 1, 0.3), (1, 64, 0.3), (12, 6, -0.2), (31, 2, 0.4),
+                                      (64, 1, 0.2), (64, 64, 0.1), (7, 9, 0.0)])
+def test_wide_group_node_pass(gpu_ctx, lpp, pn, tn, xi):
+    """One Newton step of a 32- or 64-lane group (both flavours side by side, the
+    flattened mesh, the row-swap reduction) against a 4-lane group's, at meshes
+    that do and do not fill a round.  max_iter = 0: the outputs are Omega, the
+    residual and the thermodynamics at the seed, sums of the same node terms
+    in another order, 1e-13 of their size each (|terms| summed: at most 1e3
+    times the smallest of them)."""
+    from julia_relaxtime_amd import _lib
+    r = np.random.default_rng(pn * tn)
+    n = 70
+    T, mu = r.uniform(0.2, 1.4, n), r.uniform(0.0, 2.0, n)
+    seed = np.stack([r.uniform(-1.8, -0.1, n), r.uniform(-1.8, -0.1, n), r.uniform(-2.2, -0.4, n), r.uniform(-0.3, 0.9, n),
+                     r.uniform(0.01, 0.9, n)], 1)
+    seed[::2, 1] = seed[::2, 0]     # phi_u = phi_d: two flavours, else three
+    opts = _lib.default_opts(max_iter=0, trust_region_fallback=0, auto_multiseed_fallback=0)
+    out = []
+    try:
+        for l in (4, lpp):
+            gpu_ctx.set_launch_cfg(l, 1, 8, 0)
+            out.append(gpu_ctx.solve_batch(T, mu, xi, policy=4, seed=seed, p_num=pn, t_num=tn, opts=opts))
+    finally:
+        gpu_ctx.set_launch_cfg()
+    for k in ("omega", "rho_norm", "entropy", "energy", "n_q", "n_qbar", "residual_norm", "x"):
+        a, b = out[0][k], out[1][k]
+        assert np.all(np.abs(a - b) <= 1e-13 * (1e3 + np.abs(a))), k
 
 
 def test_device_pointer_path(gpu_ctx):
