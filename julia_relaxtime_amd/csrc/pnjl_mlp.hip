@@ -34,6 +34,15 @@
 namespace mlp {
 
 constexpr int IN = 3, H = 128, OUT = 4, TILE = 32, THREADS = 256;
+// A training step is one tile per CU (batch 8192: 256 blocks), a chain of
+// short phases between barriers: 16 wavefronts per tile hide the LDS and
+// weight latency that 4 waited for (one MFMA tile per wavefront and phase).
+// 32 steps of batch 8192: the kernel 33.6 -> 26.1 us per step.
+constexpr int TRAIN_THREADS = 1024;
+// row stride of the activation tiles in LDS: 16 bytes more than a row, so that
+// the 16 rows of a fragment load lie in different banks (a stride of 256
+// bytes puts all of them in the same four)
+constexpr int LD = H + 8;
 // packed FP32 parameter vector (row-major): W1[H][IN] b1[H] W2[H][H] b2[H] W3[H][H] b3[H] W4[OUT][H] b4[OUT]
 constexpr int OFF_W1 = 0, OFF_B1 = OFF_W1 + H * IN, OFF_W2 = OFF_B1 + H, OFF_B2 = OFF_W2 + H * H,
               OFF_W3 = OFF_B2 + H, OFF_B3 = OFF_W3 + H * H, OFF_W4 = OFF_B3 + H, OFF_B4 = OFF_W4 + OUT * H,
@@ -113,15 +122,16 @@ __device__ __forceinline__ us8 gather8(const unsigned short* p, int stride)
 }
 
 // forward hidden layer: out[s][o] = silu(sum_i in[s][i] W[o][i] + b[o]); also silu'(z)
+template <int NT>
 __device__ void fwd_hidden(const unsigned short* in, const unsigned short* W, const float* b, unsigned short* out,
                            unsigned short* gout)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = lane & 15, q = lane >> 4;
-    for (int t = wave; t < (TILE / 16) * (H / 16); t += THREADS / 64) {
+    for (int t = wave; t < (TILE / 16) * (H / 16); t += NT / 64) {
         const int ts = t / (H / 16), to = t % (H / 16);
         float4v acc = mma_tile(
-            H, [&](int kk) { return ld8(in + (ts * 16 + r) * H + kk + 8 * q); },
+            H, [&](int kk) { return ld8(in + (ts * 16 + r) * LD + kk + 8 * q); },
             [&](int kk) { return ld8(W + (to * 16 + r) * H + kk + 8 * q); });
         const int o = to * 16 + r;
         const float bo = b[o];
@@ -130,74 +140,88 @@ __device__ void fwd_hidden(const unsigned short* in, const unsigned short* W, co
             const int srow = ts * 16 + 4 * q + i;
             float z = acc[i] + bo;
             float sg = sigmoidf_(z);
-            out[srow * H + o] = f2bf(z * sg);
-            if (gout) gout[srow * H + o] = f2bf(sg * (1.0f + z * (1.0f - sg)));
+            out[srow * LD + o] = f2bf(z * sg);
+            if (gout) gout[srow * LD + o] = f2bf(sg * (1.0f + z * (1.0f - sg)));
         }
     }
 }
 
 // backward through a hidden layer's weights: dh[s][i] = sum_o dz[s][o] W[o][i],
 // then dzp[s][i] = dh * g[s][i] (BF16)
+template <int NT>
 __device__ void bwd_data(const unsigned short* dz, const unsigned short* WT, const unsigned short* g,
                          unsigned short* dzp)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = lane & 15, q = lane >> 4;
-    for (int t = wave; t < (TILE / 16) * (H / 16); t += THREADS / 64) {
+    for (int t = wave; t < (TILE / 16) * (H / 16); t += NT / 64) {
         const int ts = t / (H / 16), ti = t % (H / 16);
         float4v acc = mma_tile(
-            H, [&](int kk) { return ld8(dz + (ts * 16 + r) * H + kk + 8 * q); },
+            H, [&](int kk) { return ld8(dz + (ts * 16 + r) * LD + kk + 8 * q); },
             [&](int kk) { return ld8(WT + (ti * 16 + r) * H + kk + 8 * q); });
         const int i0 = ti * 16 + r;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int srow = ts * 16 + 4 * q + i;
-            dzp[srow * H + i0] = f2bf(acc[i] * bf2f(g[srow * H + i0]));
+            dzp[srow * LD + i0] = f2bf(acc[i] * bf2f(g[srow * LD + i0]));
         }
     }
 }
 
-// weight gradient of a hidden layer: dW[o][i] = sum_s dz[s][o] in[s][i]
+// weight gradient of a hidden layer: dW[o][i] = sum_s dz[s][o] in[s][i].  A
+// wavefront takes a run of tiles of one row of tiles: dz's fragment is
+// gathered once for them.
+template <int NT>
 __device__ void bwd_weight(const unsigned short* dz, const unsigned short* in, float* dW)
 {
+    constexpr int kTiles = (H / 16) * (H / 16), kRun = kTiles / (NT / 64);
+    static_assert(TILE == 32 && kRun * (NT / 64) == kTiles && (H / 16) % kRun == 0, "one K step, whole runs");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = lane & 15, q = lane >> 4;
-    for (int t = wave; t < (H / 16) * (H / 16); t += THREADS / 64) {
-        const int to = t / (H / 16), ti = t % (H / 16);
+    const int to = wave * kRun / (H / 16);
+    const us8 a = gather8(dz + 8 * q * LD + to * 16 + r, LD);
+#pragma unroll
+    for (int u = 0; u < kRun; u++) {
+        const int ti = (wave * kRun + u) % (H / 16);
         float4v acc = mma_tile(
-            TILE, [&](int kk) { return gather8(dz + (kk + 8 * q) * H + to * 16 + r, H); },
-            [&](int kk) { return gather8(in + (kk + 8 * q) * H + ti * 16 + r, H); });
+            TILE, [&](int) { return a; }, [&](int) { return gather8(in + 8 * q * LD + ti * 16 + r, LD); });
         const int i0 = ti * 16 + r;
 #pragma unroll
         for (int i = 0; i < 4; i++) dW[(to * 16 + 4 * q + i) * H + i0] = acc[i];
     }
 }
 
-struct Smem {
+// a tile's activations
+struct Tile {
     float xs[TILE][IN];
-    float tg[TILE][OUT];
     float y[TILE][OUT];
-    float dy[TILE][OUT];
-    float red[THREADS];
-    int valid[TILE];
-    unsigned short h1[TILE * H], h2[TILE * H], h3[TILE * H];
+    alignas(16) unsigned short h1[TILE * LD], h2[TILE * LD], h3[TILE * LD];
     // silu'(z) of each hidden layer; the backward pass overwrites g_l in place
     // with dL/dz_l (each element is read once, then written by the same lane)
-    unsigned short g1[TILE * H], g2[TILE * H], g3[TILE * H];
+    unsigned short g1[TILE * LD], g2[TILE * LD], g3[TILE * LD];
+};
+static_assert(3 * sizeof(Tile) <= 160 * 1024, "three inference tiles per CU");
+
+struct Smem : Tile {
+    float tg[TILE][OUT];
+    float dy[TILE][OUT];
+    float red[TILE * OUT];
+    int valid[TILE];
 };
 static_assert(sizeof(Smem) <= 64 * 1024, "LDS budget");
 
 // first layer (K = 3) with scalar FMAs
+template <int NT>
 __device__ void fwd_first(Smem& S, const unsigned short* W1, const float* b1)
 {
-    for (int e = threadIdx.x; e < TILE * H; e += THREADS) {
-        const int s = e / H, o = e % H;
+    for (int e = threadIdx.x; e < TILE * H; e += NT) {
+        const int s = e / H, o = e % H, i = s * LD + o;
         float z = b1[o];
 #pragma unroll
         for (int k = 0; k < IN; k++) z += bf2f(W1[o * IN + k]) * S.xs[s][k];
         float sg = sigmoidf_(z);
-        S.h1[e] = f2bf(z * sg);
-        S.g1[e] = f2bf(sg * (1.0f + z * (1.0f - sg)));
+        S.h1[i] = f2bf(z * sg);
+        S.g1[i] = f2bf(sg * (1.0f + z * (1.0f - sg)));
     }
 }
 
@@ -207,19 +231,25 @@ __device__ void fwd_last(Smem& S, const unsigned short* W4, const float* b4)
     for (int e = threadIdx.x; e < TILE * OUT; e += THREADS) {
         const int s = e / OUT, j = e % OUT;
         float z = b4[j];
-        for (int o = 0; o < H; o++) z += bf2f(W4[j * H + o]) * bf2f(S.h3[s * H + o]);
+#pragma unroll 4
+        for (int o = 0; o < H; o += 8) {
+            const us8 w = ld8(W4 + j * H + o), h = ld8(S.h3 + s * LD + o);
+#pragma unroll
+            for (int i = 0; i < 8; i++) z += bf2f(w[i]) * bf2f(h[i]);
+        }
         S.y[s][j] = z;
     }
 }
 
-__global__ void __launch_bounds__(THREADS) train_tile_kernel(TrainArgs A)
+__global__ void __launch_bounds__(TRAIN_THREADS) train_tile_kernel(TrainArgs A)
 {
+    constexpr int NT = TRAIN_THREADS;
     extern __shared__ unsigned char smem_raw[];
     Smem& S = *reinterpret_cast<Smem*>(smem_raw);
     const int64_t row0 = (int64_t)blockIdx.x * TILE;
     float* G = A.partial + (int64_t)blockIdx.x * NPARAM;
     // gather the tile
-    for (int s = threadIdx.x; s < TILE; s += THREADS) {
+    for (int s = threadIdx.x; s < TILE; s += NT) {
         int64_t row = row0 + s;
         bool ok = row < A.batch;
         int64_t idx = 0;
@@ -232,35 +262,36 @@ __global__ void __launch_bounds__(THREADS) train_tile_kernel(TrainArgs A)
     }
     __syncthreads();
     // forward
-    fwd_first(S, A.w.W1, A.P + OFF_B1);
+    fwd_first<NT>(S, A.w.W1, A.P + OFF_B1);
     __syncthreads();
-    fwd_hidden(S.h1, A.w.W2, A.P + OFF_B2, S.h2, S.g2);
+    fwd_hidden<NT>(S.h1, A.w.W2, A.P + OFF_B2, S.h2, S.g2);
     __syncthreads();
-    fwd_hidden(S.h2, A.w.W3, A.P + OFF_B3, S.h3, S.g3);
+    fwd_hidden<NT>(S.h2, A.w.W3, A.P + OFF_B3, S.h3, S.g3);
     __syncthreads();
     fwd_last(S, A.w.W4, A.P + OFF_B4);
     __syncthreads();
     // MSE over the batch and the four outputs: L = sum (y - t)^2 / (4 B)
     const float inv = 1.0f / (4.0f * (float)A.batch);
-    float lsum = 0.f;
-    for (int e = threadIdx.x; e < TILE * OUT; e += THREADS) {
-        const int s = e / OUT, j = e % OUT;
+    static_assert(TILE * OUT == 128 && NT >= 128, "one output per thread, two wavefronts of them");
+    if (threadIdx.x < TILE * OUT) {
+        const int s = threadIdx.x / OUT, j = threadIdx.x % OUT;
         float d = S.valid[s] ? (S.y[s][j] - S.tg[s][j]) : 0.f;
         S.dy[s][j] = 2.0f * d * inv;
-        lsum += d * d * inv;
+        S.red[threadIdx.x] = d * d * inv;
     }
-    S.red[threadIdx.x] = lsum;
     __syncthreads();
-    for (int off = THREADS / 2; off > 0; off >>= 1) {
-        if (threadIdx.x < off) S.red[threadIdx.x] += S.red[threadIdx.x + off];
-        __syncthreads();
+    // the first wavefront sums the loss while the others go on
+    if (threadIdx.x < 64) {
+        float l = S.red[threadIdx.x] + S.red[threadIdx.x + 64];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
+        if (threadIdx.x == 0) A.loss_partial[blockIdx.x] = l;
     }
-    if (threadIdx.x == 0) A.loss_partial[blockIdx.x] = S.red[0];
     // layer 4 gradients and dz3
-    for (int e = threadIdx.x; e < OUT * H; e += THREADS) {
+    for (int e = threadIdx.x; e < OUT * H; e += NT) {
         const int j = e / H, o = e % H;
         float acc = 0.f;
-        for (int s = 0; s < TILE; s++) acc += S.dy[s][j] * bf2f(S.h3[s * H + o]);
+        for (int s = 0; s < TILE; s++) acc += S.dy[s][j] * bf2f(S.h3[s * LD + o]);
         G[OFF_W4 + e] = acc;
     }
     if (threadIdx.x < OUT) {
@@ -269,42 +300,42 @@ __global__ void __launch_bounds__(THREADS) train_tile_kernel(TrainArgs A)
         G[OFF_B4 + threadIdx.x] = acc;
     }
     __syncthreads();   // dW4 has read h3
-    for (int e = threadIdx.x; e < TILE * H; e += THREADS) {
+    for (int e = threadIdx.x; e < TILE * H; e += NT) {
         const int s = e / H, o = e % H;
         float dh = 0.f;
 #pragma unroll
         for (int j = 0; j < OUT; j++) dh += S.dy[s][j] * bf2f(A.w.W4[j * H + o]);
-        S.g3[e] = f2bf(dh * bf2f(S.g3[e]));   // dz3
+        S.g3[s * LD + o] = f2bf(dh * bf2f(S.g3[s * LD + o]));   // dz3
     }
     __syncthreads();
     // layer 3
-    bwd_weight(S.g3, S.h2, G + OFF_W3);
+    bwd_weight<NT>(S.g3, S.h2, G + OFF_W3);
     if (threadIdx.x < H) {
         float acc = 0.f;
-        for (int s = 0; s < TILE; s++) acc += bf2f(S.g3[s * H + threadIdx.x]);
+        for (int s = 0; s < TILE; s++) acc += bf2f(S.g3[s * LD + threadIdx.x]);
         G[OFF_B3 + threadIdx.x] = acc;
     }
-    bwd_data(S.g3, A.w.W3T, S.g2, S.g2);  // dz2 in g2
+    bwd_data<NT>(S.g3, A.w.W3T, S.g2, S.g2);  // dz2 in g2
     __syncthreads();
     // layer 2
-    bwd_weight(S.g2, S.h1, G + OFF_W2);
+    bwd_weight<NT>(S.g2, S.h1, G + OFF_W2);
     if (threadIdx.x < H) {
         float acc = 0.f;
-        for (int s = 0; s < TILE; s++) acc += bf2f(S.g2[s * H + threadIdx.x]);
+        for (int s = 0; s < TILE; s++) acc += bf2f(S.g2[s * LD + threadIdx.x]);
         G[OFF_B2 + threadIdx.x] = acc;
     }
-    bwd_data(S.g2, A.w.W2T, S.g1, S.g1);  // dz1 in g1
+    bwd_data<NT>(S.g2, A.w.W2T, S.g1, S.g1);  // dz1 in g1
     __syncthreads();
     // layer 1 (K = 3)
-    for (int e = threadIdx.x; e < H * IN; e += THREADS) {
+    for (int e = threadIdx.x; e < H * IN; e += NT) {
         const int o = e / IN, k = e % IN;
         float acc = 0.f;
-        for (int s = 0; s < TILE; s++) acc += bf2f(S.g1[s * H + o]) * S.xs[s][k];
+        for (int s = 0; s < TILE; s++) acc += bf2f(S.g1[s * LD + o]) * S.xs[s][k];
         G[OFF_W1 + e] = acc;
     }
     if (threadIdx.x < H) {
         float acc = 0.f;
-        for (int s = 0; s < TILE; s++) acc += bf2f(S.g1[s * H + threadIdx.x]);
+        for (int s = 0; s < TILE; s++) acc += bf2f(S.g1[s * LD + threadIdx.x]);
         G[OFF_B1 + threadIdx.x] = acc;
     }
 }
@@ -404,14 +435,14 @@ __device__ __forceinline__ void split_store(float h, unsigned short* hi, unsigne
 }
 
 // first layer on the FP32 masters, output split
-__device__ void fwd_first_split(Smem& S, const float* W1, const float* b1)
+__device__ void fwd_first_split(Tile& S, const float* W1, const float* b1)
 {
     for (int e = threadIdx.x; e < TILE * H; e += THREADS) {
         const int s = e / H, o = e % H;
         float z = b1[o];
 #pragma unroll
         for (int k = 0; k < IN; k++) z = fmaf(W1[o * IN + k], S.xs[s][k], z);
-        split_store(z * sigmoidf_(z), S.h1, S.g1, e);
+        split_store(z * sigmoidf_(z), S.h1, S.g1, s * LD + o);
     }
 }
 
@@ -427,7 +458,7 @@ __device__ void fwd_hidden_split(const unsigned short* in_hi, const unsigned sho
         const int ts = t / (H / 16), to = t % (H / 16);
         float4v acc = {0.f, 0.f, 0.f, 0.f};
         for (int kk = 0; kk < H; kk += 32) {
-            const int ia = (ts * 16 + r) * H + kk + 8 * q, iw = (to * 16 + r) * H + kk + 8 * q;
+            const int ia = (ts * 16 + r) * LD + kk + 8 * q, iw = (to * 16 + r) * H + kk + 8 * q;
             const bf16x8 ah = __builtin_bit_cast(bf16x8, ld8(in_hi + ia));
             const bf16x8 al = __builtin_bit_cast(bf16x8, ld8(in_lo + ia));
             const bf16x8 wh = __builtin_bit_cast(bf16x8, ld8(W + iw));
@@ -440,7 +471,7 @@ __device__ void fwd_hidden_split(const unsigned short* in_hi, const unsigned sho
         const float bo = b[o];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int e = (ts * 16 + 4 * q + i) * H + o;
+            const int e = (ts * 16 + 4 * q + i) * LD + o;
             const float z = acc[i] + bo;
             split_store(z * sigmoidf_(z), out_hi, out_lo, e);
         }
@@ -448,13 +479,17 @@ __device__ void fwd_hidden_split(const unsigned short* in_hi, const unsigned sho
 }
 
 // last layer on the FP32 masters over the split activations
-__device__ void fwd_last_split(Smem& S, const float* W4, const float* b4)
+__device__ void fwd_last_split(Tile& S, const float* W4, const float* b4)
 {
     for (int e = threadIdx.x; e < TILE * OUT; e += THREADS) {
         const int s = e / OUT, j = e % OUT;
         float z = b4[j];
-        for (int o = 0; o < H; o++)
-            z = fmaf(W4[j * H + o], bf2f(S.h3[s * H + o]) + bf2f(S.g3[s * H + o]), z);
+#pragma unroll 2
+        for (int o = 0; o < H; o += 8) {
+            const us8 hi = ld8(S.h3 + s * LD + o), lo = ld8(S.g3 + s * LD + o);
+#pragma unroll
+            for (int i = 0; i < 8; i++) z = fmaf(W4[j * H + o + i], bf2f(hi[i]) + bf2f(lo[i]), z);
+        }
         S.y[s][j] = z;
     }
 }
@@ -462,7 +497,7 @@ __device__ void fwd_last_split(Smem& S, const float* W4, const float* b4)
 __global__ void __launch_bounds__(THREADS) infer_kernel(InferArgs A)
 {
     extern __shared__ unsigned char smem_raw[];
-    Smem& S = *reinterpret_cast<Smem*>(smem_raw);
+    Tile& S = *reinterpret_cast<Tile*>(smem_raw);
     const int64_t row0 = (int64_t)blockIdx.x * TILE;
     for (int s = threadIdx.x; s < TILE; s += THREADS) {
         int64_t row = row0 + s;
@@ -620,7 +655,7 @@ int step(pnjl_surrogate* s, int64_t batch, int explicit_rows, uint64_t seed, flo
     T.w = s->w;
     T.partial = s->partial;
     T.loss_partial = s->loss_partial;
-    hipLaunchKernelGGL(mlp::train_tile_kernel, dim3(nblocks), dim3(mlp::THREADS), sizeof(mlp::Smem), st, T);
+    hipLaunchKernelGGL(mlp::train_tile_kernel, dim3(nblocks), dim3(mlp::TRAIN_THREADS), sizeof(mlp::Smem), st, T);
     SCHK(s, hipGetLastError());
     mlp::AdamArgs a{};
     a.P = s->P;
@@ -867,7 +902,7 @@ int pnjl_surrogate_infer(pnjl_surrogate* s, int64_t n, const double* T, const do
     a.seeds = dseed;
     SCHK(s, hipEventRecord(s->e0, st));
     hipLaunchKernelGGL(mlp::infer_kernel, dim3((unsigned)((n + mlp::TILE - 1) / mlp::TILE)), dim3(mlp::THREADS),
-                       sizeof(mlp::Smem), st, a);
+                       sizeof(mlp::Tile), st, a);
     SCHK(s, hipGetLastError());
     SCHK(s, hipEventRecord(s->e1, st));
     if (!(flags & PNJL_FLAG_DEVICE_PTRS)) SCHK(s, hipMemcpyAsync(seeds, dseed, n * 40, hipMemcpyDeviceToHost, st));
