@@ -426,6 +426,7 @@ int solve_dev(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const
     A.auto_ms = o->auto_multiseed_fallback;
     A.surr_cap = o->surrogate_max_steps;
     A.judge_mode = o->surrogate_judge;
+    A.head = pnjl::Q_HEAD;
     A.queue = fixed ? (unsigned long long*)(na + kNaQueue) : ctx->queue;
     const pnjl_launch_cfg cfg = choose_cfg(launch, A);
     A.chunk = std::max(1, cfg.chunk);
@@ -504,19 +505,23 @@ int solve_dev(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const
         A.jb = (int32_t*)jb;
         A.j2list = (int32_t*)j2list;
     }
-    // queue words: q[0] the running stage's item counter (cleared before each
-    // stage), q[Q_MCOUNT..Q_J2COUNT] the list lengths, q[kOrderWords..] the
-    // ordering pass's class sizes and cursors
+    // queue words: one item counter per stage from q[Q_HEAD], q[Q_MCOUNT..Q_J2COUNT]
+    // the list lengths, q[kOrderWords..] the ordering pass's class sizes and
+    // cursors; all cleared here, so the stages follow without launches between
     HIPCHK(ctx, hipEventRecord(ctx->ev0, stream));
-    hipLaunchKernelGGL(pnjl::zero_u64, dim3(1), dim3(64), 0, stream, q, kQueueWords);
-    if (A.passes)
-        hipLaunchKernelGGL(pnjl::zero_i32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, A.passes, n);
-    if (A.steps)
-        hipLaunchKernelGGL(pnjl::zero_i32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, A.steps, n);
     // stage-1 order: judged points first, xi = 0 points after the others
-    const dim3 ogrid((unsigned)((n + pnjl::kOrderBlock - 1) / pnjl::kOrderBlock)), oblock(pnjl::kOrderBlock);
-    hipLaunchKernelGGL(pnjl::order_kernel<false>, ogrid, oblock, 0, stream, A, (int32_t*)order, q + kOrderWords);
-    hipLaunchKernelGGL(pnjl::order_kernel<true>, ogrid, oblock, 0, stream, A, (int32_t*)order, q + kOrderWords);
+    if (n <= pnjl::kOrderBlock) {
+        hipLaunchKernelGGL(pnjl::small_setup_kernel, dim3(1), dim3((unsigned)((n + 63) / 64 * 64)), 0, stream, A,
+                           (int32_t*)order, q, kQueueWords);
+    } else {
+        hipLaunchKernelGGL(pnjl::zero_u64, dim3(1), dim3(64), 0, stream, q, kQueueWords);
+        const dim3 all((unsigned)((n + 255) / 256));
+        if (A.passes) hipLaunchKernelGGL(pnjl::zero_i32, all, dim3(256), 0, stream, A.passes, n);
+        if (A.steps) hipLaunchKernelGGL(pnjl::zero_i32, all, dim3(256), 0, stream, A.steps, n);
+        const dim3 ogrid((unsigned)((n + pnjl::kOrderBlock - 1) / pnjl::kOrderBlock)), oblock(pnjl::kOrderBlock);
+        hipLaunchKernelGGL(pnjl::order_kernel<false>, ogrid, oblock, 0, stream, A, (int32_t*)order, q + kOrderWords);
+        hipLaunchKernelGGL(pnjl::order_kernel<true>, ogrid, oblock, 0, stream, A, (int32_t*)order, q + kOrderWords);
+    }
     A.order = (const int32_t*)order;
     HIPCHK(ctx, hipGetLastError());
     // stage 1: every point (or every (point, seed) of the multi-seed plans)
@@ -524,10 +529,11 @@ int solve_dev(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const
     S.kind = surr ? pnjl::K_SURR : (multi ? pnjl::K_MPOL : (mr3 ? pnjl::K_MR3 : pnjl::K_PRIMARY));
     launch_scan(ctx, S, G, blocks, stream);
     HIPCHK(ctx, hipGetLastError());
-    // the later stages run on the persistent grid
+    // the later stages (at most three) run on the persistent grid
+    int stage = pnjl::Q_HEAD;
     auto next_stage = [&](int kind, int mult, int k_base, const void* list, int count_word) -> int {
-        hipLaunchKernelGGL(pnjl::zero_u64, dim3(1), dim3(64), 0, stream, q + pnjl::Q_HEAD, 1);
         pnjl::ScanArgs L = A;
+        L.head = ++stage;
         L.kind = kind;
         L.mult = mult;
         L.k_base = k_base;

@@ -180,7 +180,11 @@ def run_dual_branch_scan_batch(T_mev, mu_values, xi=0.0, p_num=24, t_num=8, opts
     if solver is not None:
         had, qrk = _follow_both(solver, T, xi, mu_fm)
     else:
-        had, qrk = _follow_chains(chain_solver or gpu_chain_solver(device, p_num, t_num, opts), T, xi, mu_fm)
+        # the time is the longest chain's: 64 lanes per chain while the chip holds
+        # them (45 lines x 111 mu, six grids: about 6.5 us per solver step, 9 at 32)
+        lanes = 64 if T.size <= 2048 else 32
+        solve = chain_solver or gpu_chain_solver(device, p_num, t_num, opts, lanes_per_point=lanes)
+        had, qrk = _follow_chains(solve, T, xi, mu_fm)
     # _select_physical_branch  DualBranchScan.jl:378-398
     both = had["valid"] & qrk["valid"]
     same = both & _same_solution(had, qrk)

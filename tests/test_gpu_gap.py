@@ -331,6 +331,23 @@ def test_default_geometry_picks_lanes(gpu_ctx, policy, n, chain):
     assert np.all(np.abs(a["x"] - b["x"]).max(axis=1) <= bound)
 
 
+@pytest.mark.parametrize("m", [1, 63, 64, 65, 1023, 1024])
+def test_small_call_setup(gpu_ctx, m):
+    """Calls of up to 1024 points order and clear in one launch: each point's
+    result and counts are those of the same point in a larger call."""
+    r = np.random.default_rng(5)
+    n = 1100
+    T, mu, xi = r.uniform(30, 290, n) / HB, r.uniform(0, 440, n) / HB, r.choice([0.0, 0.3, -0.2], n)
+    try:
+        gpu_ctx.set_launch_cfg(16, 1, 8, 16)
+        a = gpu_ctx.solve_batch(T, mu, xi, policy=0, p_num=16, t_num=4)
+        b = gpu_ctx.solve_batch(T[:m], mu[:m], xi[:m], policy=0, p_num=16, t_num=4)
+    finally:
+        gpu_ctx.set_launch_cfg()
+    for k in a:
+        assert np.array_equal(a[k][:m], b[k], equal_nan=True), k
+
+
 @pytest.mark.parametrize("lpp", [32, 64])
 @pytest.mark.parametrize("pn,tn,xi", [(64, 4, 0.0), (65, 3, 0.0), (1, 1, 0.3), (1, 64, 0.3), (12, 6, -0.2), (31, 2, 0.4),
                                       (64, 1, 0.2), (64, 64, 0.1), (7, 9, 0.0)])
