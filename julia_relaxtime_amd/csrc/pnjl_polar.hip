@@ -1370,27 +1370,23 @@ __device__ __forceinline__ void mass_group(const Phys& P, const pnjl_mass_query&
     constexpr int kSub = G == 1 ? 1 : G / 4;   // lanes per B0
     const double h0 = fd_step(x[0]), h1 = fd_step(x[1]);
     if constexpr (G == 1) {
-        MassB0 Bx;
-        double s[2];
-#pragma unroll 1
-        for (int w = 0; w < 5; w++) {
-            const double k0 = w == 1 ? x[0] + h0 : (w == 2 ? x[0] - h0 : x[0]);
-            const double ga = w == 3 ? x[1] + h1 : (w == 4 ? x[1] - h1 : x[1]);
-            MassB0 B = Bx;
-            if (w < 3) mass_b0<1>(P, a, k0, B);
-            if (w == 0) Bx = B;
-            double g[2];
-            mass_residual(P, a, k, B, k0, ga, g);
-            for (int i = 0; i < 2; i++) {
-                if (w == 0) f[i] = g[i];
-                else if (w == 1 || w == 3) s[i] = g[i];
-                else if (w == 2) J[i][0] = (s[i] - g[i]) / (2.0 * h0);
-                else J[i][1] = (s[i] - g[i]) / (2.0 * h1);
-            }
+        MassB0 Bx{}, Bp{}, Bm{};
+        mass_b0<1>(P, a, x[0], Bx);
+        mass_b0<1>(P, a, x[0] + h0, Bp);
+        mass_b0<1>(P, a, x[0] - h0, Bm);
+        double fp[2], fm[2], gp[2], gm[2];
+        mass_residual(P, a, k, Bx, x[0], x[1], f);
+        mass_residual(P, a, k, Bp, x[0] + h0, x[1], fp);
+        mass_residual(P, a, k, Bm, x[0] - h0, x[1], fm);
+        mass_residual(P, a, k, Bx, x[0], x[1] + h1, gp);
+        mass_residual(P, a, k, Bx, x[0], x[1] - h1, gm);
+        for (int i = 0; i < 2; i++) {
+            J[i][0] = (fp[i] - fm[i]) / (2.0 * h0);
+            J[i][1] = (gp[i] - gm[i]) / (2.0 * h1);
         }
     } else {
         const int gl = (int)(threadIdx.x % G), sub = gl / kSub, w = gl & 7;
-        MassB0 B;
+        MassB0 B{};
         mass_b0<kSub>(P, a, sub == 1 ? x[0] + h0 : (sub == 2 ? x[0] - h0 : x[0]), B);
         const int from = w == 1 ? kSub : (w == 2 ? 2 * kSub : 0);
         for (int j = 0; j < 2; j++) {

@@ -281,3 +281,20 @@ def test_meson_masses_match_oracle(gpu_ctx, oracle, P, M):
     assert r["converged"] == o["converged"] and abs(r["mass"] - o["mass"]) <= 1e-7
     with pytest.raises(ValueError):
         P.solve_meson_mass("rho", qp, tp)
+
+
+def test_pole_search_does_not_depend_on_the_lane_split(P, M):
+    """A search's result is the same bits on 64 and 16 lanes (small and large
+    batches) and on one (the one-query-per-wavefront launch)."""
+    r = np.random.default_rng(8)
+    n = 400
+    m_u, m_s = r.uniform(0.05, 1.9, n), r.uniform(1.0, 2.8, n)
+    mu = r.uniform(0.0, 2.0, n)
+    q = P.make_mass_queries(np.arange(n) % 8, r.uniform(0.2, 1.4, n), r.uniform(0.0, 0.9, n), r.uniform(0.0, 0.9, n), 0.0,
+                            m_u, m_s, mu, mu, r.uniform(-1.5, -0.2, n), r.uniform(-1.5, -0.2, n))
+    a = P.meson_mass_batch(q)
+    b = P.meson_mass_batch(q, one_per_wave=True)
+    c = P.meson_mass_batch(np.resize(q, 131073))
+    for k in a:
+        assert np.array_equal(a[k], b[k], equal_nan=True), k
+        assert np.array_equal(a[k], c[k][:n], equal_nan=True), k
