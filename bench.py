@@ -147,9 +147,9 @@ C3_METRIC = "anisotropic one-loop polarization values/s (12,582,912-value Pi gri
 # counted once: rocprofv3 FP64 VALU counters (FMA = 2) on 131,072 seeded cells
 # of the same grid evaluated one per wavefront, so that inactive lanes of
 # divergent waves are not counted (python3 bench.py --flop-probe pi):
-# 86,571 per cell (one symmetrised B0 + correction and one Pi), two Pi values
+# 31,406 per cell (one symmetrised B0 + correction and one Pi), two Pi values
 # per cell.  The A kernel (512 values) is negligible.
-C3_FLOPS_PER_VALUE = 43286.0
+C3_FLOPS_PER_VALUE = 15703.0
 
 
 def c3_points(ctx, opts):
@@ -279,11 +279,11 @@ def train_learned_seed(ctx, w, opts):
 PROP_METRIC = "meson propagator (D_S, D_P) queries/s (calculate_propagator_by_channel, 1,048,576-query batch)"
 # FP64 FLOPs per query of this batch, counted once like C3_FLOPS_PER_VALUE:
 # FP64 VALU counters on 65,536 of its queries run one (pair, query) per
-# wavefront (python3 bench.py --flop-probe prop): 119,772 per
+# wavefront (python3 bench.py --flop-probe prop): 43,474 per
 # query (1.68 quark pairs of B0 + correction per query on average).  The
 # bucketing and composition kernels (~10^2 operations per query) are not
 # counted; their time is.
-PROP_FLOPS_PER_QUERY = 119772.0
+PROP_FLOPS_PER_QUERY = 43474.0
 
 
 def prop_cpu_baseline(q, G, K, threads=None):
@@ -358,11 +358,11 @@ def run_propagators(args, w):
 MASS_METRIC = "meson pole masses solved/s (solve_meson_mass, 8 mesons x 65,536 (T, mu) points)"
 # FP64 FLOPs per pole-mass query of this batch, counted once on 8,192 seeded
 # queries run one per wavefront (python3 bench.py --flop-probe mass), summed
-# over the phase launches: 822,180 per query (38.7 trust-region iterations on
+# over the phase launches: 1,052,503 per query (38.7 trust-region iterations on
 # average; 36 % of the queries stop at the start on a non-finite residual).
 # The kernel's time is set by its longest serial chains (queries running the
 # full 1000 iterations), not by FP64 throughput.
-MASS_FLOPS_PER_QUERY = 822180.0
+MASS_FLOPS_PER_QUERY = 1052503.0
 
 
 def _mass_worker(args):
