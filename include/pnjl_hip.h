@@ -307,7 +307,10 @@ int pnjl_set_judge_mask(pnjl_ctx* ctx, int nT, int nmu, int nxi, const double* l
 /* Launch geometry of the persistent scan kernel; chosen per config by the
  * autotuner (pnjl_autotune) or set explicitly.  A context whose geometry is
  * the default {4, 4, 8, 0} leaves it to the library: each solve picks lanes
- * per point by its number of points (more lanes for fewer points).         */
+ * per point by its number of points (more lanes for fewer points), all of
+ * which add the node sums in the order of 4 lanes.  A point's results are
+ * then those of 4 lanes, bit for bit, whatever the size of its call; other
+ * geometries add in other orders (equal to rounding).                      */
 typedef struct pnjl_launch_cfg {
     int lanes_per_point;  /* 1,2,4,8,16,32,64 -> 64/lanes points per wavefront */
     int chunk;            /* points taken from the work queue per pop        */

@@ -222,8 +222,14 @@ __device__ __forceinline__ bool nodes_all_fast(double Phi, double Phib, double m
     return Phi >= -0.1 && Phib >= -0.1 && fabs(muT) <= kFastExpMax;
 }
 
-// One node of one flavour: adds C-weighted raw terms to `s` (scaled to the
-// FlavSums definitions by flav_finish).
+// Raw terms of one node of one flavour (scaled to the FlavSums definitions by
+// flav_finish): a sum of S, Sfp, Sfm, SP, SPb, SPP, SPPb, SPbPb and Sfab adds
+// C times its term, one of A1, B1 and B2 CinvE times it, A2 CinvE2 times it.
+struct NodeTerms {
+    double S, Sfp, Sfm, SP, SPb, SPP, SPPb, SPbPb, Sfab, A1, B1, B2, A2;
+    double CinvE, CinvE2;
+};
+
 // The fast path works with the unscaled arguments D = 1 + 3 c1 t + 3 c2 t^2 +
 // t^3, t = e^a (resp. e^b), for either sign of the exponents: ln F is the same
 // function as the reference's shifted form 3a + ln(e^-3a + ...) for a > 0,
@@ -236,8 +242,8 @@ __device__ __forceinline__ bool nodes_all_fast(double Phi, double Phib, double m
 // the caller has established nodes_all_fast.
 // q = p^2 (1 + xi cos^2), M2 = M^2, muT = mu/T, invT = 1/T, K2mu = exp(-2 mu/T).
 template <bool kChecked>
-__device__ __forceinline__ void node_accumulate(const double* tab, double q, double C, double M2, double muT,
-                                                double invT, double K2mu, double Phi, double Phib, FlavSums& s)
+__device__ __forceinline__ void node_terms(const double* tab, double q, double C, double M2, double muT,
+                                           double invT, double K2mu, double Phi, double Phib, NodeTerms& n)
 {
     NODE_MATH_EXACT
     double E, invE;
@@ -298,20 +304,44 @@ __device__ __forceinline__ void node_accumulate(const double* tab, double q, dou
         fp = sp.f;
         fm = sm.f;
     }
-    const double CinvE = C * invE;
-    s.S = fma(C, Q, s.S);
-    s.A1 = fma(CinvE, gs, s.A1);
-    s.A2 = fma(CinvE * invE, fma(hs, invT, gs * invE), s.A2);
-    s.B1 = fma(CinvE, k1p + k2m, s.B1);
-    s.B2 = fma(CinvE, k2p + k1m, s.B2);
-    s.SP = fma(C, r1p + r2m, s.SP);
-    s.SPb = fma(C, r2p + r1m, s.SPb);
-    s.SPP = fma(C, fma(r1p, r1p, r2m * r2m), s.SPP);
-    s.SPPb = fma(C, fma(r1p, r2p, r1m * r2m), s.SPPb);
-    s.SPbPb = fma(C, fma(r2p, r2p, r1m * r1m), s.SPbPb);
-    s.Sfp = fma(C, fp, s.Sfp);
-    s.Sfm = fma(C, fm, s.Sfm);
-    s.Sfab = fma(C, fma(fp, a, fm * b), s.Sfab);
+    n.CinvE = C * invE;
+    n.CinvE2 = n.CinvE * invE;
+    n.S = Q;
+    n.A1 = gs;
+    n.A2 = fma(hs, invT, gs * invE);
+    n.B1 = k1p + k2m;
+    n.B2 = k2p + k1m;
+    n.SP = r1p + r2m;
+    n.SPb = r2p + r1m;
+    n.SPP = fma(r1p, r1p, r2m * r2m);
+    n.SPPb = fma(r1p, r2p, r1m * r2m);
+    n.SPbPb = fma(r2p, r2p, r1m * r1m);
+    n.Sfp = fp;
+    n.Sfm = fm;
+    n.Sfab = fma(fp, a, fm * b);
+}
+
+// adds the C-weighted raw terms of one node of one flavour to `s`
+template <bool kChecked>
+__device__ __forceinline__ void node_accumulate(const double* tab, double q, double C, double M2, double muT,
+                                                double invT, double K2mu, double Phi, double Phib, FlavSums& s)
+{
+    NODE_MATH_EXACT
+    NodeTerms n;
+    node_terms<kChecked>(tab, q, C, M2, muT, invT, K2mu, Phi, Phib, n);
+    s.S = fma(C, n.S, s.S);
+    s.A1 = fma(n.CinvE, n.A1, s.A1);
+    s.A2 = fma(n.CinvE2, n.A2, s.A2);
+    s.B1 = fma(n.CinvE, n.B1, s.B1);
+    s.B2 = fma(n.CinvE, n.B2, s.B2);
+    s.SP = fma(C, n.SP, s.SP);
+    s.SPb = fma(C, n.SPb, s.SPb);
+    s.SPP = fma(C, n.SPP, s.SPP);
+    s.SPPb = fma(C, n.SPPb, s.SPPb);
+    s.SPbPb = fma(C, n.SPbPb, s.SPbPb);
+    s.Sfp = fma(C, n.Sfp, s.Sfp);
+    s.Sfm = fma(C, n.Sfm, s.Sfm);
+    s.Sfab = fma(C, n.Sfab, s.Sfab);
 }
 
 // Scales the raw node sums to the FlavSums definitions: the derivative

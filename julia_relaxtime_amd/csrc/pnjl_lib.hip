@@ -206,62 +206,73 @@ bool valid_lpp(int l) { return l == 1 || l == 2 || l == 4 || l == 8 || l == 16 |
 // within the block's budget lds_block (80 KB on a 160 KB-LDS CU); a lane
 // count whose groups do not fit next to a large table is raised to the next
 // power of two (a different summation order, equal to rounding).
+// four: the library's own geometry (8 or 64 lanes), whose groups add in the
+// order of four lanes; those of 64 have LDS rows besides their state (12 KB a
+// wavefront, less than the 4-lane groups' states, so they fit wherever those do).
 struct ScanGeom {
     int lpp, threads, groups_per_block;
     size_t lds;
+    bool four;
 };
 
-ScanGeom scan_geom(int lpp, int pn, int tn, size_t lds_block)
+ScanGeom scan_geom(int lpp, int pn, int tn, size_t lds_block, bool four)
 {
-    const size_t tab = (size_t)pnjl::table_len(pn, tn) * sizeof(double);
-    const size_t group = (size_t)pnjl::STATE_STRIDE * sizeof(double);
+    const size_t rows = four && lpp == 64 ? pnjl::Four<64>::kGroup : 0;
+    const size_t tab = (size_t)(pnjl::table_len(pn, tn) + (rows ? 1 : 0)) * sizeof(double);
+    const size_t group = (pnjl::STATE_STRIDE + rows) * sizeof(double);
     // the block's LDS budget, less its copy of the launch arguments (static LDS)
     const size_t limit = lds_block - (sizeof(pnjl::ScanArgs) + 255) / 256 * 256;
-    for (int l = lpp; l <= 64; l *= 2) {
+    for (int l = lpp; l <= (four ? lpp : 64); l *= 2) {
         for (int waves = 4; waves >= 1; waves--) {
             const int threads = 64 * waves;
             const int gpb = threads / l;
             if (gpb > 64) continue;
             const size_t lds = tab + (size_t)gpb * group;
-            if (lds <= limit) return ScanGeom{l, threads, gpb, lds};
+            if (lds <= limit) return ScanGeom{l, threads, gpb, lds, four};
         }
     }
-    return ScanGeom{64, 64, 1, tab + group};
+    if (four) return ScanGeom{lpp, 64, 64 / lpp, tab + (64 / lpp) * group, true};
+    return ScanGeom{64, 64, 1, tab + group, false};
 }
 
 // Launch geometry of a call whose context holds the default one (kDefaultCfg):
-// lanes per point by the amount of work.  A point's solve is a serial run of
-// node passes, so while its call does not fill the chip the time is that of
-// its longest solves, and more lanes per point shorten every pass; once the
-// chip is full, 8 lanes are the most efficient (below 8, the groups' LDS state
-// leaves room for one wavefront per SIMD only).  The chip holds 2^17 lanes at
-// two wavefronts per SIMD; most solves end early, so the best lane count is
-// the largest with points x lanes <= 2^19.  Measured (p 64, t 4, DefaultSeed
-// at xi != 0, max_iter 40, ms at 8 / 16 / 32 / 64 lanes): 1024 points 3.8 /
-// 2.5 / 1.9 / 1.6, 8192 points 4.4 / 3.6 / 2.9 / 2.7, 32768 points 6.9 / 6.2 /
-// 6.0 / 6.3, 131072 points 22.4 / 22.7 / 23.1 / 24.9 (fixed 4 lanes: 34, 37,
-// 38, 56).  MultiSeed's six candidates per point run long: items x lanes <=
-// 2^20 (32768 points at 8 / 16 / 32 lanes: 16.7 / 17.2 / 19.3 ms, 2048 points
-// 5.0 / 3.5 / 2.3).  The later stages hold few, long items (the listed points'
-// MultiSeed candidates): points x lanes <= 2^20, at least 16 (p 64, t 4,
-// xi != 0, stage-2 lanes 16 / 64: 16384 points 7.0 / 5.6 ms, 131072 points
-// 22.4 / 23.0).  A chain is serial over its points: 64 lanes up to 2048 chains
-// (16 points x 24 x 8 nodes, 256 chains: 14.2 ms at 8, 5.7 at 32, 4.3 at 64),
-// then 32 (12 x 6 nodes, 4096 chains: 5.7 ms at 64, 5.3 at 32).
-pnjl_launch_cfg choose_cfg(const pnjl_launch_cfg& c, const pnjl::ScanArgs& A)
+// the library's own, by the amount of work.  Its 8- and 64-lane groups add the
+// node sums in the order of four lanes (Four), so the choice moves no bit: a
+// point's result is that of the geometry {4, 4, 8, 0} and does not depend on
+// how many points share its call.  A point's solve is a serial run of node
+// passes, so while a call does not fill the chip its time is that of its
+// longest solves, and 64 lanes shorten every pass; once the chip is full, 8
+// lanes waste least (below 8 the groups' LDS state leaves room for one
+// wavefront per SIMD only).  The lines lie where 64 and 8 lanes cost about the
+// same over four meshes (p 64 t 4 at xi = 0.2 / p 64 at 0 / p 12 t 6 at 0.2 / p
+// 24 at 0; ms at 64 | 8 lanes, the later stages on 64, against 37 / 13 / 14 / 8
+// of {4, 4, 8, 0}):
+//   DefaultSeed, max_iter 40, 4096 points 2.6 / 1.7 / 1.8 / 1.7 | 3.6 / 1.9 / 2.0 /
+//   1.6, 8192 points 3.8 / 2.3 / 2.7 / 2.2 | 4.0 / 2.0 / 2.1 / 1.6;
+//   its later stages (few, long items) on 64 | 8 lanes, 32768 points 7.9 / 4.2 /
+//   4.0 / 3.4 | 9.4 / 4.2 / 3.9 / 2.8, 131072 points 23 / 13 / 12 / 11 | 22 / 10 / 10 / 7;
+//   MultiSeed (six long items per point), 1400 points 2.3 / 1.4 / 1.6 / 1.4 | 4.6 /
+//   1.7 / 1.9 / 1.2, 2800 points 3.7 / 2.2 / 2.6 / 2.2 | 4.8 / 1.8 / 2.0 / 1.3;
+//   chains of 10 points (serial over their points; p 24 t 8 at 0.2 / p 12 t 6 at
+//   0.2 / p 12 at 0), 8192 chains 9.8 / 6.3 / 6.1 | 18 / 8.1 / 5.8, 16384 chains 12.4
+//   / 9.7 / 7.8 | 20 / 9.9 / 6.0, 65536 chains 36 / 26 / 22 | 30 / 15 / 9.
+// A node table that leaves no room for 4-lane groups: the geometry as it is
+// (scan_geom raises its lanes by the table alone).
+struct Launch {
+    pnjl_launch_cfg cfg;
+    bool four;
+};
+
+Launch choose_launch(const pnjl_launch_cfg& c, const pnjl::ScanArgs& A, size_t lds_block)
 {
     if (c.lanes_per_point != kDefaultCfg.lanes_per_point || c.chunk != kDefaultCfg.chunk ||
         c.waves_per_cu != kDefaultCfg.waves_per_cu || c.tail_lanes_per_point != kDefaultCfg.tail_lanes_per_point)
-        return c;
-    auto lanes = [](int64_t items, int64_t total, int least) {
-        int l = 64;
-        while (l > least && items > total / l) l /= 2;
-        return l;
-    };
-    if (A.plan == pnjl::PLAN_CHAINS) return pnjl_launch_cfg{A.n_items <= 2048 ? 64 : 32, 1, 8, 0};
-    const bool many = A.plan == pnjl::PLAN_MULTI;
-    const int l = lanes(A.n_points * A.mult, many ? 1 << 20 : 1 << 19, 8);
-    return pnjl_launch_cfg{l, 1, l > 8 ? 8 : 16, std::max(l, lanes(A.n_points, 1 << 20, 16))};
+        return Launch{c, false};
+    if (scan_geom(c.lanes_per_point, A.pn, A.tn, lds_block, false).lpp != c.lanes_per_point) return Launch{c, false};
+    const int64_t line = A.plan == pnjl::PLAN_CHAINS ? 16384 : (A.plan == pnjl::PLAN_MULTI ? 2048 : 4096);
+    const int64_t items = A.plan == pnjl::PLAN_CHAINS ? A.n_items : A.n_points;
+    if (items <= line) return Launch{pnjl_launch_cfg{64, 1, 8, 0}, true};
+    return Launch{pnjl_launch_cfg{8, 1, 16, A.n_points <= 32768 ? 64 : 8}, true};
 }
 
 // Lets every scan_kernel instantiation take `bytes` of dynamic LDS.
@@ -269,13 +280,14 @@ bool allow_scan_lds(int bytes)
 {
     using namespace pnjl;
     const hipFuncAttribute a = hipFuncAttributeMaxDynamicSharedMemorySize;
-    return hipFuncSetAttribute((const void*)scan_kernel<1>, a, bytes) == hipSuccess &&
-           hipFuncSetAttribute((const void*)scan_kernel<2>, a, bytes) == hipSuccess &&
-           hipFuncSetAttribute((const void*)scan_kernel<4>, a, bytes) == hipSuccess &&
-           hipFuncSetAttribute((const void*)scan_kernel<8>, a, bytes) == hipSuccess &&
-           hipFuncSetAttribute((const void*)scan_kernel<16>, a, bytes) == hipSuccess &&
-           hipFuncSetAttribute((const void*)scan_kernel<32>, a, bytes) == hipSuccess &&
-           hipFuncSetAttribute((const void*)scan_kernel<64>, a, bytes) == hipSuccess;
+    bool ok = true;
+    for (const void* k : {(const void*)scan_kernel<1, false>, (const void*)scan_kernel<2, false>,
+                          (const void*)scan_kernel<4, false>, (const void*)scan_kernel<8, false>,
+                          (const void*)scan_kernel<16, false>, (const void*)scan_kernel<32, false>,
+                          (const void*)scan_kernel<64, false>, (const void*)scan_kernel<8, true>,
+                          (const void*)scan_kernel<64, true>})
+        ok = ok && hipFuncSetAttribute(k, a, bytes) == hipSuccess;
+    return ok;
 }
 
 void launch_scan(pnjl_ctx* ctx, const pnjl::ScanArgs& A, const ScanGeom& G, int blocks, hipStream_t st)
@@ -284,14 +296,20 @@ void launch_scan(pnjl_ctx* ctx, const pnjl::ScanArgs& A, const ScanGeom& G, int 
     const int k = ctx->n_scans < kMaxTimedScans ? ctx->n_scans++ : -1;
     if (k >= 0) (void)hipEventRecord(ctx->ev_scan[2 * k], st);
     const dim3 grid(blocks), block(G.threads);
-    switch (G.lpp) {
-    case 1: hipLaunchKernelGGL(scan_kernel<1>, grid, block, G.lds, st, A); break;
-    case 2: hipLaunchKernelGGL(scan_kernel<2>, grid, block, G.lds, st, A); break;
-    case 4: hipLaunchKernelGGL(scan_kernel<4>, grid, block, G.lds, st, A); break;
-    case 8: hipLaunchKernelGGL(scan_kernel<8>, grid, block, G.lds, st, A); break;
-    case 16: hipLaunchKernelGGL(scan_kernel<16>, grid, block, G.lds, st, A); break;
-    case 32: hipLaunchKernelGGL(scan_kernel<32>, grid, block, G.lds, st, A); break;
-    default: hipLaunchKernelGGL(scan_kernel<64>, grid, block, G.lds, st, A); break;
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, G.lds, st, A); };
+    if (G.four) {
+        if (G.lpp == 8) launch(scan_kernel<8, true>);
+        else launch(scan_kernel<64, true>);
+    } else {
+        switch (G.lpp) {
+        case 1: launch(scan_kernel<1, false>); break;
+        case 2: launch(scan_kernel<2, false>); break;
+        case 4: launch(scan_kernel<4, false>); break;
+        case 8: launch(scan_kernel<8, false>); break;
+        case 16: launch(scan_kernel<16, false>); break;
+        case 32: launch(scan_kernel<32, false>); break;
+        default: launch(scan_kernel<64, false>); break;
+        }
     }
     if (k >= 0) (void)hipEventRecord(ctx->ev_scan[2 * k + 1], st);
 }
@@ -428,12 +446,13 @@ int solve_dev(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const
     A.judge_mode = o->surrogate_judge;
     A.head = pnjl::Q_HEAD;
     A.queue = fixed ? (unsigned long long*)(na + kNaQueue) : ctx->queue;
-    const pnjl_launch_cfg cfg = choose_cfg(launch, A);
+    const Launch chosen = choose_launch(launch, A, ctx->lds_block);
+    const pnjl_launch_cfg& cfg = chosen.cfg;
     A.chunk = std::max(1, cfg.chunk);
     A.bnd = ctx->bnd;
     A.nb = ctx->nb;
     A.max_trips = 9LL * (2LL * o->max_iter + 4) + 16;
-    const ScanGeom G = scan_geom(cfg.lanes_per_point, pn, tn, ctx->lds_block);
+    const ScanGeom G = scan_geom(cfg.lanes_per_point, pn, tn, ctx->lds_block, chosen.four);
     const int waves_per_block = G.threads / 64;
     int blocks = std::max(1, ctx->num_cu * std::max(1, cfg.waves_per_cu) / waves_per_block);
     // never more groups than work items: a small batch gets a small grid
@@ -444,7 +463,7 @@ int solve_dev(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const
     // the later pipeline stages (few, long items) run the full persistent grid
     // at their own lanes per point
     const ScanGeom G2 = scan_geom(cfg.tail_lanes_per_point > 0 ? cfg.tail_lanes_per_point : G.lpp, pn, tn,
-                                  ctx->lds_block);
+                                  ctx->lds_block, chosen.four);
     const int fullblocks = std::max(1, ctx->num_cu * std::max(1, cfg.waves_per_cu) / (G2.threads / 64));
     unsigned long long* q = A.queue;
     if (chains) {

@@ -222,7 +222,7 @@ enum TrField { TR_R = 0, TR_J = 5, TR_D = 20, TR_P = 25, TR_DELTA = 30 };
 __shared__ ScanArgs cold_args;
 
 // The kernels' dynamic LDS: node tables, then the groups' storage.
-extern __shared__ double scan_lds[];
+extern __shared__ __align__(16) double scan_lds[];
 
 // The group's solver state.  It lives in the group's LDS block (every lane
 // of the group reads and writes the same values), which keeps it out of the
@@ -530,11 +530,157 @@ __device__ __forceinline__ void flavours_wide(const double* lds, int pn, int tn,
     reduce_store<LPP, 13 * NF>(v, s, SB_SUMS + 13 * f, gl);
 }
 
-// Node pass at state x: u, s, and d unless M_d == M_u (then d aliases u);
-// the reduced sums go to the group's LDS state.  div: see node_div.
+// ---- the pass of the library's own geometry ---------------------------------
+// Where the library picks the lanes per point (by the size of the call), the
+// sums must not depend on the pick: a point, alone, in a chunk or in a whole
+// scan, is the same numbers.  So its 8- and 64-lane groups add in the order of
+// four lanes: chain v (0..3) adds the nodes j = v, v + 4, ... of each angle node
+// in turn, and a sum is (chain 0 + chain 1) + (chain 2 + chain 3).  Half of a
+// group's lanes take the u flavour, half s (both d, where it differs from u).
+// 8 lanes are then the 4-lane loop on each half.  With 64, a half evaluates
+// kNodes nodes of every chain at once, its lanes leave the terms in LDS rows,
+// and each lane adds some of one chain's terms, in order: bound, like all of a
+// small call, by the latency of dependent FP64 instructions and of LDS.  A
+// solve of 1024 points (p 64 t 4, max_iter 40) takes 1.91 ms at xi = 0.2 and
+// 1.20 at 0 (free order, flavours_wide: 1.52 and 1.14; 4 lanes: 36 and 13); of
+// 262144 points, on 8 lanes, 40.3 and 18.2 (8 lanes in free order: 39.6 and
+// 19.8; 4 lanes: 87 and 32).
 template <int LPP>
+struct Four {
+    static constexpr int kHalf = LPP / 2;                           // lanes per flavour
+    static constexpr int kNodes = LPP >= 8 ? kHalf / 4 : 1;         // nodes of a chain per round
+    static constexpr int kOwn = (13 + kNodes - 1) / kNodes;         // terms of a chain that a lane adds
+    // doubles from a chain's nodes to the next chain's in a row: 16-byte loads,
+    // eight neighbouring lanes of which lie in different banks
+    static constexpr int kPitch = kNodes + 2;
+    static constexpr int kRow = 4 * kPitch;
+    static constexpr int kHalfRows = 16 * kRow;                     // 13 terms, C, CinvE, CinvE2
+    static constexpr int kGroup = kNodes > 1 ? 2 * kHalfRows : 0;   // doubles per group
+};
+// rows: S Sfp Sfm SP SPb SPP SPPb SPbPb Sfab (times C), A1 B1 B2 (CinvE), A2 (CinvE2)
+constexpr int kRowC = 13, kRowCinvE = 14, kRowCinvE2 = 15;
+__device__ __forceinline__ int row_field(int c) { return (int)(0x2651C98743BA0ULL >> (4 * c)) & 15; }   // SumField
+__device__ __forceinline__ int row_factor(int c) { return c < 9 ? kRowC : (c < 12 ? kRowCinvE : kRowCinvE2); }
+
+// LDS accesses of a wavefront complete in order; this keeps the compiler to it
+__device__ __forceinline__ void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// This lane's chain sums of one flavour: acc[i] of row i kNodes + sl, chain v.
+// A lane evaluates two nodes of a chain at a time (two independent sequences of
+// dependent instructions), without branches: past the chain's end, node 0
+// again, into a slot that nobody adds.
+template <int LPP, bool kChecked>
+__device__ __forceinline__ void four_loop(const double* lds, int pn, int tn, double M2, double muT, double invT,
+                                          double K2mu, double xi, double Phi, double Phib, int gl, double* rows,
+                                          double* acc)
+{
+    using G = Four<LPP>;
+    constexpr int S = G::kNodes, NB = 2;
+    const double* pp = lds + kMathTab;
+    const double* cc = pp + pn;
+    const bool iso = xi == 0.0;
+    const double* Cm = pp + pn + tn + (iso ? pn * tn : 0);
+    const int h = gl & (G::kHalf - 1), v = h & 3, sl = h >> 2;
+    const int nl = iso ? 1 : tn, nv = (pn - v + 3) >> 2;   // angle nodes, chain v's momentum nodes
+    const int total = nl * nv, longest = nl * ((pn + 3) >> 2);
+    double* const mine = rows + v * G::kPitch;
+#pragma unroll
+    for (int i = 0; i < G::kOwn; i++) acc[i] = 0.0;
+    int l = 0, q = sl;   // angle node l and momentum node j = 4 q + v of this lane's next node
+#pragma unroll 1
+    for (int r = 0; r < longest; r += NB * S) {
+        NodeTerms n[NB];
+        double C[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++, q += S) {
+            const bool in = r + b * S + sl < total;
+            while (in && q >= nv) {
+                q -= nv;
+                l++;
+            }
+            const int lb = in ? l : 0, j = in ? 4 * q + v : 0;
+            C[b] = Cm[lb * pn + j];
+            const double p2 = pp[j];
+            node_terms<kChecked>(lds, iso ? p2 : fma(xi * cc[lb], p2, p2), C[b], M2, muT, invT, K2mu, Phi, Phib, n[b]);
+        }
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            if (r + b * S >= longest) break;
+            const double t[16] = {n[b].S,   n[b].Sfp,   n[b].Sfm,  n[b].SP, n[b].SPb, n[b].SPP, n[b].SPPb, n[b].SPbPb,
+                                  n[b].Sfab, n[b].A1, n[b].B1, n[b].B2, n[b].A2, C[b], n[b].CinvE, n[b].CinvE2};
+#pragma unroll
+            for (int c = 0; c < 16; c++) mine[c * G::kRow + sl] = t[c];
+            wave_fence();
+            const int m = total - r - b * S;   // nodes in this lane's chain's slots
+            const bool full = __all(m >= S);
+#pragma unroll
+            for (int i = 0; i < G::kOwn; i++) {
+                const int c = i * S + sl;
+                if (c >= 13) continue;
+                const double* x = mine + c * G::kRow;
+                const double* f = mine + row_factor(c) * G::kRow;
+                if (full) {
+#pragma unroll
+                    for (int k = 0; k < S; k += 2) {
+                        const double2 a = *reinterpret_cast<const double2*>(x + k);
+                        const double2 w = *reinterpret_cast<const double2*>(f + k);
+                        acc[i] = fma(w.x, a.x, acc[i]);
+                        acc[i] = fma(w.y, a.y, acc[i]);
+                    }
+                } else {
+#pragma unroll 1
+                    for (int k = 0; k < S && k < m; k++) acc[i] = fma(f[k], x[k], acc[i]);
+                }
+            }
+            wave_fence();   // the rows are written again only after every lane has read them
+        }
+    }
+}
+
+// Sums of the flavour of mass M to its slot f of the group's state
+template <int LPP>
+__device__ __forceinline__ void flavour_four(const double* lds, int pn, int tn, double M, double invT, double muT,
+                                             double K2mu, double xi, double Phi, double Phib, int gl, const Scr& s, int f,
+                                             double* rows)
+{
+    using G = Four<LPP>;
+    if constexpr (G::kNodes == 1) {
+        FlavSums acc;
+        flavour_sums<4>(lds, pn, tn, M, invT, muT, K2mu, xi, Phi, Phib, gl & 3, acc);
+        store_flav(s, f, acc);
+    } else {
+        const double M2 = M * M;
+        double acc[G::kOwn];
+        if (__any(!nodes_all_fast(Phi, Phib, muT)))
+            four_loop<LPP, true>(lds, pn, tn, M2, muT, invT, K2mu, xi, Phi, Phib, gl, rows, acc);
+        else
+            four_loop<LPP, false>(lds, pn, tn, M2, muT, invT, K2mu, xi, Phi, Phib, gl, rows, acc);
+        const int sl = (gl & (G::kHalf - 1)) >> 2;
+        const double t3 = 3.0 * invT;
+#pragma unroll
+        for (int i = 0; i < G::kOwn; i++) {
+            const int c = i * G::kNodes + sl;
+            // flav_finish's factor of the row
+            const double k = c < 3 || c == 8 ? 1.0 : (c < 5 ? 3.0 : (c < 8 ? -9.0 : (c < 12 ? -t3 : t3)));
+            const double a = group_sum<4>(acc[i]) * k;
+            if (i * G::kNodes + G::kNodes <= 13 || c < 13) s.at(SB_SUMS + 13 * f + row_field(c)) = a;
+        }
+    }
+    wave_fence();   // the other half reads them
+}
+
+// Node pass at state x: u, s, and d unless M_d == M_u (then d aliases u);
+// the reduced sums go to the group's LDS state.  div: see node_div; rows: the
+// group's LDS rows (kFour).
+template <int LPP, bool kFour = false>
 __device__ __forceinline__ void node_pass(const DevParams& P, const double* lds, int pn, int tn, unsigned div, const Scr& s,
-                                          const double* x, double T, double mu, double xi, bool sym, int gl)
+                                          const double* x, double T, double mu, double xi, bool sym, int gl,
+                                          double* rows = nullptr)
 {
     double M[3];
     mass_vec(P, x, M);
@@ -542,7 +688,14 @@ __device__ __forceinline__ void node_pass(const DevParams& P, const double* lds,
     const double invT = 1.0 / T;
     const double muT = mu * invT;
     const double K2mu = exp(-2.0 * muT);
-    if constexpr (LPP >= 32) {
+    if constexpr (kFour) {
+        const int half = gl / Four<LPP>::kHalf;
+        double* const mine = rows + half * Four<LPP>::kHalfRows;
+#pragma unroll 1
+        for (int f = 0; f < (sym ? 1 : 2); f++)
+            flavour_four<LPP>(lds, pn, tn, f ? M[1] : (half ? M[2] : M[0]), invT, muT, K2mu, xi, x[3], x[4], gl, s,
+                              f ? 2 : half, mine);
+    } else if constexpr (LPP >= 32) {
         const double Mus[2] = {M[0], M[2]};
         flavours_wide<LPP, 2>(lds, pn, tn, div, Mus, invT, muT, K2mu, xi, x[3], x[4], gl, s, 0);
         if (!sym) flavours_wide<LPP, 1>(lds, pn, tn, div, M + 1, invT, muT, K2mu, xi, x[3], x[4], gl, s, 2);
@@ -1771,7 +1924,8 @@ __host__ __device__ inline int table_len(int pn, int tn) { return kMathTab + pn 
 // trust-region step) is out of line and reads the block's LDS copy of the
 // arguments, and no local array's address reaches a call, so the loop's
 // state stays in registers and LDS.
-template <int LPP>
+// kFour: the library's own geometry (Four).
+template <int LPP, bool kFour>
 __global__ void __launch_bounds__(256, 2) scan_kernel(ScanArgs A)
 {
     double* const lds = scan_lds;
@@ -1784,6 +1938,9 @@ __global__ void __launch_bounds__(256, 2) scan_kernel(ScanArgs A)
     const Scr s{(int)(tab_len + (threadIdx.x / LPP) * STATE_STRIDE)};
     const bool chains = (A.plan == PLAN_CHAINS);
     const unsigned div = node_div(A.pn);
+    // the groups' rows follow their states (16-byte aligned)
+    const int states = tab_len + (int)(blockDim.x / LPP) * STATE_STRIDE;
+    double* const rows = lds + (states + 1) / 2 * 2 + (int)(threadIdx.x / LPP) * Four<LPP>::kGroup;
     St& st = s.st();
     st.phase = PH_IDLE;
     st.item = 0;
@@ -1814,7 +1971,7 @@ __global__ void __launch_bounds__(256, 2) scan_kernel(ScanArgs A)
             double x[5];
 #pragma unroll
             for (int i = 0; i < 5; i++) x[i] = st.x[i];
-            node_pass<LPP>(A.P, lds, A.pn, A.tn, div, s, x, st.T, st.mu, st.xi, st.sym, gl);
+            node_pass<LPP, kFour>(A.P, lds, A.pn, A.tn, div, s, x, st.T, st.mu, st.xi, st.sym, gl, rows);
             st.passes += st.sym ? 2 : 3;
         }
         control_step<LPP>(A, s, st, gl);

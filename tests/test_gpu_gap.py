@@ -331,6 +331,39 @@ def test_default_geometry_picks_lanes(gpu_ctx, policy, n, chain):
     assert np.all(np.abs(a["x"] - b["x"]).max(axis=1) <= bound)
 
 
+@pytest.mark.parametrize("policy,n,chain,pn,tn", [(0, 36000, 0, 16, 4), (3, 4100, 0, 16, 4), (5, 16390 * 2, 2, 12, 3),
+                                                  (4, 4200, 0, 7, 3), (0, 4200, 0, 65, 2), (4, 300, 0, 3, 5),
+                                                  (3, 60, 0, 1, 1), (0, 40, 0, 64, 64), (0, 9, 0, 4096, 1)])
+def test_default_results_do_not_depend_on_the_call(policy, n, chain, pn, tn):
+    """At the default geometry a point's results are the same bits alone, in a
+    chunk and in a whole scan (sizes on both sides of every line between lane
+    counts, the transition band among the points), and those of 4 lanes: the
+    library's own groups add in the order of 4 lanes, whatever the mesh."""
+    from julia_relaxtime_amd import _lib
+    r = np.random.default_rng(n)
+    T, mu, xi = r.uniform(20, 290, n) / HB, r.uniform(0, 440, n) / HB, r.choice([0.0, 0.3, -0.2], n)
+    kw = {}
+    if chain:
+        T, mu, xi = (np.sort(T.reshape(-1, chain), 1).ravel(), np.repeat(mu[::chain], chain), np.repeat(xi[::chain], chain))
+    if policy == 4:
+        seed = np.stack([r.uniform(-1.8, -0.1, n), r.uniform(-1.8, -0.1, n), r.uniform(-2.2, -0.4, n),
+                         r.uniform(-0.3, 0.9, n), r.uniform(0.01, 0.9, n)], 1)
+        seed[::2, 1] = seed[::2, 0]     # phi_u = phi_d: two flavours, else three
+        kw["seed"] = seed
+    opts = _lib.default_opts(max_iter=40, chain_len=chain)
+    ctx = _lib.Context(0)
+    f = lambda m: ctx.solve_batch(T[:m], mu[:m], xi[:m], policy=policy, p_num=pn, t_num=tn, opts=opts,  # noqa: E731
+                                  **{k: v[:m] for k, v in kw.items()})
+    # chain lines: 16384 chains; MultiSeed 2048 points; the rest 4096 and 32768
+    cuts = [m for m in (1, 63, 2048, 2049, 4096, 4097, 32768, 32770) if m < n and m % max(chain, 1) == 0] + [n]
+    own = {m: f(m) for m in cuts}
+    ctx.set_launch_cfg(4, 1, 8, 0)
+    four = f(n)
+    for m, a in own.items():
+        for k in a:
+            assert np.array_equal(a[k], four[k][:m], equal_nan=True), (m, k)
+
+
 @pytest.mark.parametrize("m", [1, 63, 64, 65, 1023, 1024])
 def test_small_call_setup(gpu_ctx, m):
     """Calls of up to 1024 points order and clear in one launch: each point's
