@@ -547,12 +547,8 @@ def run_tmu(args, w):
     stats = dict(ms=0.0, passes=0.0, launches=0)
 
     def solve(T, mu, xi, seeds):
-        saved = ctx.launch_cfg()
-        ctx.set_launch_cfg(lanes_per_point=32, chunk=1, waves_per_cu=8, tail_lanes_per_point=32)
-        try:
+        with ctx.launch(lanes_per_point=32, chunk=1, waves_per_cu=8, tail_lanes_per_point=32):
             r = ctx.solve_batch(T, mu, xi, policy=_lib.SEED_EXPLICIT, seed=seeds, p_num=24, t_num=8, opts=opts)
-        finally:
-            ctx.set_launch_cfg(**saved)
         stats["ms"] += ctx.last_kernel_ms()
         stats["passes"] += float(np.sum(r["passes"])) * 24.0
         stats["launches"] += 1
@@ -679,11 +675,9 @@ def root_agreement(ctx, w, opts, T, mu, xi, Td, mud, xid, Q, P, cfg, plain_polic
     more than 1e-9 (next to the critical end point the Hessian is nearly
     singular)."""
     from julia_relaxtime_amd.surrogate import same_root
-    saved = ctx.launch_cfg()
-    ctx.set_launch_cfg(**cfg)
-    P2 = {k: v.cpu().numpy() for k, v in ctx.solve_batch(Td, mud, xid, policy=plain_policy, p_num=w["p_num"],
-                                                          t_num=w["t_num"], opts=opts).items()}
-    ctx.set_launch_cfg(**saved)
+    with ctx.launch(**cfg):
+        P2 = {k: v.cpu().numpy() for k, v in ctx.solve_batch(Td, mud, xid, policy=plain_policy, p_num=w["p_num"],
+                                                              t_num=w["t_num"], opts=opts).items()}
     same = same_root(Q, P)
     off = np.flatnonzero(~same)
     unstable = ~same_root({k: P2[k][off] for k in ("x", "masses", "omega")},

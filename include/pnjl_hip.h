@@ -304,13 +304,13 @@ int pnjl_set_phase_boundary(pnjl_ctx* ctx, int nrows, const double* xi, const do
 int pnjl_set_judge_mask(pnjl_ctx* ctx, int nT, int nmu, int nxi, const double* lo3, const double* hi3,
                         const uint8_t* mask);
 
-/* Launch geometry of the persistent scan kernel; chosen per config by the
- * autotuner (pnjl_autotune) or set explicitly.  A context whose geometry is
- * the default {4, 4, 8, 0} leaves it to the library: each solve picks lanes
- * per point by its number of points (more lanes for fewer points), all of
- * which add the node sums in the order of 4 lanes.  A point's results are
- * then those of 4 lanes, bit for bit, whatever the size of its call; other
- * geometries add in other orders (equal to rounding).                      */
+/* Launch geometry of the persistent scan kernel.  A new context leaves it to
+ * the library: each solve picks lanes per point by its number of points (more
+ * lanes for fewer points), all of which add the node sums in the order of 4
+ * lanes, so that a point's results are those of {4, 4, 8, 0}, bit for bit,
+ * whatever the size of its call.  Once a geometry was set (pnjl_set_launch_cfg)
+ * or tuned (pnjl_autotune), every solve runs that one; lanes other than 4 add
+ * in other orders (equal to rounding).                                     */
 typedef struct pnjl_launch_cfg {
     int lanes_per_point;  /* 1,2,4,8,16,32,64 -> 64/lanes points per wavefront */
     int chunk;            /* points taken from the work queue per pop        */
@@ -322,7 +322,12 @@ typedef struct pnjl_launch_cfg {
 } pnjl_launch_cfg;
 
 int pnjl_set_launch_cfg(pnjl_ctx* ctx, const pnjl_launch_cfg* cfg);
+/* the geometry that was set or tuned, {4, 4, 8, 0} where none was          */
 int pnjl_get_launch_cfg(const pnjl_ctx* ctx, pnjl_launch_cfg* cfg);
+/* The geometry is the library's again, as in a new context; and whether it
+ * is (1 or 0): save it with the geometry to restore both.                  */
+int pnjl_set_launch_auto(pnjl_ctx* ctx);
+int pnjl_get_launch_auto(const pnjl_ctx* ctx);
 
 /* Autotuner: times launch geometries on the first `sample` points of the
  * batch (host pointers as in pnjl_solve_fixedmu_batch; each candidate warmed

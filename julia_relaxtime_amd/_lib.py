@@ -5,6 +5,7 @@ Loading fails loudly when it is missing: there is no CPU fallback.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import os
 
@@ -136,6 +137,8 @@ def load():
     L.pnjl_set_judge_mask.argtypes = [vp, C.c_int, C.c_int, C.c_int, _DP, _DP, C.POINTER(C.c_uint8)]
     L.pnjl_set_launch_cfg.argtypes = [vp, C.POINTER(LaunchCfg)]
     L.pnjl_get_launch_cfg.argtypes = [vp, C.POINTER(LaunchCfg)]
+    L.pnjl_set_launch_auto.argtypes = [vp]
+    L.pnjl_get_launch_auto.argtypes = [vp]
     L.pnjl_solve_fixedmu_batch.argtypes = [vp, C.c_int64, vp, vp, vp, vp, C.c_int, C.c_int, C.c_int,
                                            C.POINTER(SolveOpts), C.POINTER(SolveOut), C.c_int, vp]
     L.pnjl_solve_fixedmu_batch_noalloc.argtypes = L.pnjl_solve_fixedmu_batch.argtypes
@@ -146,7 +149,8 @@ def load():
     L.pnjl_autotune.argtypes = [vp, C.c_int64, _DP, _DP, _DP, _DP, C.c_int, C.c_int, C.c_int,
                                 C.POINTER(SolveOpts), C.POINTER(LaunchCfg), C.POINTER(C.c_double)]
     for name in ("pnjl_ctx_create", "pnjl_gauleg", "pnjl_nodes", "pnjl_set_phase_boundary", "pnjl_set_judge_mask",
-                 "pnjl_set_launch_cfg", "pnjl_get_launch_cfg", "pnjl_solve_fixedmu_batch",
+                 "pnjl_set_launch_cfg", "pnjl_get_launch_cfg", "pnjl_set_launch_auto", "pnjl_get_launch_auto",
+                 "pnjl_solve_fixedmu_batch",
                  "pnjl_solve_fixedmu_batch_noalloc",
                  "pnjl_gap_residual_batch", "pnjl_thermo_derivatives_batch", "pnjl_implicit_derivatives2_batch",
                  "pnjl_autotune"):
@@ -261,6 +265,27 @@ class Context:
         cfg = LaunchCfg()
         self._check(self._L.pnjl_get_launch_cfg(self.h, C.byref(cfg)), "pnjl_get_launch_cfg")
         return cfg.as_dict()
+
+    def set_launch_auto(self):
+        """Leaves the launch geometry to the library again, as in a new context."""
+        self._check(self._L.pnjl_set_launch_auto(self.h), "pnjl_set_launch_auto")
+
+    def launch_auto(self):
+        """Whether the library chooses the launch geometry (none was set or tuned)."""
+        return bool(self._L.pnjl_get_launch_auto(self.h))
+
+    @contextlib.contextmanager
+    def launch(self, **cfg):
+        """The launch geometry `cfg` (set_launch_cfg) inside a with block."""
+        saved, auto = self.launch_cfg(), self.launch_auto()
+        self.set_launch_cfg(**cfg)
+        try:
+            yield
+        finally:
+            if auto:
+                self.set_launch_auto()
+            else:
+                self.set_launch_cfg(**saved)
 
     def last_kernel_ms(self):
         return self._L.pnjl_last_kernel_ms(self.h)

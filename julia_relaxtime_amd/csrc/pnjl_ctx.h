@@ -18,8 +18,9 @@ constexpr int kOrderWords = 8;
 // persistent-kernel launches timed per solve
 constexpr int kMaxTimedScans = 8;
 
-// the launch geometry of a new context; a call that finds it unchanged picks
-// its own by the amount of work (choose_cfg)
+// the launch geometry whose results a context gives until one is set or tuned;
+// its calls pick their own, with the same results, by the amount of work
+// (choose_launch)
 constexpr pnjl_launch_cfg kDefaultCfg{4, 4, 8, 0};
 
 struct pnjl_ctx {
@@ -29,6 +30,7 @@ struct pnjl_ctx {
     pnjl::DevParams dp{};
     std::string err;
     pnjl_launch_cfg cfg = kDefaultCfg;
+    bool auto_launch = true;            // no geometry was set or tuned
     std::map<std::pair<int, int>, double*> tabs;
     size_t lds_block = 64 * 1024;       // LDS budget of one scan-kernel block (bytes)
     unsigned long long* queue = nullptr;

@@ -235,8 +235,7 @@ ScanGeom scan_geom(int lpp, int pn, int tn, size_t lds_block, bool four)
     return ScanGeom{64, 64, 1, tab + group, false};
 }
 
-// Launch geometry of a call whose context holds the default one (kDefaultCfg):
-// the library's own, by the amount of work.  Its 8- and 64-lane groups add the
+// The library's own launch geometry, by the amount of work.  Its 8- and 64-lane groups add the
 // node sums in the order of four lanes (Four), so the choice moves no bit: a
 // point's result is that of the geometry {4, 4, 8, 0} and does not depend on
 // how many points share its call.  A point's solve is a serial run of node
@@ -256,19 +255,17 @@ ScanGeom scan_geom(int lpp, int pn, int tn, size_t lds_block, bool four)
 //   chains of 10 points (serial over their points; p 24 t 8 at 0.2 / p 12 t 6 at
 //   0.2 / p 12 at 0), 8192 chains 9.8 / 6.3 / 6.1 | 18 / 8.1 / 5.8, 16384 chains 12.4
 //   / 9.7 / 7.8 | 20 / 9.9 / 6.0, 65536 chains 36 / 26 / 22 | 30 / 15 / 9.
-// A node table that leaves no room for 4-lane groups: the geometry as it is
+// A node table that leaves no room for 4-lane groups: kDefaultCfg itself
 // (scan_geom raises its lanes by the table alone).
 struct Launch {
     pnjl_launch_cfg cfg;
     bool four;
 };
 
-Launch choose_launch(const pnjl_launch_cfg& c, const pnjl::ScanArgs& A, size_t lds_block)
+Launch choose_launch(const pnjl::ScanArgs& A, size_t lds_block)
 {
-    if (c.lanes_per_point != kDefaultCfg.lanes_per_point || c.chunk != kDefaultCfg.chunk ||
-        c.waves_per_cu != kDefaultCfg.waves_per_cu || c.tail_lanes_per_point != kDefaultCfg.tail_lanes_per_point)
-        return Launch{c, false};
-    if (scan_geom(c.lanes_per_point, A.pn, A.tn, lds_block, false).lpp != c.lanes_per_point) return Launch{c, false};
+    const int four = kDefaultCfg.lanes_per_point;
+    if (scan_geom(four, A.pn, A.tn, lds_block, false).lpp != four) return Launch{kDefaultCfg, false};
     const int64_t line = A.plan == pnjl::PLAN_CHAINS ? 16384 : (A.plan == pnjl::PLAN_MULTI ? 2048 : 4096);
     const int64_t items = A.plan == pnjl::PLAN_CHAINS ? A.n_items : A.n_points;
     if (items <= line) return Launch{pnjl_launch_cfg{64, 1, 8, 0}, true};
@@ -391,10 +388,10 @@ int check_policy(int p)
 // table, queue words, the items' candidate records and the per-point lists
 // live in the device's no-alloc scratch (n <= kNaPoints) instead of buffers
 // the context allocates; the launch, and with it every point's result, is the
-// same either way.
+// same either way.  launch: the geometry, null for the library's own.
 int solve_dev(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const double* xi, const double* seed,
               int policy, int pn, int tn, const pnjl_solve_opts* o, const pnjl_solve_out* out,
-              const pnjl_launch_cfg& launch, hipStream_t stream, bool fixed = false)
+              const pnjl_launch_cfg* launch, hipStream_t stream, bool fixed = false)
 {
     double* tab = nullptr;
     int rc = fixed ? na_table(ctx, pn, tn, stream, &tab) : get_tab(ctx, pn, tn, &tab);
@@ -446,7 +443,7 @@ int solve_dev(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const
     A.judge_mode = o->surrogate_judge;
     A.head = pnjl::Q_HEAD;
     A.queue = fixed ? (unsigned long long*)(na + kNaQueue) : ctx->queue;
-    const Launch chosen = choose_launch(launch, A, ctx->lds_block);
+    const Launch chosen = launch ? Launch{*launch, false} : choose_launch(A, ctx->lds_block);
     const pnjl_launch_cfg& cfg = chosen.cfg;
     A.chunk = std::max(1, cfg.chunk);
     A.bnd = ctx->bnd;
@@ -827,8 +824,19 @@ int pnjl_set_launch_cfg(pnjl_ctx* ctx, const pnjl_launch_cfg* cfg)
         cfg->waves_per_cu > 64)
         return set_err(ctx, PNJL_ERR_ARG, "pnjl_set_launch_cfg: invalid geometry");
     ctx->cfg = *cfg;
+    ctx->auto_launch = false;
     return PNJL_OK;
 }
+
+int pnjl_set_launch_auto(pnjl_ctx* ctx)
+{
+    if (!ctx) return PNJL_ERR_ARG;
+    ctx->cfg = kDefaultCfg;
+    ctx->auto_launch = true;
+    return PNJL_OK;
+}
+
+int pnjl_get_launch_auto(const pnjl_ctx* ctx) { return ctx && ctx->auto_launch ? 1 : 0; }
 
 int pnjl_get_launch_cfg(const pnjl_ctx* ctx, pnjl_launch_cfg* cfg)
 {
@@ -839,7 +847,7 @@ int pnjl_get_launch_cfg(const pnjl_ctx* ctx, pnjl_launch_cfg* cfg)
 
 static int solve_impl(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const double* xi,
                       const double* seed, int policy, int pn, int tn, const pnjl_solve_opts* opts,
-                      const pnjl_solve_out* out, int flags, void* stream, const pnjl_launch_cfg& cfg,
+                      const pnjl_solve_out* out, int flags, void* stream, const pnjl_launch_cfg* cfg,
                       bool fixed = false)
 {
     if (!ctx) return PNJL_ERR_ARG;
@@ -946,7 +954,8 @@ int pnjl_solve_fixedmu_batch(pnjl_ctx* ctx, int64_t n, const double* T, const do
                              const pnjl_solve_out* out, int flags, void* stream)
 {
     if (!ctx) return PNJL_ERR_ARG;
-    return solve_impl(ctx, n, T, mu, xi, seed, seed_policy, p_num, t_num, opts, out, flags, stream, ctx->cfg);
+    return solve_impl(ctx, n, T, mu, xi, seed, seed_policy, p_num, t_num, opts, out, flags, stream,
+                      ctx->auto_launch ? nullptr : &ctx->cfg);
 }
 
 int pnjl_solve_fixedmu_batch_noalloc(pnjl_ctx* ctx, int64_t n, const double* T, const double* mu, const double* xi,
@@ -965,8 +974,8 @@ int pnjl_solve_fixedmu_batch_noalloc(pnjl_ctx* ctx, int64_t n, const double* T, 
                                               " points per call");
     if (ctx->device < 0 || ctx->device >= kNaMaxDevices || !g_na[ctx->device].base)
         return set_err(ctx, PNJL_ERR_STATE, "pnjl_solve_fixedmu_batch_noalloc: no scratch on this device");
-    return solve_impl(ctx, n, T, mu, xi, seed, seed_policy, p_num, t_num, opts, out, flags, stream, ctx->cfg,
-                      true);
+    return solve_impl(ctx, n, T, mu, xi, seed, seed_policy, p_num, t_num, opts, out, flags, stream,
+                      ctx->auto_launch ? nullptr : &ctx->cfg, true);
 }
 
 int pnjl_gap_residual_batch(pnjl_ctx* ctx, int64_t n, const double* x, const double* T, const double* mu,
@@ -1063,7 +1072,7 @@ int pnjl_autotune(pnjl_ctx* ctx, int64_t sample, const double* T, const double* 
         // around the pipeline)
         double t = 1e300;
         for (int rep = 0; rep < 3; rep++) {
-            int rc = solve_impl(ctx, sample, T, mu, xi, seed, policy, pn, tn, opts, &out, 0, nullptr, cfg);
+            int rc = solve_impl(ctx, sample, T, mu, xi, seed, policy, pn, tn, opts, &out, 0, nullptr, &cfg);
             if (rc) return rc;
             if (rep > 0) t = std::min(t, ctx->last_ms);
         }
@@ -1097,6 +1106,7 @@ int pnjl_autotune(pnjl_ctx* ctx, int64_t sample, const double* T, const double* 
         if (t != b2.lanes_per_point)
             if (int rc = trial(pnjl_launch_cfg{b2.lanes_per_point, b2.chunk, b2.waves_per_cu, t}, nullptr)) return rc;
     ctx->cfg = bcfg;
+    ctx->auto_launch = false;
     if (best) *best = bcfg;
     if (ns_per_point) *ns_per_point = bms * 1e6 / (double)sample;
     return PNJL_OK;

@@ -44,13 +44,8 @@ def gpu_solver(device=0, p_num=24, t_num=8, opts=None, lanes_per_point=32):
     o = opts or _lib.default_opts()
 
     def solve(T, mu, xi, policy, seed):
-        saved = ctx.launch_cfg()
-        ctx.set_launch_cfg(lanes_per_point=lanes_per_point, chunk=1, waves_per_cu=8,
-                           tail_lanes_per_point=lanes_per_point)
-        try:
+        with ctx.launch(lanes_per_point=lanes_per_point, chunk=1, waves_per_cu=8, tail_lanes_per_point=lanes_per_point):
             return ctx.solve_batch(T, mu, xi, policy=policy, seed=seed, p_num=p_num, t_num=t_num, opts=o)
-        finally:
-            ctx.set_launch_cfg(**saved)
     return solve
 
 
@@ -69,13 +64,8 @@ def gpu_chain_solver(device=0, p_num=24, t_num=8, opts=None, lanes_per_point=32)
         for f, _ in _lib.SolveOpts._fields_:
             setattr(o, f, getattr(base, f))
         o.chain_len = int(chain_len)
-        saved = ctx.launch_cfg()
-        ctx.set_launch_cfg(lanes_per_point=lanes_per_point, chunk=1, waves_per_cu=8,
-                           tail_lanes_per_point=lanes_per_point)
-        try:
+        with ctx.launch(lanes_per_point=lanes_per_point, chunk=1, waves_per_cu=8, tail_lanes_per_point=lanes_per_point):
             return ctx.solve_batch(T, mu, xi, policy=policy, p_num=p_num, t_num=t_num, opts=o)
-        finally:
-            ctx.set_launch_cfg(**saved)
     return solve
 
 

@@ -480,6 +480,11 @@ set_launch_cfg!(cfg::LaunchCfg, ctx::Context=default_context()) =
     check(ctx, ccall((:pnjl_set_launch_cfg, LIB), Cint, (Ptr{Cvoid}, Ref{LaunchCfg}), ctx.h, cfg),
           "pnjl_set_launch_cfg")
 
+# whether the library chooses the geometry (none was set or tuned); and left to it again
+launch_auto(ctx::Context=default_context()) = ccall((:pnjl_get_launch_auto, LIB), Cint, (Ptr{Cvoid},), ctx.h) != 0
+set_launch_auto!(ctx::Context=default_context()) =
+    check(ctx, ccall((:pnjl_set_launch_auto, LIB), Cint, (Ptr{Cvoid},), ctx.h), "pnjl_set_launch_auto")
+
 mutable struct Surrogate
     h::Ptr{Cvoid}
     in_lo::Vector{Float64}
@@ -662,7 +667,7 @@ context's GPU).
 function learned_seed(ctx::Context=default_context(); device::Integer=0, p_num::Integer=64, t_num::Integer=4,
                       iterations::Integer=40, ftol::Real=1e-10, n_train::Integer=200_000, schedule=LR_SCHEDULE,
                       batch::Integer=8192, n_probe::Integer=1_000_000, rng=Random.Xoshiro(4))
-    saved = launch_cfg(ctx)
+    saved, auto = launch_cfg(ctx), launch_auto(ctx)
     set_launch_cfg!(SETUP_LAUNCH, ctx)
     try
         T, mu, xi = training_points(n_train, rng)
@@ -679,7 +684,7 @@ function learned_seed(ctx::Context=default_context(); device::Integer=0, p_num::
                           iterations=iterations, ftol=ftol)
         return s
     finally
-        set_launch_cfg!(saved, ctx)
+        auto ? set_launch_auto!(ctx) : set_launch_cfg!(saved, ctx)
     end
 end
 

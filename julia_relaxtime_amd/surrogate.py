@@ -330,9 +330,7 @@ def learned_seed(ctx, p_num=64, t_num=4, opts=None, n_train=200_000, schedule=LR
     import threading
     import time
     t0 = time.perf_counter()
-    saved = ctx.launch_cfg()
-    ctx.set_launch_cfg(**SETUP_LAUNCH)
-    try:
+    with ctx.launch(**SETUP_LAUNCH):
         T, mu, xi = training_points(n_train, seed=4)
         tr = ctx.solve_batch(T, mu, xi, policy=_lib.SEED_DEFAULT, p_num=p_num, t_num=t_num, opts=opts)
         ok = tr["converged"] == 1
@@ -361,8 +359,6 @@ def learned_seed(ctx, p_num=64, t_num=4, opts=None, n_train=200_000, schedule=LR
         t2 = time.perf_counter()
         s.build_judge_mask(ctx, probes["T"], probes["mu"], probes["xi"], p_num=p_num, t_num=t_num, opts=opts,
                            multi_max_iter=multi_max_iter)
-    finally:
-        ctx.set_launch_cfg(**saved)
     info = dict(train_points=int(ok.sum()), adam_steps=int(sum(n for n, _ in schedule)), batch=batch,
                 lr=[list(ph) for ph in schedule], train_kernel_ms=train_ms,
                 final_loss=float(np.mean(loss[-200:])), judge_probes=n_train + n_probe,

@@ -27,6 +27,13 @@ def gpu_ctx():
     return pnjl.context(0)
 
 
+@pytest.fixture(autouse=True)
+def library_geometry(request):
+    """Every GPU test starts at the launch geometry of a new context."""
+    if "gpu_ctx" in request.fixturenames:
+        request.getfixturevalue("gpu_ctx").set_launch_auto()
+
+
 def golden_rows(name):
     import csv
     with open(os.path.join(GOLDEN, name)) as f:

@@ -319,12 +319,10 @@ def test_default_geometry_picks_lanes(gpu_ctx, policy, n, chain):
         T, mu, xi = (np.sort(T.reshape(-1, chain), 1).ravel(), np.repeat(mu[::chain], chain), np.repeat(xi[::chain], chain))
     opts = _lib.default_opts(ftol=1e-10, xtol=1e-14, max_iter=40, chain_len=chain)
     assert gpu_ctx.launch_cfg() == dict(lanes_per_point=4, chunk=4, waves_per_cu=8, tail_lanes_per_point=0)
+    assert gpu_ctx.launch_auto()
     a = gpu_ctx.solve_batch(T, mu, xi, policy=policy, p_num=16, t_num=4, opts=opts)
-    try:
-        gpu_ctx.set_launch_cfg(4, 1, 8, 0)
+    with gpu_ctx.launch(lanes_per_point=4, chunk=1):
         b = gpu_ctx.solve_batch(T, mu, xi, policy=policy, p_num=16, t_num=4, opts=opts)
-    finally:
-        gpu_ctx.set_launch_cfg()
     assert a["converged"].all() and b["converged"].all()
     J = gpu_ctx.residual_batch(b["x"], T, mu, xi, 16, 4)[1]
     bound = 2e-10 * np.abs(np.linalg.inv(J)).sum(axis=2).max(axis=1) + 1e-13
@@ -364,6 +362,41 @@ def test_default_results_do_not_depend_on_the_call(policy, n, chain, pn, tn):
             assert np.array_equal(a[k], four[k][:m], equal_nan=True), (m, k)
 
 
+def test_set_geometry_is_the_one_that_runs():
+    """A geometry that was set or tuned runs as it is, {4, 4, 8, 0} too (512 points
+    on 4 lanes take ten times the library's own choice: asserted at three),
+    and the library's choice comes back with set_launch_auto and after a
+    launch() block; the tuner times what it names and keeps it."""
+    from julia_relaxtime_amd import _lib
+    r = np.random.default_rng(2)
+    n = 512
+    T, mu = r.uniform(190, 290, n) / HB, r.uniform(5, 390, n) / HB
+    xi = np.full(n, 0.3)
+    opts = _lib.default_opts(max_iter=40)
+    ctx = _lib.Context(0)
+    four = dict(lanes_per_point=4, chunk=4, waves_per_cu=8, tail_lanes_per_point=0)
+
+    def ms():
+        t = []
+        for _ in range(3):
+            ctx.solve_batch(T, mu, xi, policy=0, p_num=64, t_num=4, opts=opts)
+            t.append(ctx.last_kernel_ms())
+        return min(t)
+    own = ms()
+    assert ctx.launch_auto() and ctx.launch_cfg() == four
+    ctx.set_launch_cfg()
+    assert not ctx.launch_auto() and ctx.launch_cfg() == four and ms() > 3 * own
+    ctx.set_launch_auto()
+    with ctx.launch(**four):
+        assert not ctx.launch_auto() and ms() > 3 * own
+    assert ctx.launch_auto() and ms() < 2 * own
+    best, _ = ctx.autotune(T, mu, xi, policy=0, p_num=64, t_num=4, opts=opts)
+    assert not ctx.launch_auto() and ctx.launch_cfg() == best
+    with ctx.launch(**four):
+        pass
+    assert not ctx.launch_auto() and ctx.launch_cfg() == best
+
+
 @pytest.mark.parametrize("m", [1, 63, 64, 65, 1023, 1024])
 def test_small_call_setup(gpu_ctx, m):
     """Calls of up to 1024 points order and clear in one launch: each point's
@@ -371,12 +404,9 @@ def test_small_call_setup(gpu_ctx, m):
     r = np.random.default_rng(5)
     n = 1100
     T, mu, xi = r.uniform(30, 290, n) / HB, r.uniform(0, 440, n) / HB, r.choice([0.0, 0.3, -0.2], n)
-    try:
-        gpu_ctx.set_launch_cfg(16, 1, 8, 16)
+    with gpu_ctx.launch(lanes_per_point=16, chunk=1, tail_lanes_per_point=16):
         a = gpu_ctx.solve_batch(T, mu, xi, policy=0, p_num=16, t_num=4)
         b = gpu_ctx.solve_batch(T[:m], mu[:m], xi[:m], policy=0, p_num=16, t_num=4)
-    finally:
-        gpu_ctx.set_launch_cfg()
     for k in a:
         assert np.array_equal(a[k][:m], b[k], equal_nan=True), k
 
@@ -400,12 +430,9 @@ def test_wide_group_node_pass(gpu_ctx, lpp, pn, tn, xi):
     seed[::2, 1] = seed[::2, 0]     # phi_u = phi_d: two flavours, else three
     opts = _lib.default_opts(max_iter=0, trust_region_fallback=0, auto_multiseed_fallback=0)
     out = []
-    try:
-        for l in (4, lpp):
-            gpu_ctx.set_launch_cfg(l, 1, 8, 0)
+    for l in (4, lpp):
+        with gpu_ctx.launch(lanes_per_point=l, chunk=1):
             out.append(gpu_ctx.solve_batch(T, mu, xi, policy=4, seed=seed, p_num=pn, t_num=tn, opts=opts))
-    finally:
-        gpu_ctx.set_launch_cfg()
     for k in ("omega", "rho_norm", "entropy", "energy", "n_q", "n_qbar", "residual_norm", "x"):
         a, b = out[0][k], out[1][k]
         assert np.all(np.abs(a - b) <= 1e-13 * (1e3 + np.abs(a))), k
