@@ -170,10 +170,13 @@ def run_dual_branch_scan_batch(T_mev, mu_values, xi=0.0, p_num=24, t_num=8, opts
     if solver is not None:
         had, qrk = _follow_both(solver, T, xi, mu_fm)
     else:
-        # the time is the longest chain's: 64 lanes per chain while the chip holds
-        # them (45 lines x 111 mu, six grids: about 6.5 us per solver step, 9 at 32)
-        lanes = 64 if T.size <= 2048 else 32
-        solve = chain_solver or gpu_chain_solver(device, p_num, t_num, opts, lanes_per_point=lanes)
+        # the time is the longest chain's: 64 lanes per chain (45 lines x 111 mu, six
+        # grids: about 6.5 us per solver step, 9 at 32 lanes), whatever the number of
+        # lines, since the lanes set the order of the node sums and a line's numbers
+        # must not depend on the lines beside it.  Whole scans, ms at 64 | 32 lanes:
+        # 655 lines x 60 mu 136 | 172, 2500 x 40 270 | 278, 6000 x 30 521 | 418, 20000
+        # x 20 1423 | 1030.
+        solve = chain_solver or gpu_chain_solver(device, p_num, t_num, opts, lanes_per_point=64)
         had, qrk = _follow_chains(solve, T, xi, mu_fm)
     # _select_physical_branch  DualBranchScan.jl:378-398
     both = had["valid"] & qrk["valid"]

@@ -86,3 +86,19 @@ def test_branch_chains_match_per_step_solves(gpu_ctx):
             else:
                 assert not skipped[l].any()
         assert np.all(r["converged"].reshape(T.size, mu.size)[skipped] == 0)
+
+
+def test_a_line_does_not_depend_on_the_lines_beside_it(gpu_ctx):
+    """A line's branches are the same bits alone, among a few and among
+    thousands of lines (a scan split over calls is the whole scan)."""
+    from julia_relaxtime_amd import dual_branch as DB
+    r = np.random.default_rng(6)
+    n = 2100
+    T, xi, mu = r.uniform(45.0, 140.0, n), r.choice([0.0, 0.2, 0.4], n), [250.0, 320.0, 340.0, 400.0]
+    whole = DB.run_dual_branch_scan_batch(T, mu, xi, p_num=12, t_num=4)
+    for sel in (slice(0, 1), slice(40, 80)):
+        part = DB.run_dual_branch_scan_batch(T[sel], mu, xi[sel], p_num=12, t_num=4)
+        for a, b in zip(part, whole[sel]):
+            for branch in ("hadron", "quark", "physical"):
+                for k in a[branch]:
+                    assert np.array_equal(a[branch][k], b[branch][k], equal_nan=True), (branch, k)
