@@ -5,7 +5,7 @@
 // master weights updated by Adam.
 //
 // Kernels
-//   train_tile_kernel   one 32-sample tile per block (4 waves): forward, MSE
+//   train_tile_kernel   one 32-sample tile per block (8 waves): forward, MSE
 //                       loss, backward; writes the block's partial gradient
 //   adam_kernel         sums the block partials and applies Adam; refreshes
 //                       the BF16 (and transposed BF16) weight copies and the
@@ -34,11 +34,13 @@
 namespace mlp {
 
 constexpr int IN = 3, H = 128, OUT = 4, TILE = 32, THREADS = 256;
-// A training step is one tile per CU (batch 8192: 256 blocks), a chain of
-// short phases between barriers: 16 wavefronts per tile hide the LDS and
-// weight latency that 4 waited for (one MFMA tile per wavefront and phase).
-// 32 steps of batch 8192: the kernel 33.6 -> 26.1 us per step.
-constexpr int TRAIN_THREADS = 1024;
+// A training step is a chain of short phases between barriers: 8 wavefronts per
+// tile hide the LDS and weight latency that 4 waited for, and leave room for a
+// second tile on the CU where a batch has more tiles than CUs (16 wavefronts of
+// 83 VGPRs do not).  A step with Adam on 4 / 8 / 16 wavefronts, us: batch 1024
+// 29.4 / 23.5 / 25.0, 8192 40.9 / 34.4 / 35.2, 16384 53.9 / 46.4 / 59.0, 131072
+// 388 / 337 / 445.
+constexpr int TRAIN_THREADS = 512;
 // row stride of the activation tiles in LDS: 16 bytes more than a row, so that
 // the 16 rows of a fragment load lie in different banks (a stride of 256
 // bytes puts all of them in the same four)
