@@ -104,24 +104,24 @@ struct NodeSums {
     }
 };
 
-// f(l, j, t) leaves the terms of node (l, j) in t; o gets their sums over the mesh
-template <int NL, int NC, int NP, class F>
-__device__ __forceinline__ void node_sums(double* lds_rows, int pn, int tn, double* o, const F& f)
+// o gets the sums over the mesh of S's members (NP doubles each): f(l, j, put)
+// hands the terms of node (l, j) over as put(&S::member, value).  One lane adds
+// each as it comes (all terms of a node first, then their sums, held both in
+// registers: second order, 60 000 roots on 64 x 32 nodes, 15.2 -> 14.4 ms).
+template <int NL, int NP, class S, class F>
+__device__ __forceinline__ void node_sums(double* lds_rows, int pn, int tn, S& o, const F& f)
 {
-    double t[NC * NP];
+    S t{};
     if constexpr (NL == 1) {
-#pragma unroll
-        for (int i = 0; i < NC * NP; i++) o[i] = 0.0;
+        auto put = [&](auto m, auto v) { t.*m += v; };
 #pragma unroll 1
         for (int l = 0; l < tn; l++)
 #pragma unroll 1
-            for (int j = 0; j < pn; j++) {
-                f(l, j, t);
-#pragma unroll
-                for (int i = 0; i < NC * NP; i++) o[i] += t[i];
-            }
+            for (int j = 0; j < pn; j++) f(l, j, put);
+        o = t;
     } else {
-        NodeSums<NL, NC, NP> sums(lds_rows);
+        auto put = [&](auto m, auto v) { t.*m = v; };
+        NodeSums<NL, sizeof(S) / sizeof(double) / NP, NP> sums(lds_rows);
         const int total = pn * tn;
         int l = 0, j = (int)(threadIdx.x % NL);
 #pragma unroll 1
@@ -130,10 +130,10 @@ __device__ __forceinline__ void node_sums(double* lds_rows, int pn, int tn, doub
                 j -= pn;
                 l++;
             }
-            if (l < tn) f(l, j, t);
-            sums.add(t, total - e < NL ? total - e : NL);
+            if (l < tn) f(l, j, put);
+            sums.add(reinterpret_cast<const double*>(&t), total - e < NL ? total - e : NL);
         }
-        sums.take(o);
+        sums.take(reinterpret_cast<double*>(&o));
     }
 }
 
@@ -145,8 +145,8 @@ __device__ void flavour_d(const double* tab, double* rows, int pn, int tn, doubl
     const double* cc = pp + pn;
     const double* Cm = pp + pn + tn;
     const double invT = 1.0 / T, invT2 = invT * invT, M2 = M * M;
-    node_sums<NL, sizeof(FlavD) / sizeof(double), 1>(rows, pn, tn, &o.S, [&](int l, int j, double* t) {
-        FlavD& n = *reinterpret_cast<FlavD*>(t);
+    using N = FlavD;
+    node_sums<NL, 1>(rows, pn, tn, o, [&](int l, int j, const auto& put) {
         const double xc = xi * cc[l];
         const double C = Cm[l * pn + j];
         double E, invE;
@@ -164,28 +164,28 @@ __device__ void flavour_d(const double* tab, double* rows, int pn, int tn, doubl
         const double QP = 3.0 * (sp.r1 + sm.r2), QPb = 3.0 * (sp.r2 + sm.r1);
         const double QEP = -(ac1p + ac2m) * invT, QEPb = -(ac2p + ac1m) * invT;
         const double EM = M * invE, EMM = (1.0 - EM * EM) * invE;
-        n.S = C * Q;
-        n.SM = C * (QE * EM);
-        n.SP = C * QP;
-        n.SPb = C * QPb;
-        n.SMM = C * (QEE * EM * EM + QE * EMM);
-        n.SMP = C * (QEP * EM);
-        n.SMPb = C * (QEPb * EM);
-        n.SPP = C * (-9.0 * (sp.r1 * sp.r1 + sm.r2 * sm.r2));
-        n.SPPb = C * (-9.0 * (sp.r1 * sp.r2 + sm.r1 * sm.r2));
-        n.SPbPb = C * (-9.0 * (sp.r2 * sp.r2 + sm.r1 * sm.r1));
+        put(&N::S, C * Q);
+        put(&N::SM, C * (QE * EM));
+        put(&N::SP, C * QP);
+        put(&N::SPb, C * QPb);
+        put(&N::SMM, C * (QEE * EM * EM + QE * EMM));
+        put(&N::SMP, C * (QEP * EM));
+        put(&N::SMPb, C * (QEPb * EM));
+        put(&N::SPP, C * (-9.0 * (sp.r1 * sp.r1 + sm.r2 * sm.r2)));
+        put(&N::SPPb, C * (-9.0 * (sp.r1 * sp.r2 + sm.r1 * sm.r2)));
+        put(&N::SPbPb, C * (-9.0 * (sp.r2 * sp.r2 + sm.r1 * sm.r1)));
         // da/dmu = 1/T, db/dmu = -1/T, da/dT = -a/T, db/dT = -b/T, da/dE = db/dE = -1/T
-        n.Smu = C * (gp - gm) * invT;
-        n.ST = C * (-(gp * a + gm * b) * invT);
-        n.Smumu = C * (hp + hm) * invT2;
-        n.SmuT = C * (-(gp - gm) - (hp * a - hm * b)) * invT2;
-        n.STT = C * (2.0 * (gp * a + gm * b) + hp * a * a + hm * b * b) * invT2;
-        n.SMmu = C * (-(hp - hm) * invT2) * EM;
-        n.SMT = C * ((gp + gm + hp * a + hm * b) * invT2) * EM;
-        n.SPmu = C * (ac1p - ac2m) * invT;
-        n.SPbmu = C * (ac2p - ac1m) * invT;
-        n.SPT = C * (-(ac1p * a + ac2m * b) * invT);
-        n.SPbT = C * (-(ac2p * a + ac1m * b) * invT);
+        put(&N::Smu, C * (gp - gm) * invT);
+        put(&N::ST, C * (-(gp * a + gm * b) * invT));
+        put(&N::Smumu, C * (hp + hm) * invT2);
+        put(&N::SmuT, C * (-(gp - gm) - (hp * a - hm * b)) * invT2);
+        put(&N::STT, C * (2.0 * (gp * a + gm * b) + hp * a * a + hm * b * b) * invT2);
+        put(&N::SMmu, C * (-(hp - hm) * invT2) * EM);
+        put(&N::SMT, C * ((gp + gm + hp * a + hm * b) * invT2) * EM);
+        put(&N::SPmu, C * (ac1p - ac2m) * invT);
+        put(&N::SPbmu, C * (ac2p - ac1m) * invT);
+        put(&N::SPT, C * (-(ac1p * a + ac2m * b) * invT));
+        put(&N::SPbT, C * (-(ac2p * a + ac1m * b) * invT));
     });
 }
 
@@ -563,10 +563,8 @@ __device__ void flavour_r(const double* tab, double* rows, int pn, int tn, R M, 
     const double* cc = pp + pn;
     const double* Cm = pp + pn + tn;
     const R invT = 1.0 / T, invT2 = invT * invT, M2 = M * M;
-    constexpr int kParts = sizeof(R) / sizeof(double);
-    node_sums<NL, sizeof(FlavR<R>) / sizeof(R), kParts>(rows, pn, tn, reinterpret_cast<double*>(&o), [&](int l, int j,
-                                                                                                       double* t) {
-        FlavR<R>& n = *reinterpret_cast<FlavR<R>*>(t);
+    using N = FlavR<R>;
+    node_sums<NL, sizeof(R) / sizeof(double)>(rows, pn, tn, o, [&](int l, int j, const auto& put) {
         const double xc = xi * cc[l];
         const double C = Cm[l * pn + j];
         R E, invE;
@@ -581,21 +579,21 @@ __device__ void flavour_r(const double* tab, double* rows, int pn, int tn, R M, 
         const R QE = -(gp + gm) * invT, QEE = (hp + hm) * invT2;
         const R QEP = -(ac1p + ac2m) * invT, QEPb = -(ac2p + ac1m) * invT;
         const R EM = M * invE, EMM = (1.0 - EM * EM) * invE;
-        n.SM = C * (QE * EM);
-        n.SP = C * (3.0 * (sp.r1 + sm.r2));
-        n.SPb = C * (3.0 * (sp.r2 + sm.r1));
-        n.SMM = C * (QEE * EM * EM + QE * EMM);
-        n.SMP = C * (QEP * EM);
-        n.SMPb = C * (QEPb * EM);
-        n.SPP = C * (-9.0 * (sp.r1 * sp.r1 + sm.r2 * sm.r2));
-        n.SPPb = C * (-9.0 * (sp.r1 * sp.r2 + sm.r1 * sm.r2));
-        n.SPbPb = C * (-9.0 * (sp.r2 * sp.r2 + sm.r1 * sm.r1));
-        n.SMmu = C * (-(hp - hm) * invT2) * EM;
-        n.SMT = C * ((gp + gm + hp * a + hm * b) * invT2) * EM;
-        n.SPmu = C * (ac1p - ac2m) * invT;
-        n.SPbmu = C * (ac2p - ac1m) * invT;
-        n.SPT = C * (-(ac1p * a + ac2m * b) * invT);
-        n.SPbT = C * (-(ac2p * a + ac1m * b) * invT);
+        put(&N::SM, C * (QE * EM));
+        put(&N::SP, C * (3.0 * (sp.r1 + sm.r2)));
+        put(&N::SPb, C * (3.0 * (sp.r2 + sm.r1)));
+        put(&N::SMM, C * (QEE * EM * EM + QE * EMM));
+        put(&N::SMP, C * (QEP * EM));
+        put(&N::SMPb, C * (QEPb * EM));
+        put(&N::SPP, C * (-9.0 * (sp.r1 * sp.r1 + sm.r2 * sm.r2)));
+        put(&N::SPPb, C * (-9.0 * (sp.r1 * sp.r2 + sm.r1 * sm.r2)));
+        put(&N::SPbPb, C * (-9.0 * (sp.r2 * sp.r2 + sm.r1 * sm.r1)));
+        put(&N::SMmu, C * (-(hp - hm) * invT2) * EM);
+        put(&N::SMT, C * ((gp + gm + hp * a + hm * b) * invT2) * EM);
+        put(&N::SPmu, C * (ac1p - ac2m) * invT);
+        put(&N::SPbmu, C * (ac2p - ac1m) * invT);
+        put(&N::SPT, C * (-(ac1p * a + ac2m * b) * invT));
+        put(&N::SPbT, C * (-(ac2p * a + ac1m * b) * invT));
     });
 }
 
