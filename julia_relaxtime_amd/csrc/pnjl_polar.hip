@@ -1989,9 +1989,11 @@ int pnjl_meson_mass_batch(pnjl_ctx* ctx, int64_t n, const pnjl_mass_query* q, co
     // for every other phase (524 288 queries: 111 ms, with one lane in the
     // first two phases 153), 64 in the tail while the longest searches set the
     // time (tail at 16 / 64 lanes: 18 432 queries 21.7 / 13.0 ms, 131 072
-    // queries 50 / 43); one lane past the launch limit of 2^32 threads.
+    // queries 50 / 43); one lane where 16 pass the launch limit of 2^32 - 1
+    // threads (the last 16 batch sizes of all).
     constexpr int kTailPhase = 2;
-    const int head = stride > 1 || n > ((int64_t)1 << 27) ? 1 : 16, tail = (head > 1 && n <= 131072) ? 64 : head;
+    const bool one = stride > 1 || 256 * (int64_t)blocks_for(16 * n) > 0xffffffffLL;
+    const int head = one ? 1 : 16, tail = (!one && n <= 131072) ? 64 : head;
     for (int ph = 0; ph < kPhases; ph++) {
         const int32_t* in_list = ph == 0 ? nullptr : lists[(ph - 1) & 1];
         const unsigned* in_count = ph == 0 ? nullptr : cnt + ph - 1;
