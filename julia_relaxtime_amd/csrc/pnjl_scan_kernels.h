@@ -541,10 +541,10 @@ __device__ __forceinline__ void flavours_wide(const double* lds, int pn, int tn,
 // kNodes nodes of every chain at once, its lanes leave the terms in LDS rows,
 // and each lane adds some of one chain's terms, in order: bound, like all of a
 // small call, by the latency of dependent FP64 instructions and of LDS.  A
-// solve of 1024 points (p 64 t 4, max_iter 40) takes 1.91 ms at xi = 0.2 and
-// 1.20 at 0 (free order, flavours_wide: 1.52 and 1.14; 4 lanes: 36 and 13); of
-// 262144 points, on 8 lanes, 40.3 and 18.2 (8 lanes in free order: 39.6 and
-// 19.8; 4 lanes: 87 and 32).
+// solve of 1024 points (p 64 t 4, max_iter 40) takes 1.78 ms at xi = 0.2 and
+// 1.17 at 0 (free order, flavours_wide: 1.52 and 1.14; 4 lanes: 36 and 13); of
+// 262144 points, on 8 lanes, 39.2 and 18.1 (8 lanes in free order: 39.6 and
+// 19.8; 4 lanes: 81 and 31).
 template <int LPP>
 struct Four {
     static constexpr int kHalf = LPP / 2;                           // lanes per flavour
@@ -573,7 +573,9 @@ __device__ __forceinline__ void wave_fence()
 // This lane's chain sums of one flavour: acc[i] of row i kNodes + sl, chain v.
 // A lane evaluates two nodes of a chain at a time (two independent sequences of
 // dependent instructions), without branches: past the chain's end, node 0
-// again, into a slot that nobody adds.
+// again, into a slot that nobody adds.  The second node's terms are stored and
+// loaded behind the first's before either is added (one after the other: the
+// 1024 points above 1.91 and 1.20 ms; one node at a time 1.92 and 1.21).
 template <int LPP, bool kChecked>
 __device__ __forceinline__ void four_loop(const double* lds, int pn, int tn, double M2, double muT, double invT,
                                           double K2mu, double xi, double Phi, double Phib, int gl, double* rows,
@@ -608,36 +610,54 @@ __device__ __forceinline__ void four_loop(const double* lds, int pn, int tn, dou
             const double p2 = pp[j];
             node_terms<kChecked>(lds, iso ? p2 : fma(xi * cc[lb], p2, p2), C[b], M2, muT, invT, K2mu, Phi, Phib, n[b]);
         }
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            if (r + b * S >= longest) break;
+        auto store = [&](int b) {
             const double t[16] = {n[b].S,   n[b].Sfp,   n[b].Sfm,  n[b].SP, n[b].SPb, n[b].SPP, n[b].SPPb, n[b].SPbPb,
                                   n[b].Sfab, n[b].A1, n[b].B1, n[b].B2, n[b].A2, C[b], n[b].CinvE, n[b].CinvE2};
 #pragma unroll
             for (int c = 0; c < 16; c++) mine[c * G::kRow + sl] = t[c];
             wave_fence();
-            const int m = total - r - b * S;   // nodes in this lane's chain's slots
-            const bool full = __all(m >= S);
+        };
+        if (__all(r + NB * S <= total)) {
+            // all loads of both nodes' terms before the sums: one LDS latency
+            double2 x[NB][G::kOwn][S / 2], f[NB][G::kOwn][S / 2];
 #pragma unroll
-            for (int i = 0; i < G::kOwn; i++) {
-                const int c = i * S + sl;
-                if (c >= 13) continue;
-                const double* x = mine + c * G::kRow;
-                const double* f = mine + row_factor(c) * G::kRow;
-                if (full) {
+            for (int b = 0; b < NB; b++) {
+                store(b);
 #pragma unroll
-                    for (int k = 0; k < S; k += 2) {
-                        const double2 a = *reinterpret_cast<const double2*>(x + k);
-                        const double2 w = *reinterpret_cast<const double2*>(f + k);
-                        acc[i] = fma(w.x, a.x, acc[i]);
-                        acc[i] = fma(w.y, a.y, acc[i]);
+                for (int i = 0; i < G::kOwn; i++) {
+                    const int c = i * S + sl < 13 ? i * S + sl : 12;   // past the last row: its sum is not used
+#pragma unroll
+                    for (int k = 0; k < S / 2; k++) {
+                        x[b][i][k] = *reinterpret_cast<const double2*>(mine + c * G::kRow + 2 * k);
+                        f[b][i][k] = *reinterpret_cast<const double2*>(mine + row_factor(c) * G::kRow + 2 * k);
                     }
-                } else {
+                }
+                wave_fence();   // the rows are written again only after every lane has read them
+            }
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int k = 0; k < S / 2; k++)
+#pragma unroll
+                    for (int i = 0; i < G::kOwn; i++) {
+                        acc[i] = fma(f[b][i][k].x, x[b][i][k].x, acc[i]);
+                        acc[i] = fma(f[b][i][k].y, x[b][i][k].y, acc[i]);
+                    }
+        } else {
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                store(b);
+                const int m = total - r - b * S;   // nodes in this lane's chain's slots
+#pragma unroll
+                for (int i = 0; i < G::kOwn; i++) {
+                    const int c = i * S + sl < 13 ? i * S + sl : 12;
+                    const double* x = mine + c * G::kRow;
+                    const double* f = mine + row_factor(c) * G::kRow;
 #pragma unroll 1
                     for (int k = 0; k < S && k < m; k++) acc[i] = fma(f[k], x[k], acc[i]);
                 }
+                wave_fence();
             }
-            wave_fence();   // the rows are written again only after every lane has read them
         }
     }
 }
