@@ -243,18 +243,23 @@ ScanGeom scan_geom(int lpp, int pn, int tn, size_t lds_block, bool four)
 // longest solves, and 64 lanes shorten every pass; once the chip is full, 8
 // lanes waste least (below 8 the groups' LDS state leaves room for one
 // wavefront per SIMD only).  The lines lie where 64 and 8 lanes cost about the
-// same over four meshes (p 64 t 4 at xi = 0.2 / p 64 at 0 / p 12 t 6 at 0.2 / p
-// 24 at 0; ms at 64 | 8 lanes, the later stages on 64, against 37 / 13 / 14 / 8
-// of {4, 4, 8, 0}):
-//   DefaultSeed, max_iter 40, 4096 points 2.6 / 1.7 / 1.8 / 1.7 | 3.6 / 1.9 / 2.0 /
-//   1.6, 8192 points 3.8 / 2.3 / 2.7 / 2.2 | 4.0 / 2.0 / 2.1 / 1.6;
-//   its later stages (few, long items) on 64 | 8 lanes, 32768 points 7.9 / 4.2 /
-//   4.0 / 3.4 | 9.4 / 4.2 / 3.9 / 2.8, 131072 points 23 / 13 / 12 / 11 | 22 / 10 / 10 / 7;
-//   MultiSeed (six long items per point), 1400 points 2.3 / 1.4 / 1.6 / 1.4 | 4.6 /
-//   1.7 / 1.9 / 1.2, 2800 points 3.7 / 2.2 / 2.6 / 2.2 | 4.8 / 1.8 / 2.0 / 1.3;
-//   chains of 10 points (serial over their points; p 24 t 8 at 0.2 / p 12 t 6 at
-//   0.2 / p 12 at 0), 8192 chains 9.8 / 6.3 / 6.1 | 18 / 8.1 / 5.8, 16384 chains 12.4
-//   / 9.7 / 7.8 | 20 / 9.9 / 6.0, 65536 chains 36 / 26 / 22 | 30 / 15 / 9.
+// same; a pass of more nodes keeps 64 lanes busy, so they grow with the mesh, as
+// the root of p sqrt(t) (between its nodes at xi = 0, p, and elsewhere, p t).
+// Measured on p 64 t 4 at xi = 0.2 / p 64 at 0 / p 12 t 6 at 0.2 / p 24 at 0, ms on
+// 64 | 8 lanes | {4, 4, 8, 0}:
+//   DefaultSeed, max_iter 40, the later stages (few, long items) on 64 lanes:
+//   1024 points 1.8 / 1.2 / 1.3 / 1.2 | 3.5 / 1.8 / 1.8 / 1.4 | 36 / 13 / 14 / 8, 8192
+//   points 3.7 / 2.2 / 2.7 / 2.3 | 3.9 / 2.0 / 2.1 / 1.6 | 38 / 13 / 14 / 8; 64 x 32
+//   nodes 8192 points 19 | 24, 16384 points 29 | 33;
+//   8 lanes with the later stages on 64 | 8: 32768 points 7.7 / 4.1 / 3.9 / 3.4 | 9.2 /
+//   4.2 / 3.9 / 2.8, 131072 points 22.6 / 12.6 / 11.5 / 10.7 | 22.0 / 10.0 / 9.7 / 6.9;
+//   MultiSeed (six long items per point): 1400 points 2.3 / 1.4 / 1.7 / 1.4 | 4.6 /
+//   1.7 / 1.9 / 1.2 | 19 / 7 / 7 / 4, 2800 points 3.7 / 2.2 / 2.7 / 2.3 | 4.7 / 1.9 /
+//   2.0 / 1.3 | 19 / 7 / 8 / 4;
+//   chains of 10 points (serial over their points), p 24 t 8 at 0.2 / p 12 t 6 at
+//   0.2 / p 12 at 0: 8192 chains 9.1 / 6.5 / 6.3 | 18 / 8.0 / 6.1 | 55 / 26 / 13, 16384
+//   chains 11.9 / 9.7 / 8.1 | 21 / 10.2 / 6.0 | 58 / 23 / 12, 65536 chains 35 / 27 / 23 |
+//   33 / 16 / 9 | 63 / 30 / 16.
 // A node table that leaves no room for 4-lane groups: kDefaultCfg itself
 // (scan_geom raises its lanes by the table alone).
 struct Launch {
@@ -266,10 +271,11 @@ Launch choose_launch(const pnjl::ScanArgs& A, size_t lds_block)
 {
     const int four = kDefaultCfg.lanes_per_point;
     if (scan_geom(four, A.pn, A.tn, lds_block, false).lpp != four) return Launch{kDefaultCfg, false};
-    const int64_t line = A.plan == pnjl::PLAN_CHAINS ? 16384 : (A.plan == pnjl::PLAN_MULTI ? 2048 : 4096);
-    const int64_t items = A.plan == pnjl::PLAN_CHAINS ? A.n_items : A.n_points;
+    const double unit = sqrt(A.pn * sqrt((double)A.tn));
+    const double line = (A.plan == pnjl::PLAN_CHAINS ? 1900 : (A.plan == pnjl::PLAN_MULTI ? 220 : 600)) * unit;
+    const double items = (double)(A.plan == pnjl::PLAN_CHAINS ? A.n_items : A.n_points);
     if (items <= line) return Launch{pnjl_launch_cfg{64, 1, 8, 0}, true};
-    return Launch{pnjl_launch_cfg{8, 1, 16, A.n_points <= 32768 ? 64 : 8}, true};
+    return Launch{pnjl_launch_cfg{8, 1, 16, items <= 8 * line ? 64 : 8}, true};
 }
 
 // Lets every scan_kernel instantiation take `bytes` of dynamic LDS.

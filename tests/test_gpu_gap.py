@@ -330,7 +330,7 @@ def test_default_geometry_picks_lanes(gpu_ctx, policy, n, chain):
 
 
 @pytest.mark.parametrize("policy,n,chain,pn,tn", [(0, 36000, 0, 16, 4), (3, 4100, 0, 16, 4), (5, 16390 * 2, 2, 12, 3),
-                                                  (4, 4200, 0, 7, 3), (0, 4200, 0, 65, 2), (4, 300, 0, 3, 5),
+                                                  (4, 4200, 0, 7, 3), (0, 6000, 0, 65, 2), (4, 300, 0, 3, 5),
                                                   (3, 60, 0, 1, 1), (0, 40, 0, 64, 64), (0, 9, 0, 4096, 1)])
 def test_default_results_do_not_depend_on_the_call(policy, n, chain, pn, tn):
     """At the default geometry a point's results are the same bits alone, in a
@@ -352,8 +352,10 @@ def test_default_results_do_not_depend_on_the_call(policy, n, chain, pn, tn):
     ctx = _lib.Context(0)
     f = lambda m: ctx.solve_batch(T[:m], mu[:m], xi[:m], policy=policy, p_num=pn, t_num=tn, opts=opts,  # noqa: E731
                                   **{k: v[:m] for k, v in kw.items()})
-    # chain lines: 16384 chains; MultiSeed 2048 points; the rest 4096 and 32768
-    cuts = [m for m in (1, 63, 2048, 2049, 4096, 4097, 32768, 32770) if m < n and m % max(chain, 1) == 0] + [n]
+    # 64 lanes, then 8 (the later stages on 64), then 8: the lines are DefaultSeed's
+    # 3394 and 27153 points, MultiSeed's 1244, 8661 chains, and the explicit seeds' 2089
+    cuts = [m for m in (1, 64, 1200, 1300, 2000, 2100, 3300, 3500, 17300, 17400, 27000, 27400)
+            if m < n and m % max(chain, 1) == 0] + [n]
     own = {m: f(m) for m in cuts}
     ctx.set_launch_cfg(4, 1, 8, 0)
     four = f(n)
