@@ -417,12 +417,14 @@ def test_small_call_setup(gpu_ctx, m):
 @pytest.mark.parametrize("pn,tn,xi", [(64, 4, 0.0), (65, 3, 0.0), (1, 1, 0.3), (1, 64, 0.3), (12, 6, -0.2), (31, 2, 0.4),
                                       (64, 1, 0.2), (64, 64, 0.1), (7, 9, 0.0)])
 def test_wide_group_node_pass(gpu_ctx, lpp, pn, tn, xi):
-    """One Newton step of a 32- or 64-lane group (both flavours side by side, the
+    """The pass of a 32- or 64-lane group (both flavours side by side, the
     flattened mesh, the row-swap reduction) against a 4-lane group's, at meshes
-    that do and do not fill a round.  max_iter = 0: the outputs are Omega, the
-    residual and the thermodynamics at the seed, sums of the same node terms
-    in another order, 1e-13 of their size each (|terms| summed: at most 1e3
-    times the smallest of them)."""
+    that do and do not fill a round.  max_iter = 0: Omega, the residual and the
+    thermodynamics at the seed, sums of the same node terms in another order,
+    1e-13 of their size each (|terms| summed: at most 1e3).  max_iter = 1: x
+    after one Newton step p = -J^-1 F, which takes every sum of the pass: errors
+    dF and dJ of that size move it by |J^-1| (dF + 5 dJ |p|), twice that for the
+    second order."""
     from julia_relaxtime_amd import _lib
     r = np.random.default_rng(pn * tn)
     n = 70
@@ -430,14 +432,21 @@ def test_wide_group_node_pass(gpu_ctx, lpp, pn, tn, xi):
     seed = np.stack([r.uniform(-1.8, -0.1, n), r.uniform(-1.8, -0.1, n), r.uniform(-2.2, -0.4, n), r.uniform(-0.3, 0.9, n),
                      r.uniform(0.01, 0.9, n)], 1)
     seed[::2, 1] = seed[::2, 0]     # phi_u = phi_d: two flavours, else three
-    opts = _lib.default_opts(max_iter=0, trust_region_fallback=0, auto_multiseed_fallback=0)
-    out = []
+    out = {}
     for l in (4, lpp):
-        with gpu_ctx.launch(lanes_per_point=l, chunk=1):
-            out.append(gpu_ctx.solve_batch(T, mu, xi, policy=4, seed=seed, p_num=pn, t_num=tn, opts=opts))
+        for it in (0, 1):
+            opts = _lib.default_opts(max_iter=it, trust_region_fallback=0, auto_multiseed_fallback=0)
+            with gpu_ctx.launch(lanes_per_point=l, chunk=1):
+                out[l, it] = gpu_ctx.solve_batch(T, mu, xi, policy=4, seed=seed, p_num=pn, t_num=tn, opts=opts)
     for k in ("omega", "rho_norm", "entropy", "energy", "n_q", "n_qbar", "residual_norm", "x"):
-        a, b = out[0][k], out[1][k]
+        a, b = out[4, 0][k], out[lpp, 0][k]
         assert np.all(np.abs(a - b) <= 1e-13 * (1e3 + np.abs(a))), k
+    a, b = out[4, 1]["x"], out[lpp, 1]["x"]
+    assert np.all(out[4, 1]["newton_steps"] == 1) and np.all(out[lpp, 1]["newton_steps"] == 1)
+    J = gpu_ctx.residual_batch(seed, T, mu, np.full(n, xi), pn, tn)[1]
+    inv = np.abs(np.linalg.inv(J)).sum(axis=2).max(axis=1)
+    p = np.abs(a - seed).max(axis=1)
+    assert np.all(np.abs(a - b).max(axis=1) <= 2 * inv * 1e-10 * (1 + 5 * p))
 
 
 def test_device_pointer_path(gpu_ctx):
