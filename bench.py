@@ -356,13 +356,17 @@ def run_propagators(args, w):
 
 
 MASS_METRIC = "meson pole masses solved/s (solve_meson_mass, 8 mesons x 65,536 (T, mu) points)"
-# FP64 FLOPs per pole-mass query of this batch, counted once on 8,192 seeded
-# queries run one per wavefront (python3 bench.py --flop-probe mass), summed
-# over the phase launches: 1,052,503 per query (38.7 trust-region iterations on
-# average; 36 % of the queries stop at the start on a non-finite residual).
-# The kernel's time is set by its longest serial chains (queries running the
-# full 1000 iterations), not by FP64 throughput.
-MASS_FLOPS_PER_QUERY = 1052503.0
+# FP64 FLOPs that NLsolve's iteration needs per pole-mass query of this batch:
+# B0 of the meson's quark pairs at every trial k0, and at k0 +- h where the step
+# is accepted, 94.2 pair evaluations per query on 8,192 seeded queries (38.7
+# iterations on average; 36 % of the queries stop at the start on a non-finite
+# residual).  The kernel evaluates k0 +- h on every trip: 224.6 evaluations,
+# 1,052,503 FLOPs counted one query per wavefront (python3 bench.py
+# --flop-probe mass), 4,686 each.  (33.7 evaluations, 158,031 FLOPs, without the
+# trips after a search's state has stopped to change.)  The kernel's time is
+# set by its longest serial chains (queries running the full 1000 iterations),
+# not by FP64 throughput.
+MASS_FLOPS_PER_QUERY = 441418.0
 
 
 def _mass_worker(args):
@@ -473,7 +477,7 @@ def run_dual(args, w):
     from julia_relaxtime_amd.pnjl import context
     ctx = context(0)
     T, xi, mu = dual_lines()
-    gsolve = DB.gpu_chain_solver(0, 24, 8)
+    gsolve = DB.gpu_chain_solver(0, 24, 8, lanes_per_point=64)   # as the scan itself
     stats = dict(ms=0.0, passes=0.0, points=0, launches=0)
     t_eff = lambda x: np.where(x == 0.0, 1, 8)
 
@@ -621,7 +625,7 @@ def run_maxwell(args, w):
     from julia_relaxtime_amd.pnjl import context
     ctx = context(0)
     T, xi, mu = maxwell_lines()
-    gsolve, gchain = DB.gpu_solver(0, 24, 8), DB.gpu_chain_solver(0, 24, 8)
+    gsolve, gchain = DB.gpu_solver(0, 24, 8), DB.gpu_chain_solver(0, 24, 8, lanes_per_point=64)
     stats = dict(ms=0.0, passes=0.0, points=0, launches=0)
     t_eff = lambda x: np.where(x == 0.0, 1, 8)
 

@@ -9,9 +9,9 @@
 // the exact integrals.  All of it is FP64 arithmetic on tables in LDS, bound
 // by instruction issue: B0's terms that differ only in the distribution's
 // sign are evaluated together, every rule and integrand of an evaluation goes
-// through one node loop, and the nodes' functions are table-driven.  On the
-// 256-point x 3 pairs x 128 k0 x 64 k grid a replay takes 10.4 ms (30.4 ms
-// with one loop per rule, term by term, on the library's functions).  For the
+// through one node loop, and the nodes' functions are table-driven.  On six
+// 256-point x 3 pairs x 128 k0 x 64 k grids a call takes 10.6 to 11.2 ms (29.1
+// to 31.0 with one loop per rule, term by term, on the library's functions).  For the
 // grid call, the threads of a wavefront share (point, pair) and take an 8 x 8
 // tile of (k0, k), so their segment structures differ only smoothly; the
 // propagator batch sorts its work into buckets of similar (pair, mass,
@@ -895,7 +895,7 @@ __global__ void __launch_bounds__(256) grid_a_kernel(Phys P, int npts, const pnj
 }
 
 // k extent of a wavefront's (k0, k) tile: 8 x 8 tiles keep the lanes of a
-// wavefront closer in both momenta than a 1 x 64 row (measured on the 256 x
+// wavefront closer in both momenta than a 1 x 64 row (measured on one 256 x
 // 128 x 64 grid: 10.5 ms per call against 12.8 ms for 1 x 64 rows, 10.6 for
 // 4 x 16, 10.8 for 16 x 4, 11.3 for 32 x 2).
 #ifndef PNJL_GRID_TILE_K
