@@ -258,6 +258,10 @@ class Context:
                                                 m.ctypes.data_as(C.POINTER(C.c_uint8))), "pnjl_set_judge_mask")
 
     def set_launch_cfg(self, lanes_per_point=4, chunk=4, waves_per_cu=8, tail_lanes_per_point=0):
+        """The launch geometry of every solve from now on.  A new context leaves
+        it to the library, whose choice by the size of the call gives the
+        results of 4 lanes per point, bit for bit; other lanes add the node
+        sums in another order (equal to rounding)."""
         cfg = LaunchCfg(lanes_per_point, chunk, waves_per_cu, tail_lanes_per_point)
         self._check(self._L.pnjl_set_launch_cfg(self.h, C.byref(cfg)), "pnjl_set_launch_cfg")
 

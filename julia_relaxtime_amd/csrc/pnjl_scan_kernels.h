@@ -5,7 +5,9 @@
 // by the autotuner) owns one work item at a time; 64/LPP groups share a
 // wavefront.  Each lane integrates every LPP-th momentum node; the group's
 // partial sums are combined with xor-butterfly shuffles, so every lane of a
-// group holds bit-identical sums and runs the identical control logic.
+// group holds bit-identical sums and runs the identical control logic.  (The
+// groups that the library itself chooses split the nodes and add the sums
+// otherwise, in the order of four lanes: struct Four.)
 //
 // One trip of the loop = one node pass at the group's current state x
 // (Omega, F = grad P, J = dF/dx and the thermodynamic sums, all fused) plus

@@ -307,9 +307,10 @@ def test_launch_geometry_does_not_change_results(gpu_ctx):
 @pytest.mark.parametrize("policy,n,chain", [(0, 1, 0), (0, 8191, 0), (0, 8193, 0), (0, 16385, 0), (0, 32769, 0), (3, 2731, 0),
                                             (3, 2730, 0), (5, 3 * 2048, 3), (5, 3 * 2049, 3)])
 def test_default_geometry_picks_lanes(gpu_ctx, policy, n, chain):
-    """The default launch geometry chooses lanes per point by the number of
-    points (here on both sides of its lines): the same roots as a fixed 4-lane
-    geometry.  Both runs stop at |F|_inf < ftol near one root (MultiSeed's may
+    """The default launch geometry chooses lanes per point by the size of the
+    call: the same roots as a fixed 4-lane geometry at small and large calls
+    (the bits and the lines between lane counts are the next test's).  Both
+    runs stop at |F|_inf < ftol near one root (MultiSeed's may
     be another candidate's), so they differ by at most 2 ftol |J^-1|_inf to
     first order; 1e-13 for the rounding of the node sums."""
     from julia_relaxtime_amd import _lib
